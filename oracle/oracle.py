@@ -14,7 +14,7 @@ import numpy as np
 HERE = os.path.dirname(os.path.abspath(__file__))
 ORACLE_LIB = os.path.join(HERE, "liboracle.so")
 REF_LIB = os.path.join(HERE, "_ref", "libref.so")
-REF_TREE = "/root/reference"
+REF_SOURCE = "/root/reference/crates/rocketsim-cuda/csrc/phase.cpp"  # what _ref/ is compiled from
 
 ARENA_WORDS = 2784
 TICK_WORDS = 2567
@@ -24,9 +24,9 @@ _u32, _u64 = ctypes.c_uint32, ctypes.c_uint64
 
 
 def build(ref=None):
-    """Compiles liboracle.so (and _ref/libref.so when the reference tree is present, or when ref=True)."""
+    """Compiles liboracle.so (and _ref/libref.so when the reference's source is present, or when ref=True)."""
     subprocess.run(["make", "-s", "-C", HERE, "liboracle.so", "liboracle_libm.so"], check=True)
-    if ref or (ref is None and os.path.isdir(REF_TREE)):
+    if ref or (ref is None and os.path.isfile(REF_SOURCE)):
         subprocess.run(["make", "-s", "-C", HERE, "ref"], check=True)
 
 
