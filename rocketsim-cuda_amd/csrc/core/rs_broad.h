@@ -109,7 +109,7 @@ RS_FN void remove_pair(ArenaState& s, const StaticData& w, uint32_t ha, uint32_t
 constexpr uint32_t SAP_HE_WORDS = 3u * NUM_HANDLES;  // then the axis's edges, at most 64 slots (NUM_EDGES of them used)
 static_assert(sizeof(HandleEdges) == 12 && sizeof(Edge) == 4 && sizeof(((ArenaState*)nullptr)->handle_edges) == 4 * SAP_HE_WORDS,
               "HandleEdges is six u16 in three words, an Edge one word");
-static_assert(NUM_HANDLES <= 32 && NUM_EDGES <= 64 && SAP_HE_WORDS + 64u <= (uint32_t)LANE_LDS_WORDS,
+static_assert(NUM_HANDLES <= 32 && NUM_EDGES <= 64 && SAP_HE_WORDS + 64u == (uint32_t)SWEEP_WORDS,
               "masked indices stay in the lane's slice");
 struct SapCopy {
 #if !defined(__HIP_DEVICE_COMPILE__)

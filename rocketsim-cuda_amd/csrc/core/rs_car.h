@@ -710,8 +710,9 @@ RS_INLINE void car_pre_tick(ArenaState& s, const StaticData& w, int ci, const Wh
 // car's update apart from the rest of the phase (measured faster than inlining it). Its state and world pointers carry
 // their address spaces, so its accesses compile to scratch_ and global_ instructions.
 // UW: every lane steps in the same world (its pointer is then made wave-uniform).
-template <bool UW>
-RS_NOINL void car_pre_tick_in(RS_PRIVATE_AS ArenaState* sp, const RS_CONST_AS StaticData* wp, int ci,
+// M: where the state lives (InPrivate, InLds).
+template <bool UW, class M>
+RS_NOINL void car_pre_tick_in(typename M::template Ptr<ArenaState> sp, const RS_CONST_AS StaticData* wp, int ci,
                               const RS_PRIVATE_AS WheelRayPrep* pp) {
   if (UW) wp = rs_uniform_ptr(wp);
   RS_UNIFORM_INDEX(ci);
@@ -719,6 +720,7 @@ RS_NOINL void car_pre_tick_in(RS_PRIVATE_AS ArenaState* sp, const RS_CONST_AS St
 }
 // Both cars' wheel-ray screens and mesh walks, before either car's pre-tick (exact: see WheelRayPrep). A demoed car casts
 // no rays this tick (its pre-tick respawns it at most); its share is empty.
+template <class M>
 RS_FN void wheel_rays_prepare(const ArenaState& s, const StaticData& w, WheelRayPrep& prep) {
   prep.tb.n_jobs = prep.tb.n_leaves = prep.tb.next = 0;
   prep.tb.leaves = 1;
@@ -737,16 +739,17 @@ RS_FN void wheel_rays_prepare(const ArenaState& s, const StaticData& w, WheelRay
     }
     prep.end_job[ci] = prep.tb.n_jobs;
   }
-  trav_run(w, prep.tb);
+  trav_run<M>(w, prep.tb);
 }
-template <bool UW = false>
+template <bool UW = false, class M = InPrivate>
 RS_INLINE void phase_p1(ArenaState& s, const StaticData& w) {
   for (int ci = 0; ci < NUM_CARS; ++ci) car_flip_zdamp(s, w, ci);
   WheelRayPrep prep;
-  wheel_rays_prepare(s, w, prep);
+  wheel_rays_prepare<M>(s, w, prep);
   for (int ci = 0; ci < NUM_CARS; ++ci) {
     uint32_t was = s.cars[ci].is_on_ground;
-    car_pre_tick_in<UW>((RS_PRIVATE_AS ArenaState*)&s, (const RS_CONST_AS StaticData*)&w, ci, (const RS_PRIVATE_AS WheelRayPrep*)&prep);
+    car_pre_tick_in<UW, M>((typename M::template Ptr<ArenaState>)&s, (const RS_CONST_AS StaticData*)&w, ci,
+                           (const RS_PRIVATE_AS WheelRayPrep*)&prep);
     if (!was && s.cars[ci].is_on_ground) s.events |= 1u << (EV_LANDED + ci);
   }
 }

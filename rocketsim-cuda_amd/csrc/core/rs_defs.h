@@ -30,17 +30,21 @@
 // StaticData through pointers qualified with these compiles their accesses to scratch_* / global_* instructions; through
 // generic pointers they would be flat instructions, which wait on both the vector-memory and the LDS/scalar counters and
 // need 64-bit VGPR addresses. Empty on the host.
+// The state is private memory in most kernels and LDS in the one for small batches: the qualifier comes from InPrivate or
+// InLds (below), which the phase functions take as a template parameter.
 // RS_PRIVATE(p) states the same for a pointer parameter that always points into the lane's private memory. The StaticData
 // is passed as constant memory (RS_CONST_AS): no kernel writes it, and the compiler may then read it with scalar loads
 // wherever the address is the same in every lane (it cannot prove that of global memory inside a non-kernel function).
 #if defined(__HIP_DEVICE_COMPILE__)
 #define RS_PRIVATE_AS __attribute__((address_space(5)))
 #define RS_GLOBAL_AS __attribute__((address_space(1)))
+#define RS_LDS_AS __attribute__((address_space(3)))
 #define RS_CONST_AS __attribute__((address_space(4)))
 #define RS_PRIVATE(p) __builtin_assume(__builtin_amdgcn_is_private((const void*)(p)))
 #else
 #define RS_PRIVATE_AS
 #define RS_GLOBAL_AS
+#define RS_LDS_AS
 #define RS_CONST_AS
 #define RS_PRIVATE(p) ((void)0)
 #endif
@@ -77,6 +81,19 @@ inline T* rs_uniform_ptr(T* p) { return p; }
 #endif
 
 namespace rs {
+
+// Where the lanes' ArenaStates live, and how many arenas a wave steps at most: private memory, one arena per lane, or LDS,
+// a few arenas per wave.
+struct InPrivate {
+  static constexpr uint32_t ARENAS = 64;
+  template <class T>
+  using Ptr = RS_PRIVATE_AS T*;
+};
+struct InLds {
+  static constexpr uint32_t ARENAS = 3;
+  template <class T>
+  using Ptr = RS_LDS_AS T*;
+};
 
 RS_FN uint32_t fbits(float a) { return __builtin_bit_cast(uint32_t, a); }
 RS_FN float ffrom(uint32_t u) { return __builtin_bit_cast(float, u); }

@@ -816,6 +816,7 @@ RS_FN int mesh_job_of(const Np& c, uint32_t a, uint32_t b, uint32_t* body, uint3
   return mesh_of(c.w, other) ? TJ_CAR : -1;
 }
 // P3b (:230-282): the retained pairs in pair-array order. Returns the number of unimplemented pair algorithms reached.
+template <class M>
 RS_INLINE uint32_t phase_p3b_body(ArenaState& s, const StaticData& w) {
   // the records' event bits and count are kept in registers and written once (nothing else reads them before P7)
   const uint32_t n_records0 = s.n_records;
@@ -834,7 +835,7 @@ RS_INLINE uint32_t phase_p3b_body(ArenaState& s, const StaticData& w) {
     jb.mesh_body = mesh_b;
     jb.box = kind == TJ_CAR ? car_mesh_frame(c, body, mesh_b).local_box : ball_mesh_box(c, body, mesh_b);
   }
-  trav_run(w, tb);
+  trav_run<M>(w, tb);
   c.tb = &tb;
   SatBatch sb;
   sb.n_jobs = sb.n_tasks = sb.next_job = sb.ok = 0;
@@ -854,14 +855,15 @@ RS_INLINE uint32_t phase_p3b_body(ArenaState& s, const StaticData& w) {
 // scratch_ and global_ instructions (through generic pointers they would be flat ones, which wait on both the vector-memory
 // and the LDS counters and need 64-bit addresses).
 // UW: every lane steps in the same world (its pointer is then made wave-uniform).
-template <bool UW>
-RS_NOINL uint32_t phase_p3b_in(RS_PRIVATE_AS ArenaState* sp, const RS_CONST_AS StaticData* wp) {
+// M: where the state lives.
+template <bool UW, class M>
+RS_NOINL uint32_t phase_p3b_in(typename M::template Ptr<ArenaState> sp, const RS_CONST_AS StaticData* wp) {
   if (UW) wp = rs_uniform_ptr(wp);
-  return phase_p3b_body(*(ArenaState*)sp, *(const StaticData*)wp);
+  return phase_p3b_body<M>(*(ArenaState*)sp, *(const StaticData*)wp);
 }
-template <bool UW = false>
+template <bool UW = false, class M = InPrivate>
 RS_FN uint32_t phase_p3b(ArenaState& s, const StaticData& w) {
-  return phase_p3b_in<UW>((RS_PRIVATE_AS ArenaState*)&s, (const RS_CONST_AS StaticData*)&w);
+  return phase_p3b_in<UW, M>((typename M::template Ptr<ArenaState>)&s, (const RS_CONST_AS StaticData*)&w);
 }
 
 }  // namespace rs

@@ -90,7 +90,7 @@ RS_INLINE void phase_p4(ArenaState& s, const StaticData& w) {  // :100-150
 
 // ---- P5 rows (solver_constraint.cuh) -----------------------------------------------------------------------------------------
 constexpr int MAX_ROWS = 32;
-constexpr int MAX_SOLVER_BODIES = 8;
+constexpr int MAX_SOLVER_BODIES = 4;  // one per dynamic body, and the fixed one
 constexpr int SOLVER_ITERATIONS = 10;
 constexpr float ERP2 = 0.8f;
 constexpr float SPLIT_TURN_ERP = 0.1f;

@@ -1,9 +1,8 @@
 // The traversal stack of the BVH4 walks (wheel rays: quad_ray_shapes.cuh:377-406; mesh jobs: bvh.cuh:31-56): capacity 128
 // entries, and a push onto a full stack is dropped, as the reference's guard does.
 //
-// On the GPU the bottom TRAV_LDS entries of each lane's stack live in LDS (the kernel's dynamic shared memory, laid out
-// entry-major with the work-group's lanes contiguous, so the lanes of a wave touching the same depth hit distinct banks);
-// deeper entries spill to private memory. A pop is then an LDS read instead of a scratch round trip, which is what the
+// On the GPU the bottom TRAV_LDS entries of each lane's stack live in LDS (the kernel's dynamic shared memory, in a slice of
+// its own per lane, so that the lanes of a wave touching the same depth hit distinct banks); deeper entries spill to private memory. A pop is then an LDS read instead of a scratch round trip, which is what the
 // walk's node-by-node loop waits on. Kernels that step arenas launch with trav_lds_bytes(block) of dynamic LDS.
 #pragma once
 #include "rs_vec.h"
@@ -12,18 +11,22 @@ namespace rs {
 
 constexpr int TRAV_CAP = 128;
 constexpr int TRAV_LDS = 32;
-// The solver's bank (below): per solver body (up to 8) the mutable velocity and split-impulse deltas, its inverse mass and
+// The solver's bank (below): per solver body (up to 4) the mutable velocity and split-impulse deltas, its inverse mass and
 // whether it is a dynamic body (16 words); then the contact rows' applied impulses (up to 32), which the friction rows read.
-constexpr int BANK_BODIES = 8;
+constexpr int BANK_BODIES = 4;
 constexpr int BANK_BODY_WORDS = 16;
 constexpr int BANK_ROWS = 32;
 constexpr int BANK_WORDS = BANK_BODIES * BANK_BODY_WORDS + BANK_ROWS;
-// Both live in the same per-lane LDS slice, as does the broadphase sweep's working copy (rs_broad.h): each is used in a
-// phase of its own (the walks in P1 and P3b, the sweep in P3a, the bank in P5). Each wave of the work-group owns
-// 64 * LANE_LDS_WORDS words, entry-major: word k of lane l of wave v is at v * 64 * LANE_LDS_WORDS + k * 64 + l. The layout
-// does not depend on the work-group size (a kernel allocates whole waves), so the device functions never read it: they
-// need no dispatch-packet pointer, which every call would otherwise carry.
-constexpr int LANE_LDS_WORDS = TRAV_LDS > BANK_WORDS ? TRAV_LDS : BANK_WORDS;
+// The broadphase sweep's working copy (rs_broad.h): six u16 edge indices of 24 handles, then up to 64 edges of one axis.
+constexpr int SWEEP_WORDS = 3 * 24 + 64;
+// All three live in the same per-lane LDS slice: each is used in a phase of its own (the walks in P1 and P3b, the sweep in
+// P3a, the bank in P5). Each wave of the work-group owns 64 slices, lane-major: word k of lane l of wave v is at
+// (v * 64 + l) * LANE_LDS_WORDS + k. The slice is an odd number of words, so lanes reading the same k hit distinct banks,
+// and a wave that steps only a few arenas needs only as many slices. The layout does not depend on the work-group size (a
+// kernel allocates whole waves), so the device functions never read it: they need no dispatch-packet pointer, which every
+// call would otherwise carry.
+constexpr int LANE_LDS_WORDS = SWEEP_WORDS | 1;
+static_assert(LANE_LDS_WORDS >= TRAV_LDS && LANE_LDS_WORDS >= BANK_WORDS, "every use fits the slice");
 constexpr uint32_t WAVE_LDS_WORDS = 64u * (uint32_t)LANE_LDS_WORDS;
 RS_HD inline size_t trav_lds_bytes(uint32_t block) {
   return (size_t)WAVE_LDS_WORDS * ((block + 63u) / 64u) * sizeof(uint32_t);
@@ -39,8 +42,8 @@ __device__ inline uint32_t* wave_lds() {
   return (uint32_t*)(__attribute__((address_space(3))) uint32_t*)byte;
 }
 // Word k of this lane's slice, and word k of lane `slot`'s slice of the same wave.
-__device__ inline uint32_t* lane_word(uint32_t k) { return wave_lds() + (k * 64u + (threadIdx.x & 63u)); }
-__device__ inline uint32_t* wave_lane_word(uint32_t slot, uint32_t k) { return wave_lds() + (k * 64u + slot); }
+__device__ inline uint32_t* lane_word(uint32_t k) { return wave_lds() + ((threadIdx.x & 63u) * (uint32_t)LANE_LDS_WORDS + k); }
+__device__ inline uint32_t* wave_lane_word(uint32_t slot, uint32_t k) { return wave_lds() + (slot * (uint32_t)LANE_LDS_WORDS + k); }
 struct TravStack {
   uint32_t spill[TRAV_CAP - TRAV_LDS];
   int n;
@@ -66,13 +69,13 @@ struct DeltaBank {
   __device__ static float* at(uint32_t word) { return reinterpret_cast<float*>(lane_word(word)); }
   __device__ V3 get(int body, int field) const {
     const float* p = at((uint32_t)(body * BANK_BODY_WORDS + field * 3));
-    return V3{p[0], p[64], p[128]};
+    return V3{p[0], p[1], p[2]};
   }
   __device__ void set(int body, int field, V3 v) {
     float* p = at((uint32_t)(body * BANK_BODY_WORDS + field * 3));
     p[0] = v.x;
-    p[64] = v.y;
-    p[128] = v.z;
+    p[1] = v.y;
+    p[2] = v.z;
   }
   __device__ bool dynamic(int body) const { return *at((uint32_t)(body * BANK_BODY_WORDS + 15)) != 0.0f; }
   __device__ void set_dynamic(int body, bool d) { *at((uint32_t)(body * BANK_BODY_WORDS + 15)) = d ? 1.0f : 0.0f; }

@@ -353,18 +353,19 @@ enum PhaseStatus : int { PHASE_OK = 0, PHASE_UNIMPLEMENTED = -1, PHASE_BAD_INDEX
 
 // Phase k of one tick (0 P0, 1 P1, 2 P2, 3 P3a, 4 P3b, 5 P4, 6 P5, 7 P6, 8 P7, 9 P8): state at boundary k to boundary k + 1.
 // UW: every lane steps in the same world (its pointer is then made wave-uniform); k is the same in every lane.
-template <bool UW>
-RS_NOINL int run_phase_in(int kk, RS_PRIVATE_AS ArenaState* sp, const RS_CONST_AS StaticData* wp) {
+// M: where the state lives (InPrivate, InLds).
+template <bool UW, class M>
+RS_NOINL int run_phase_in(int kk, typename M::template Ptr<ArenaState> sp, const RS_CONST_AS StaticData* wp) {
   if (UW) wp = rs_uniform_ptr(wp);
   RS_UNIFORM_INDEX(kk);
   ArenaState& s = *(ArenaState*)sp;
   const StaticData& w = *(const StaticData*)wp;
   switch (kk) {
     case 0: phase_p0(s, w); return PHASE_OK;
-    case 1: phase_p1<UW>(s, w); return PHASE_OK;
+    case 1: phase_p1<UW, M>(s, w); return PHASE_OK;
     case 2: phase_p2(s, w); return PHASE_OK;
     case 3: phase_p3a(s, w); return PHASE_OK;
-    case 4: return phase_p3b<UW>(s, w) == 0 ? PHASE_OK : PHASE_UNIMPLEMENTED;
+    case 4: return phase_p3b<UW, M>(s, w) == 0 ? PHASE_OK : PHASE_UNIMPLEMENTED;
     case 5: phase_p4(s, w); return PHASE_OK;
     case 6: phase_p5(s, w); return PHASE_OK;
     case 7: phase_p6(s, w); return PHASE_OK;
@@ -373,18 +374,18 @@ RS_NOINL int run_phase_in(int kk, RS_PRIVATE_AS ArenaState* sp, const RS_CONST_A
     default: return PHASE_BAD_INDEX;
   }
 }
-// Every caller holds its arena in a lane-private copy and the StaticData in global memory. UW (uniform world): the
-// caller's lanes all step in the same world.
-template <bool UW = false>
+// Every caller holds its arena where M says (a lane-private copy, or LDS) and the StaticData in global memory. UW (uniform
+// world): the caller's lanes all step in the same world.
+template <bool UW = false, class M = InPrivate>
 RS_FN int run_phase(int kk, ArenaState& s, const StaticData& w) {
-  return run_phase_in<UW>(kk, (RS_PRIVATE_AS ArenaState*)&s, (const RS_CONST_AS StaticData*)&w);
+  return run_phase_in<UW, M>(kk, (typename M::template Ptr<ArenaState>)&s, (const RS_CONST_AS StaticData*)&w);
 }
 // One tick (base.rs step_tick): the ten phases in order.
-template <bool UW = false>
+template <bool UW = false, class M = InPrivate>
 RS_FN int step_tick(ArenaState& s, const StaticData& w) {
   int st = PHASE_OK;
   for (int kk = 0; kk < NUM_PHASES; ++kk)
-    if (run_phase<UW>(kk, s, w) != PHASE_OK) st = PHASE_UNIMPLEMENTED;
+    if (run_phase<UW, M>(kk, s, w) != PHASE_OK) st = PHASE_UNIMPLEMENTED;
   return st;
 }
 RS_FN bool ball_scored(const ArenaState& s, const StaticData& w) {  // base.rs is_ball_scored, Soccar

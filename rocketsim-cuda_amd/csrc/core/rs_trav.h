@@ -92,17 +92,25 @@ RS_FN void trav_walk(const StaticData& w, TravBatch& tb) {  // each job's own de
   }
 }
 #if defined(__HIP_DEVICE_COMPILE__)
-// The pooled walk's LDS area (words of the wave's 64 lane slices): job records, per-job leaf counts and first slots, the
-// control words, two frontiers and the leaf list.
-constexpr uint32_t PT_JOBS = 64 * TJ_MAX, PT_Q = 1024, PT_L = 1024, PT_DEPTH = 15;
-constexpr uint32_t PT_REC = 10;  // a job record: box (6 words), the address of its mesh's first node (2), the mesh's node count
-constexpr uint32_t PT_JOB_W = 0, PT_CNT_W = PT_JOB_W + PT_REC * PT_JOBS, PT_START_W = PT_CNT_W + PT_JOBS, PT_CTRL_W = PT_START_W + PT_JOBS,
-                   PT_Q_W = PT_CTRL_W + 4, PT_L_W = PT_Q_W + 4 * PT_Q, PT_WORDS = PT_L_W + 2 * PT_L;
-static_assert(PT_WORDS <= 64u * (uint32_t)LANE_LDS_WORDS, "the pooled walk fits the wave's LDS slices");
+// The pooled walk's LDS area (the wave's slices taken together): job records, per-job leaf counts and first slots, the
+// control words, two frontiers and the leaf list, for waves of ARENAS arenas.
+template <uint32_t ARENAS>
+struct PoolArea {
+  static constexpr uint32_t JOBS = ARENAS * TJ_MAX, Q = ARENAS == 64 ? 940 : 256, L = ARENAS == 64 ? 960 : 256;
+  static constexpr uint32_t REC = 10;  // a job record: box (6 words), the address of its mesh's first node (2), the mesh's node count
+  static constexpr uint32_t JOB_W = 0, CNT_W = JOB_W + REC * JOBS, START_W = CNT_W + JOBS, CTRL_W = START_W + JOBS, Q_W = CTRL_W + 4,
+                            L_W = Q_W + 4 * Q, WORDS = L_W + 2 * L;
+};
+static_assert(PoolArea<64>::WORDS <= WAVE_LDS_WORDS, "the pooled walk fits the wave's LDS slices");
+constexpr uint32_t PT_DEPTH = 15;
 __device__ inline uint32_t* wave_word(uint32_t j) { return wave_lds() + j; }
-__device__ inline uint32_t* pt_q(uint32_t which, uint32_t i, uint32_t k) { return wave_word(PT_Q_W + which * 2 * PT_Q + 2 * i + k); }
 
+template <uint32_t ARENAS>
 __device__ inline bool trav_pooled(const StaticData& w, TravBatch& tb) {
+  using A = PoolArea<ARENAS>;
+  constexpr uint32_t PT_JOBS = A::JOBS, PT_Q = A::Q, PT_L = A::L, PT_REC = A::REC, PT_JOB_W = A::JOB_W, PT_CNT_W = A::CNT_W,
+                     PT_START_W = A::START_W, PT_CTRL_W = A::CTRL_W, PT_L_W = A::L_W;
+  auto pt_q = [](uint32_t which, uint32_t i, uint32_t k) { return wave_word(A::Q_W + which * 2 * A::Q + 2 * i + k); };
   const uint32_t lane = threadIdx.x & 63u;
   const uint64_t below = lane ? (~0ull >> (64u - lane)) : 0ull;
   const uint64_t active = __ballot(1);
@@ -263,9 +271,10 @@ __device__ inline bool trav_pooled(const StaticData& w, TravBatch& tb) {
   return true;
 }
 #endif
+template <class M>
 RS_FN void trav_run(const StaticData& w, TravBatch& tb) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  if (trav_pooled(w, tb)) return;
+  if (trav_pooled<M::ARENAS>(w, tb)) return;
 #endif
   trav_walk(w, tb);
 }

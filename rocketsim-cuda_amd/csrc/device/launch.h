@@ -42,6 +42,11 @@ hipError_t launch_sim8_ticks(hipStream_t st, const Sim8Args& p, uint32_t block, 
 // first; order: null or a permutation of the ceil(n / 64) block indices.
 hipError_t launch_run_queue(hipStream_t st, const Sim8Args& p, uint32_t decisions, uint32_t block, const uint32_t* order,
                             uint32_t* next, uint32_t workgroups);
+// The kernel of small batches (small_kernels.hip): n <= SMALL_MAX_N arenas, `decisions` decisions, with a trace for one.
+constexpr uint32_t SMALL_MAX_N = 3072;  // three arenas on each of 1,024 SIMDs
+constexpr uint32_t SPREAD_MAX_N = 32768;  // 32 arenas on each: up to here a work-group of SIM8_BLOCK is a wave of 32 lanes
+hipError_t launch_small(hipStream_t st, const Sim8Args& p, uint32_t decisions);
+hipError_t small_static_lds(size_t* bytes);
 // The largest static LDS (group segment of fixed size) of the kernels that step arenas: their device functions address the
 // dynamic LDS from LDS address 0, which holds only while this is 0.
 hipError_t stepping_static_lds(size_t* bytes);

@@ -13,6 +13,7 @@
 //   k_sim8_ticks                    one decision as several launches of a few ticks (the state in HBM between them)
 //   k_run                           several decisions per launch, the arena held in the lane from first to last
 //   k_run_queue                     k_run with persistent work-groups taking AoSoA blocks from a queue
+//   k_small (small_kernels.hip)     k_sim8 and k_run for small batches, the states in LDS
 //   k_copy_words                    a streaming copy of a state buffer (restores between timed runs)
 #include "device/launch.h"
 #include "device/aosoa.h"
@@ -216,7 +217,16 @@ hipError_t launch_step_tick(hipStream_t st, uint32_t* buf, const StaticData* w, 
   k_step_tick<<<grid_of(n, SIM8_BLOCK), SIM8_BLOCK, trav_lds_bytes(SIM8_BLOCK), st>>>(buf, w, n, status);
   return hipGetLastError();
 }
+// The lanes of a work-group that asks for SIM8_BLOCK, the production size: one wave, of fewer arenas where the batch leaves
+// SIMDs idle, since a wave pays for the union of its arenas' paths. 32 lanes as long as they fill at most one wave per
+// SIMD; fewer lose more to the half-empty rows of private memory that crowd the caches than their shorter unions gain
+// (ms per decision at 16 / 32 / 64 lanes, contact mix: 4,096 arenas 3.26 / 3.55 / 4.07, 16,384 arenas 4.54 / 4.02 / 4.44,
+// 32,768 arenas 8.43 / 4.91 / 5.18; kickoffs: 3,500 arenas 1.47 / 1.33 / 1.35, 16,384 arenas 2.04 / 1.64 / 1.63). Any
+// other size is the caller's own choice.
+static uint32_t wave_lanes(uint32_t n, uint32_t block) { return block == SIM8_BLOCK && n <= SPREAD_MAX_N ? 32u : block; }
 hipError_t launch_run(hipStream_t st, const Sim8Args& p, uint32_t decisions, uint32_t block) {
+  if (block == SIM8_BLOCK && p.n <= SMALL_MAX_N) return launch_small(st, p, decisions);
+  block = wave_lanes(p.n, block);
   k_run<<<grid_of(p.n, block), block, trav_lds_bytes(block), st>>>(p, decisions);
   return hipGetLastError();
 }
@@ -238,6 +248,8 @@ hipError_t stepping_static_lds(size_t* bytes) {
                            (const void*)k_sim8_ticks<false>, (const void*)k_sim8_ticks<true>, (const void*)k_run,
                            (const void*)k_run_queue};
   size_t most = 0;
+  hipError_t small = small_static_lds(&most);
+  if (small != hipSuccess) return small;
   for (const void* k : kernels) {
     hipFuncAttributes a;
     hipError_t e = hipFuncGetAttributes(&a, k);
@@ -262,6 +274,10 @@ hipError_t launch_run_queue(hipStream_t st, const Sim8Args& p, uint32_t decision
   return hipGetLastError();
 }
 hipError_t launch_sim8(hipStream_t st, const Sim8Args& p, uint32_t block) {
+  if (!p.cycles) {  // a timed call's clock is the wave's it asked for
+    if (block == SIM8_BLOCK && p.n <= SMALL_MAX_N) return launch_small(st, p, 1);
+    block = wave_lanes(p.n, block);
+  }
   const size_t lds = trav_lds_bytes(block);  // the BVH walks' traversal stacks
   const dim3 g = grid_of(p.n, block);
   if (p.trace && p.variant) k_sim8<true, true><<<g, block, lds, st>>>(p);

@@ -495,6 +495,13 @@ int rsim_run_queued(rsim_device* dev, rsim_states* states, const rsim_world* wor
   if (variant && variant->n < n) return fail(RSIM_ERR_SHORT, "rsim_run_queued: variant buffer too short");
   if (order && order->n < nblocks) return fail(RSIM_ERR_SHORT, "rsim_run_queued: order shorter than the block count");
   if (!n || !decisions) return RSIM_OK;
+  if (!workgroups && !order && block == RSIM_SIM8_BLOCK && n <= rs::dev::SPREAD_MAX_N) {
+    // every wave of the batch is resident at once: nothing to queue for, and rsim_run's narrower waves fill more SIMDs
+    rs::dev::Sim8Args p{states->d, world->d, world->count, variant ? variant->d : nullptr,
+                        reinterpret_cast<const Controls*>(controls->d), results->d, n, nullptr, nullptr};
+    RSIM_HIP(rs::dev::launch_run(dev->stream, p, decisions, block), "run_queued launch");
+    return RSIM_OK;
+  }
   if (!workgroups) workgroups = rs::dev::run_queue_capacity(block);
   const uint32_t waves = block / 64;
   const uint32_t useful = (nblocks + waves - 1) / waves;  // more work-groups than that would find the queue empty

@@ -1,0 +1,88 @@
+"""The launch shapes of the production block by batch size, each against the oracle word for word: one and three arenas per
+wave with the states in LDS (small_kernels.hip), waves of 32 lanes, and full waves. The sizes are the edges of those
+ranges and their remainders; each shape also with a world table, a trace, several decisions per launch, the queue's
+entry point, goals, overflows and a world index past the table."""
+import numpy as np
+import pytest
+
+import forced_cases as fc
+from conftest import first_diff
+from helpers import TICK_WORDS
+
+pytestmark = pytest.mark.gpu
+
+EDGES = [1, 63, 511, 512, 513, 514, 515, 3071, 3072, 3073, 32767, 32768, 32769]
+
+
+def same(got, want, what):
+    fd = first_diff(got[:, :TICK_WORDS], want[:, :TICK_WORDS])
+    assert fd is None, "%s: arena %d word %d differs" % (what, fd[0], fd[1])
+
+
+@pytest.mark.parametrize("n", EDGES)
+def test_sim8_at_the_edges(rsim, oracle, world, device, dev_world, n):
+    print("[case] sim8, %d contact arenas, 2 decisions" % n, flush=True)
+    states = rsim.sample_arenas(world, rsim.SCEN_CONTACT, 900, n)
+    d, r, cpu = device.upload_states(states), device.alloc_words(n), states.copy()
+    for k in range(2):
+        ctl = rsim.sample_controls(901, k, n)
+        device.sim8(d, dev_world, device.upload_controls(ctl), r)
+        assert np.array_equal(device.read_words(r), oracle.sim8(cpu, world, ctl, threads=8)), k
+    same(device.download_states(d), cpu, "sim8 %d" % n)
+
+
+@pytest.mark.parametrize("entry", ["run", "run_queued"])
+@pytest.mark.parametrize("n", [2, 512, 514, 3072, 3075, 4100])
+def test_worlds_and_decisions(rsim, oracle, device, n, entry):
+    print("[case] %s, %d arenas in 5 worlds, 3 decisions" % (entry, n), flush=True)
+    worlds = np.stack([rsim.build_world(p, p) for p in range(5)])
+    variant = np.random.default_rng(n).integers(0, 5, n).astype(np.uint32)
+    states = rsim.sample_arenas_in(worlds, variant, rsim.SCEN_OPEN_CONTACT, 902)
+    ctl = np.stack([rsim.sample_controls(903, k, n) for k in range(3)])
+    d, dw = device.upload_states(states), device.upload_worlds(worlds)
+    c, r, v = device.upload_words(ctl), device.alloc_words(3 * n), device.upload_words(variant)
+    getattr(device, entry)(d, dw, c, r, 3, variant=v)
+    got, cpu = device.read_words(r).reshape(3, n), states.copy()
+    for k in range(3):
+        assert np.array_equal(got[k], oracle.sim8_in(cpu, worlds, variant, ctl[k], threads=8)), k
+    same(device.download_states(d), cpu, "%s %d" % (entry, n))
+    bad = variant.copy()
+    bad[n // 2] = 5  # past the table: flagged, and the arena left as it was
+    d2 = device.upload_states(states)
+    device.sim8_variants(d2, dw, device.upload_words(bad), device.upload_controls(ctl[0]), r)
+    one, after = device.read_words(r, n), device.download_states(d2)
+    assert one[n // 2] == rsim.SIM8_BAD_VARIANT and np.array_equal(after[n // 2], states[n // 2])
+    assert np.array_equal(np.delete(one, n // 2), np.delete(got[0], n // 2))
+
+
+@pytest.mark.parametrize("variants", [False, True])
+@pytest.mark.parametrize("n", [128, 700, 3200])
+def test_trace_goals_and_overflow(rsim, oracle, world, device, dev_world, n, variants):
+    print("[case] traced sim8, %d arenas with goals on every tick and overflows, variants %d" % (n, variants), flush=True)
+    goals, over = fc.goal_states(rsim, world, 7)[0][::2], fc.overflow_states(rsim, world, 64, 17)
+    some = np.concatenate([goals, over])[:n]
+    states = np.concatenate([some, rsim.sample_arenas(world, rsim.SCEN_GOALFRAME, 904, n)])[:n]
+    states = np.ascontiguousarray(states[np.random.default_rng(3).permutation(n)])
+    ctl = np.zeros((n, 16), np.uint32)
+    d, r = device.upload_states(states), device.alloc_words(n)
+    trace = device.alloc_words(8 * rsim.aosoa_words(n))
+    if variants:
+        device.sim8_variants(d, dev_world, device.upload_words(np.zeros(n, np.uint32)), device.upload_controls(ctl), r, trace=trace)
+    else:
+        device.sim8(d, dev_world, device.upload_controls(ctl), r, trace=trace)
+    word = device.read_words(r)
+    slabs = device.read_words(trace).reshape(8, -1)
+    cpu, ticks = states.copy(), states.copy()
+    assert np.array_equal(word, oracle.sim8(cpu, world, ctl, threads=8))
+    assert ((word & 0xFF) > 0).any() and (word & rsim.SIM8_OVERFLOW).any()
+    same(device.download_states(d), cpu, "traced %d" % n)
+    scored = word & 0xFF
+    for t in range(1, 9):
+        live = (scored == 0) | (scored >= t)
+        idx = np.nonzero(live[:100])[0]
+        for a in idx:
+            oracle.set_controls(ticks[a], ctl[a])
+            oracle.step_tick(ticks[a], world)
+        got = rsim.aosoa_unpack(slabs[t - 1], n)
+        same(got[idx], ticks[idx], "trace tick %d" % t)
+        assert not got[~live].any(), "ticks after a goal are not written"
