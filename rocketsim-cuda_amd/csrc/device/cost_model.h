@@ -9,7 +9,8 @@ constexpr int COST_FEATURES = 48;
 // offsets into the fp32 parameter vector: W1[48][64], b1[64], W2[64][64], b2[64], W3[64][2], b3[2]
 constexpr int COST_W1 = 0, COST_B1 = 48 * 64, COST_W2 = COST_B1 + 64, COST_B2 = COST_W2 + 64 * 64, COST_W3 = COST_B2 + 64,
               COST_B3 = COST_W3 + 64 * 2, COST_PARAMS = COST_B3 + 2;
-constexpr int COST_ACT_WORDS = 48 + 64 + 64 + 2 + 64 + 64;  // per training arena: x, h1, h2, dy, dh1, dh2
+// Training scratch words per batch row (the caller's buffer): room for one COST_PARAMS share of the gradient per 25 rows.
+constexpr int COST_ACT_WORDS = 306;
 
 // The order by predicted cost: ORDER_BUCKETS buckets of the normalised log cost over [ORDER_HI - ORDER_BUCKETS /
 // ORDER_SCALE, ORDER_HI), bucket 0 the most expensive (above the range), NaN in the last.

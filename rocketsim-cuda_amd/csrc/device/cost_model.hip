@@ -4,9 +4,9 @@
 //   k_features     48 features per arena from the AoSoA-64 states (positions, velocities, wall and gap distances, counts)
 //   k_mlp_infer    inference: bf16 weights and activations, fp32 accumulation, on v_mfma_f32_16x16x16_bf16 (one wave, 64
 //                  arenas as four 16-row tiles; weights staged transposed in LDS, activations re-laid through LDS)
-//   k_mlp_train    training forward + backward per arena in fp32 (the same bf16 rounding points as inference; the rounding
-//                  is treated as the identity in the backward pass), writing activations and their gradients
-//   k_mlp_reduce   parameter gradients: sums over the batch of outer products of activations and gradients
+//   k_mlp_train    training forward + backward in fp32 (the same bf16 rounding points as inference; the rounding is treated
+//                  as the identity in the backward pass), and each work-group's share of the parameter gradient
+//   k_mlp_reduce   the parameter gradient: the sum of the shares
 //   k_adam         Adam update of the fp32 master parameters
 //   k_gather_words / k_scatter_words / k_gather_states   the regrouping permutations (states stay AoSoA-64)
 //
@@ -141,73 +141,168 @@ __global__ void __launch_bounds__(64) k_mlp_infer(const float* __restrict__ para
 }
 
 // ---- training ------------------------------------------------------------------------------------------------------------------
-// Per arena: the forward pass in fp32 with bf16-rounded weights and activations (the inference kernel's rounding points,
-// its sums in a different order), the losses (squared error on the normalised log cost, logistic loss on the contact
-// flag, both averaged over the batch) and the backward pass down to the first layer's pre-activations.
-__global__ void __launch_bounds__(128) k_mlp_train(const float* __restrict__ params, const float* __restrict__ feat,
+// One work-group per TRAIN_ROWS batch rows (and every gridDim.x * TRAIN_ROWS further ones): the forward pass in fp32 with
+// bf16-rounded weights and activations (the inference kernel's rounding points; each sum runs over its inputs in order, as
+// one accumulator), the losses (squared error on the normalised log cost, logistic loss on the contact flag, both averaged
+// over the batch), the backward pass, and the rows' share of the parameter gradient, kept in registers over the group's
+// rows and written once. k_mlp_reduce sums the groups' shares in a fixed order.
+//
+// Forward: lane j of each wave holds column j of W1 and W2 in registers and takes eight rows, whose inputs it reads from LDS
+// as broadcasts. The layer-1 gradient and the two weight gradients are contractions in fp32 and run on
+// v_mfma_f32_16x16x4_f32 (A: row l % 16, k = l / 16; B: k = l / 16, column l % 16; D: rows 4 (l / 16) + 0..3, column
+// l % 16). 4,096 rows: 128 groups, one wave per SIMD on half the CUs; bound by the forward's instruction chain. Before, one
+// lane per row wrote its activations to memory and one thread per parameter summed 4,096 rows in turn: 1,340 us.
+constexpr uint32_t TRAIN_ROWS = 32, TRAIN_MAX_GROUPS = 256;
+constexpr int TS = 80;  // LDS row stride of the 64-wide activations: the four rows an MFMA operand reads fall in distinct banks
+__global__ void __launch_bounds__(256) k_mlp_train(const float* __restrict__ params, const float* __restrict__ feat,
                                                    const float* __restrict__ target, const float* __restrict__ contact,
-                                                   uint32_t b, float* __restrict__ acts, float* __restrict__ loss) {
-  uint32_t a = blockIdx.x * blockDim.x + threadIdx.x;
-  if (a >= b) return;
+                                                   uint32_t b, float* __restrict__ shares, float* __restrict__ loss) {
+  __shared__ float4 x4[TRAIN_ROWS * COST_FEATURES / 4], h14[TRAIN_ROWS * TS / 4], h24[TRAIN_ROWS * TS / 4];
+  __shared__ float d1[TRAIN_ROWS * TS], d2[TRAIN_ROWS * TS], dy[TRAIN_ROWS * 2];
+  float *x = (float*)x4, *h1 = (float*)h14, *h2 = (float*)h24;
   const float *W1 = params + COST_W1, *B1 = params + COST_B1, *W2 = params + COST_W2, *B2 = params + COST_B2,
               *W3 = params + COST_W3, *B3 = params + COST_B3;
-  float* row = acts + (size_t)a * COST_ACT_WORDS;  // x[48] h1[64] h2[64] dy[2] dh1[64] dh2[64]
-  float *x = row, *h1 = row + 48, *h2 = row + 112, *dy = row + 176, *dh1 = row + 178, *dh2 = row + 242;
-  for (int i = 0; i < COST_FEATURES; ++i) x[i] = bf16_round(feat[(size_t)a * COST_FEATURES + i]);
-  for (int j = 0; j < 64; ++j) {
-    float s = 0.0f;
-    for (int i = 0; i < COST_FEATURES; ++i) s += bf16_round(W1[i * 64 + j]) * x[i];
-    s += B1[j];
-    h1[j] = bf16_round(s > 0.0f ? s : 0.0f);
-  }
-  for (int j = 0; j < 64; ++j) {
-    float s = 0.0f;
-    for (int i = 0; i < 64; ++i) s += bf16_round(W2[i * 64 + j]) * h1[i];
-    s += B2[j];
-    h2[j] = bf16_round(s > 0.0f ? s : 0.0f);
-  }
-  float y[2];
-  for (int k = 0; k < 2; ++k) {
-    float s = 0.0f;
-    for (int i = 0; i < 64; ++i) s += bf16_round(W3[i * 2 + k]) * h2[i];
-    y[k] = s + B3[k];
-  }
+  constexpr int F = COST_FEATURES, PER = (int)TRAIN_ROWS / 4;  // rows per wave
+  const int tid = threadIdx.x, l = tid % 64, wave = tid / 64, lr = l % 16, lk = l / 16;
+  float w1[F], w2[64], w2r[16];
+#pragma unroll
+  for (int i = 0; i < F; ++i) w1[i] = bf16_round(W1[i * 64 + l]);
+#pragma unroll
+  for (int i = 0; i < 64; ++i) w2[i] = bf16_round(W2[i * 64 + l]);
+#pragma unroll
+  for (int k = 0; k < 16; ++k) w2r[k] = bf16_round(W2[(wave * 16 + lr) * 64 + 4 * k + lk]);  // dh1's B operand: W2 transposed
+  const float b1 = B1[l], b2 = B2[l], w3a = bf16_round(W3[l * 2]), w3b = bf16_round(W3[l * 2 + 1]);
   const float inv_b = 1.0f / (float)b;
-  float e = y[0] - target[a], c = contact[a];
-  float sig = 1.0f / (1.0f + expf(-y[1]));
-  dy[0] = 2.0f * e * inv_b;
-  dy[1] = (sig - c) * inv_b;
-  float sp = y[1] > 0.0f ? y[1] + log1pf(expf(-y[1])) : log1pf(expf(y[1]));  // softplus
-  loss[a] = e * e + (sp - c * y[1]);
-  for (int j = 0; j < 64; ++j) {
-    float g = bf16_round(W3[j * 2 + 0]) * dy[0] + bf16_round(W3[j * 2 + 1]) * dy[1];
-    dh2[j] = h2[j] > 0.0f ? g : 0.0f;
+  v4f g1[3] = {}, g2[4] = {};
+  float g_vec = 0.0f, g_b3 = 0.0f;
+  for (uint32_t r0 = blockIdx.x * TRAIN_ROWS; r0 < b; r0 += gridDim.x * TRAIN_ROWS) {
+    const uint32_t rows = b - r0 < TRAIN_ROWS ? b - r0 : TRAIN_ROWS;
+    for (uint32_t e = tid; e < TRAIN_ROWS * F; e += 256)  // rows past the batch: zeros, and no share below
+      x[e] = e < rows * F ? bf16_round(feat[(size_t)r0 * F + e]) : 0.0f;
+    __syncthreads();
+    // two rows at a time: enough independent sums to fill the pipeline without holding all rows' inputs in registers
+#pragma unroll 1
+    for (int r = wave * PER; r < (wave + 1) * PER; r += 2) {
+      float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll
+      for (int i = 0; i < F; i += 4) {
+        const float4 v = x4[(r * F + i) / 4], u = x4[((r + 1) * F + i) / 4];
+        s0 += w1[i] * v.x, s1 += w1[i] * u.x;
+        s0 += w1[i + 1] * v.y, s1 += w1[i + 1] * u.y;
+        s0 += w1[i + 2] * v.z, s1 += w1[i + 2] * u.z;
+        s0 += w1[i + 3] * v.w, s1 += w1[i + 3] * u.w;
+      }
+      s0 += b1, s1 += b1;
+      h1[r * TS + l] = (uint32_t)r < rows ? bf16_round(s0 > 0.0f ? s0 : 0.0f) : 0.0f;
+      h1[(r + 1) * TS + l] = (uint32_t)r + 1 < rows ? bf16_round(s1 > 0.0f ? s1 : 0.0f) : 0.0f;
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int r = wave * PER; r < (wave + 1) * PER; r += 2) {
+      float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 64; i += 4) {
+        const float4 v = h14[(r * TS + i) / 4], u = h14[((r + 1) * TS + i) / 4];
+        s0 += w2[i] * v.x, s1 += w2[i] * u.x;
+        s0 += w2[i + 1] * v.y, s1 += w2[i + 1] * u.y;
+        s0 += w2[i + 2] * v.z, s1 += w2[i + 2] * u.z;
+        s0 += w2[i + 3] * v.w, s1 += w2[i + 3] * u.w;
+      }
+      s0 += b2, s1 += b2;
+      h2[r * TS + l] = (uint32_t)r < rows ? bf16_round(s0 > 0.0f ? s0 : 0.0f) : 0.0f;
+      h2[(r + 1) * TS + l] = (uint32_t)r + 1 < rows ? bf16_round(s1 > 0.0f ? s1 : 0.0f) : 0.0f;
+    }
+    __syncthreads();
+    if (l < 2 * PER) {  // one lane per (row, output): its sum over h2 in order, then the row's losses and their gradients
+      const int r = wave * PER + l / 2, k = l % 2;
+      float y = 0.0f;
+      for (int i = 0; i < 64; i += 4) {
+        const float4 v = h24[(r * TS + i) / 4];
+        y += bf16_round(W3[i * 2 + k]) * v.x;
+        y += bf16_round(W3[(i + 1) * 2 + k]) * v.y;
+        y += bf16_round(W3[(i + 2) * 2 + k]) * v.z;
+        y += bf16_round(W3[(i + 3) * 2 + k]) * v.w;
+      }
+      y += B3[k];
+      const bool valid = (uint32_t)r < rows;
+      const float want = valid ? (k == 0 ? target[r0 + r] : contact[r0 + r]) : 0.0f;
+      float part, grad;
+      if (k == 0) {
+        const float e = y - want;
+        part = e * e;
+        grad = 2.0f * e * inv_b;
+      } else {
+        const float sig = 1.0f / (1.0f + expf(-y));
+        const float sp = y > 0.0f ? y + log1pf(expf(-y)) : log1pf(expf(y));  // softplus
+        part = sp - want * y;
+        grad = (sig - want) * inv_b;
+      }
+      const float other = __shfl_xor(part, 1);
+      if (valid && k == 0) loss[r0 + r] = part + other;
+      dy[r * 2 + k] = valid ? grad : 0.0f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+      const int r = wave * PER + q;
+      const float g = w3a * dy[r * 2] + w3b * dy[r * 2 + 1];
+      d2[r * TS + l] = h2[r * TS + l] > 0.0f ? g : 0.0f;
+    }
+    __syncthreads();
+    v4f acc[2] = {};  // dh1 = dh2 W2^T: this wave's 16 columns of all rows
+#pragma unroll
+    for (int k = 0; k < 16; ++k)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(d2[(t * 16 + lr) * TS + 4 * k + lk], w2r[k], acc[t], 0, 0, 0);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int at = (t * 16 + 4 * lk + i) * TS + wave * 16 + lr;
+        d1[at] = h1[at] > 0.0f ? acc[t][i] : 0.0f;
+      }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < (int)TRAIN_ROWS / 4; ++k) {  // the weights' shares: input activations transposed times output gradients
+      const int r = 4 * k + lk;
+      const float ah = h1[r * TS + wave * 16 + lr], bd = d1[r * TS + wave * 16 + lr];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) g2[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ah, d2[r * TS + j * 16 + lr], g2[j], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) g1[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[r * F + i * 16 + lr], bd, g1[i], 0, 0, 0);
+    }
+    // the rest, one per thread: W3 (128), b1 (64), b2 (64); b3 beside them
+    for (int r = 0; r < (int)TRAIN_ROWS; ++r)
+      g_vec += tid < 128 ? h2[r * TS + tid / 2] * dy[r * 2 + tid % 2] : tid < 192 ? d1[r * TS + l] : d2[r * TS + l];
+    if (tid < 2)
+      for (int r = 0; r < (int)TRAIN_ROWS; ++r) g_b3 += dy[r * 2 + tid];
+    __syncthreads();  // the next rows overwrite the LDS
   }
-  for (int i = 0; i < 64; ++i) {
-    float g = 0.0f;
-    for (int j = 0; j < 64; ++j) g += bf16_round(W2[i * 64 + j]) * dh2[j];
-    dh1[i] = h1[i] > 0.0f ? g : 0.0f;
+  float* out = shares + (size_t)blockIdx.x * COST_PARAMS;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) out[COST_W2 + (wave * 16 + 4 * lk + i) * 64 + j * 16 + lr] = g2[j][i];
+#pragma unroll
+    for (int t = 0; t < 3; ++t) out[COST_W1 + (t * 16 + 4 * lk + i) * 64 + wave * 16 + lr] = g1[t][i];
   }
+  out[tid < 128 ? COST_W3 + tid : tid < 192 ? COST_B1 + l : COST_B2 + l] = g_vec;
+  if (tid < 2) out[COST_B3 + tid] = g_b3;
 }
 
-// grad[p] = sum over the batch of (input activation) x (output gradient) for the weights, (output gradient) for the biases.
-__global__ void __launch_bounds__(256) k_mlp_reduce(const float* __restrict__ acts, uint32_t b, float* __restrict__ grad) {
-  uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= COST_PARAMS) return;
-  int in_off = -1, out_off, i = 0, j;
-  if (p < (uint32_t)COST_B1) { i = p / 64; j = p % 64; in_off = 0; out_off = 178; }
-  else if (p < (uint32_t)COST_W2) { j = p - COST_B1; out_off = 178; }
-  else if (p < (uint32_t)COST_B2) { uint32_t q = p - COST_W2; i = q / 64; j = q % 64; in_off = 48; out_off = 242; }
-  else if (p < (uint32_t)COST_W3) { j = p - COST_B2; out_off = 242; }
-  else if (p < (uint32_t)COST_B3) { uint32_t q = p - COST_W3; i = q / 2; j = q % 2; in_off = 112; out_off = 176; }
-  else { j = p - COST_B3; out_off = 176; }
+// grad[p] = the groups' shares summed: 64 parameters per work-group, each by four threads over every fourth share.
+__global__ void __launch_bounds__(256) k_mlp_reduce(const float* __restrict__ shares, uint32_t groups, float* __restrict__ grad) {
+  __shared__ float part[4][64];
+  const uint32_t l = threadIdx.x % 64, q = threadIdx.x / 64, p = blockIdx.x * 64 + l;
   float s = 0.0f;
-  for (uint32_t a = 0; a < b; ++a) {
-    const float* row = acts + (size_t)a * COST_ACT_WORDS;
-    float g = row[out_off + j];
-    s += in_off >= 0 ? row[in_off + i] * g : g;
+  if (p < (uint32_t)COST_PARAMS) {
+#pragma unroll 8
+    for (uint32_t g = q; g < groups; g += 4) s += shares[(size_t)g * COST_PARAMS + p];
   }
-  grad[p] = s;
+  part[q][l] = s;
+  __syncthreads();
+  if (q == 0 && p < (uint32_t)COST_PARAMS) grad[p] = (part[0][l] + part[1][l]) + (part[2][l] + part[3][l]);
 }
 
 __global__ void __launch_bounds__(256) k_adam(float* __restrict__ params, float* __restrict__ m, float* __restrict__ v,
@@ -388,8 +483,16 @@ hipError_t launch_mlp_infer(hipStream_t st, const float* params, const float* fe
 }
 hipError_t launch_mlp_train(hipStream_t st, const float* params, const float* feat, const float* target, const float* contact,
                             uint32_t b, float* acts, float* loss, float* grad) {
-  k_mlp_train<<<blocks_of(b, 128), 128, 0, st>>>(params, feat, target, contact, b, acts, loss);
-  k_mlp_reduce<<<blocks_of(COST_PARAMS, 256), 256, 0, st>>>(acts, b, grad);
+  // as many groups as have rows, the chip has CUs for, and the scratch (COST_ACT_WORDS per row) has room for shares of
+  const uint32_t rows = (b + TRAIN_ROWS - 1) / TRAIN_ROWS, room = (uint32_t)((uint64_t)b * COST_ACT_WORDS / COST_PARAMS);
+  uint32_t groups = rows < TRAIN_MAX_GROUPS ? rows : TRAIN_MAX_GROUPS;
+  if (groups > room) groups = room;
+  if (groups <= 1) {  // one group's share is the gradient
+    k_mlp_train<<<1, 256, 0, st>>>(params, feat, target, contact, b, grad, loss);
+    return hipGetLastError();
+  }
+  k_mlp_train<<<groups, 256, 0, st>>>(params, feat, target, contact, b, acts, loss);
+  k_mlp_reduce<<<blocks_of(COST_PARAMS, 64), 256, 0, st>>>(acts, groups, grad);
   return hipGetLastError();
 }
 hipError_t launch_adam(hipStream_t st, float* params, float* m, float* v, const float* grad, float lr, float bc1, float bc2) {
