@@ -202,6 +202,9 @@ int rsim_set_permutation(rsim_device* dev, const uint32_t* perm, uint32_t n, rsi
  * at least dst->n indices; an index past src leaves that arena of dst as it was). With dst->n == src->n and a permutation
  * this is a reordering; with a smaller dst, a sample. */
 int rsim_gather_states(rsim_device* dev, const rsim_states* src, const rsim_words* perm, rsim_states* dst);
+/* The arenas of `states` reordered in place: arena i becomes the former arena perm[i]. perm holds at least n indices, a
+ * permutation of 0..n-1 (rsim_cost_order's output); spare: another buffer of n arenas, whose contents are undefined after. */
+int rsim_permute_states(rsim_device* dev, rsim_states* states, const rsim_words* perm, rsim_states* spare);
 /* Items of words_per_item words: gather (dst[i] = src[perm[i]]) or, with scatter != 0, dst[perm[i]] = src[i]. */
 int rsim_permute_words(rsim_device* dev, const rsim_words* src, const rsim_words* perm, uint32_t n, uint32_t words_per_item,
                        int scatter, rsim_words* dst);
@@ -213,7 +216,8 @@ int rsim_phase(rsim_device* dev, int k, rsim_states* states, const rsim_world* w
 int rsim_step_tick(rsim_device* dev, rsim_states* states, const rsim_world* world, int32_t* status_out);
 
 /* HIP graphs over the device's stream: between rsim_capture_begin and rsim_capture_end the asynchronous entry points
- * (rsim_sim8*, rsim_run, rsim_copy_states, rsim_cost_features / predict / order, rsim_gather_states, rsim_permute_words)
+ * (rsim_sim8*, rsim_run, rsim_copy_states, rsim_cost_features / predict / order, rsim_gather_states, rsim_permute_states,
+ * rsim_permute_words)
  * are recorded instead of run; a synchronising call fails inside a capture and ends it. rsim_graph_launch replays the
  * recorded work on the stream (asynchronously) with the buffers it was recorded with. No counterpart in the reference. */
 typedef struct rsim_graph rsim_graph;

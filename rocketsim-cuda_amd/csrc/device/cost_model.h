@@ -14,7 +14,7 @@ constexpr int COST_ACT_WORDS = 306;
 
 // The order by predicted cost: ORDER_BUCKETS buckets of the normalised log cost over [ORDER_HI - ORDER_BUCKETS /
 // ORDER_SCALE, ORDER_HI), bucket 0 the most expensive (above the range), NaN in the last.
-constexpr uint32_t ORDER_BUCKETS = 256, ORDER_BLOCK = 256, ORDER_SCAN = 1024;
+constexpr uint32_t ORDER_BUCKETS = 256, ORDER_BLOCK = 256;
 constexpr float ORDER_HI = 3.0f, ORDER_SCALE = 64.0f;
 constexpr int ORDER_SORTED = 0, ORDER_BALANCED = 1;
 uint64_t order_work_words(uint32_t n);
@@ -36,6 +36,8 @@ hipError_t launch_mlp_train(hipStream_t st, const float* params, const float* fe
 hipError_t launch_adam(hipStream_t st, float* params, float* m, float* v, const float* grad, float lr, float bc1, float bc2);
 hipError_t launch_gather_words(hipStream_t st, const uint32_t* src, const uint32_t* perm, uint32_t* dst, uint32_t n, uint32_t words,
                                bool scatter);
+// The arenas of `states` reordered in place (arena i = the former arena perm[i]); spare: a buffer of the same size.
+hipError_t launch_permute_states(hipStream_t st, uint32_t* states, uint32_t* spare, const uint32_t* perm, uint32_t n);
 hipError_t launch_gather_states(hipStream_t st, const uint32_t* src, uint32_t n_src, const uint32_t* perm, uint32_t* dst,
                                 uint32_t n);
 

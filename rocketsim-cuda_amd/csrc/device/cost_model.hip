@@ -2,8 +2,8 @@
 // (wall-clock ticks of a wave running that arena alone) and a contact logit; and the kernels that regroup arenas by it.
 //
 //   k_features     48 features per arena from the AoSoA-64 states (positions, velocities, wall and gap distances, counts)
-//   k_mlp_infer    inference: bf16 weights and activations, fp32 accumulation, on v_mfma_f32_16x16x16_bf16 (one wave, 64
-//                  arenas as four 16-row tiles; weights staged transposed in LDS, activations re-laid through LDS)
+//   k_mlp_infer    inference: bf16 weights and activations, fp32 accumulation, on v_mfma_f32_16x16x16_bf16, weights and
+//                  activations in registers
 //   k_mlp_train    training forward + backward in fp32 (the same bf16 rounding points as inference; the rounding is treated
 //                  as the identity in the backward pass), and each work-group's share of the parameter gradient
 //   k_mlp_reduce   the parameter gradient: the sum of the shares
@@ -39,9 +39,12 @@ __device__ inline float clamp1(float x) { return x < -4.0f ? -4.0f : (x > 4.0f ?
 }  // namespace
 
 // ---- features ------------------------------------------------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) k_features(const uint32_t* __restrict__ states, uint32_t n, float* __restrict__ feat) {
-  uint32_t a = blockIdx.x * blockDim.x + threadIdx.x;
-  if (a >= n) return;
+// One wave per AoSoA block: each lane reads its arena's words (256-byte rows) and computes its features; the rows of 48 then
+// leave through LDS, so that the wave writes its 12 KB as one run. Bound by the latency of one round of loads.
+constexpr int FEATURE_STRIDE = COST_FEATURES + 1;  // odd: lanes writing the same feature hit distinct banks
+__global__ void __launch_bounds__(64) k_features(const uint32_t* __restrict__ states, uint32_t n, float* __restrict__ feat) {
+  __shared__ float rows[AOSOA_LANES * FEATURE_STRIDE];
+  const uint32_t a0 = blockIdx.x * AOSOA_LANES, a = a0 + threadIdx.x;  // a lane past n reads the padding of its block
   float f[COST_FEATURES];
   const size_t ball = offsetof(ArenaState, ball);
   V3 bp = vword(states, a, ball + offsetof(Ball, pos)), bv = vword(states, a, ball + offsetof(Ball, vel));
@@ -73,70 +76,83 @@ __global__ void __launch_bounds__(256) k_features(const uint32_t* __restrict__ s
   f[45] = (float)word_of(states, a, offsetof(ArenaState, n_pairs) / 4) / 16.0f;
   f[46] = (float)word_of(states, a, offsetof(ArenaState, n_manifolds) / 4) / 16.0f;
   f[47] = (float)word_of(states, a, offsetof(ArenaState, n_dyn_cells) / 4) / 64.0f;
-  for (int i = 0; i < COST_FEATURES; ++i) feat[(size_t)a * COST_FEATURES + i] = clamp1(f[i]);
+  for (int i = 0; i < COST_FEATURES; ++i) rows[threadIdx.x * FEATURE_STRIDE + i] = clamp1(f[i]);
+  __syncthreads();
+  const uint32_t words = (n - a0 < AOSOA_LANES ? n - a0 : AOSOA_LANES) * (uint32_t)COST_FEATURES;
+  for (uint32_t e = threadIdx.x; e < words; e += 64u)
+    feat[(size_t)a0 * COST_FEATURES + e] = rows[e / COST_FEATURES * FEATURE_STRIDE + e % COST_FEATURES];
 }
 
 // ---- inference on MFMA ---------------------------------------------------------------------------------------------------------
-// One wave, 64 arenas. v_mfma_f32_16x16x16_bf16 lane layout: A (16x16, rows x k): lane l holds row l % 16, k = 4 (l / 16)
-// + 0..3; B (k x cols): col l % 16, k = 4 (l / 16) + 0..3; D (rows x cols): col l % 16, rows 4 (l / 16) + 0..3. Weights sit
-// transposed in LDS (wt[out][in], bf16) so that both operands are four consecutive bf16 per lane.
-constexpr int KP = 64;  // padded input width of every layer
+// v_mfma_f32_16x16x16_bf16 lane layout: A (16x16, rows x k): lane l holds row l % 16, k = 4 (l / 16) + 0..3; B (k x cols):
+// col l % 16, k = 4 (l / 16) + 0..3; D (rows x cols): col l % 16, rows 4 (l / 16) + 0..3. The product is taken transposed,
+// outputs as rows and arenas as columns: a layer's D is then, lane for lane, the next layer's B, so the activations stay in
+// registers from the features to the prediction. The weights stay in registers too, as A operands (a column of 16 outputs'
+// weights per lane), and each wave takes every waves-th tile of 16 arenas. Bound by reading the features: 65,536 arenas
+// (12.6 MB) took 1,099 us with the weights staged in LDS by every wave of 64 arenas and the activations re-laid through LDS.
+constexpr uint32_t INFER_WAVES = 2048;  // two per SIMD: a wave's weights (about 130 words per lane) pay off over its tiles
+__device__ inline v4s weight_frag(const float* __restrict__ w, int in0, int out, int stride, bool used) {
+  v4s f = v4s{0, 0, 0, 0};
+  if (used)
+    for (int i = 0; i < 4; ++i) f[i] = (short)bf16_bits(w[(in0 + i) * stride + out]);
+  return f;
+}
+__device__ inline v4s hidden_frag(v4f acc, v4f bias) {  // the layer's activation, rounded as the next layer's input
+  v4s f;
+  for (int i = 0; i < 4; ++i) {
+    const float v = acc[i] + bias[i];
+    f[i] = (short)bf16_bits(v > 0.0f ? v : 0.0f);
+  }
+  return f;
+}
 __global__ void __launch_bounds__(64) k_mlp_infer(const float* __restrict__ params, const float* __restrict__ feat, uint32_t n,
                                                   float* __restrict__ out) {
-  __shared__ uint16_t w1t[64 * KP], w2t[64 * KP], w3t[16 * KP];
-  __shared__ uint16_t act[64 * KP];  // the 64 arenas' current activations, bf16, row-major [arena][k]
-  __shared__ float bias[64 + 64 + 16];
-  const int l = threadIdx.x;
+  const int l = threadIdx.x, lr = l % 16, lk = 4 * (l / 16);
   const float *W1 = params + COST_W1, *B1 = params + COST_B1, *W2 = params + COST_W2, *B2 = params + COST_B2,
               *W3 = params + COST_W3, *B3 = params + COST_B3;
-  for (int e = l; e < 64 * KP; e += 64) {  // e = out * KP + in
-    int o = e / KP, i = e % KP;
-    w1t[e] = i < COST_FEATURES ? bf16_bits(W1[i * 64 + o]) : (uint16_t)0;
-    w2t[e] = bf16_bits(W2[i * 64 + o]);
+  constexpr int K1 = COST_FEATURES / 16;  // 16-wide input steps of the first layer
+  v4s w1[4][K1], w2[4][4], w3[4];
+  v4f b1[4], b2[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+#pragma unroll
+    for (int ks = 0; ks < K1; ++ks) w1[j][ks] = weight_frag(W1, ks * 16 + lk, j * 16 + lr, 64, true);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) w2[j][ks] = weight_frag(W2, ks * 16 + lk, j * 16 + lr, 64, true);
+    w3[j] = weight_frag(W3, j * 16 + lk, lr, 2, lr < 2);
+    for (int i = 0; i < 4; ++i) b1[j][i] = B1[j * 16 + lk + i], b2[j][i] = B2[j * 16 + lk + i];
   }
-  for (int e = l; e < 16 * KP; e += 64) {
-    int o = e / KP, i = e % KP;
-    w3t[e] = o < 2 ? bf16_bits(W3[i * 2 + o]) : (uint16_t)0;
-  }
-  bias[l] = B1[l];
-  bias[64 + l] = B2[l];
-  if (l < 16) bias[128 + l] = l < 2 ? B3[l] : 0.0f;
-  const uint32_t base = blockIdx.x * 64;
-  for (int r = 0; r < 64; ++r) {  // the block's 64 feature rows, padded with zeros (and zero rows past n)
-    uint32_t a = base + r;
-    float x = (a < n && l < COST_FEATURES) ? feat[(size_t)a * COST_FEATURES + l] : 0.0f;
-    act[r * KP + l] = bf16_bits(x);
-  }
-  __syncthreads();
-  const int lr = l % 16, lk = 4 * (l / 16);
-  for (int layer = 0; layer < 3; ++layer) {
-    const uint16_t* wt = layer == 0 ? w1t : layer == 1 ? w2t : w3t;
-    const int nt = layer == 2 ? 1 : 4;  // 16-column output tiles
-    v4f acc[4][4];
-    for (int t = 0; t < 4; ++t)
-      for (int j = 0; j < nt; ++j) {
-        acc[t][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-        for (int ks = 0; ks < KP / 16; ++ks) {
-          const uint16_t* pa = act + (t * 16 + lr) * KP + ks * 16 + lk;
-          const uint16_t* pb = wt + (j * 16 + lr) * KP + ks * 16 + lk;
-          v4s av = v4s{(short)pa[0], (short)pa[1], (short)pa[2], (short)pa[3]};
-          v4s bv = v4s{(short)pb[0], (short)pb[1], (short)pb[2], (short)pb[3]};
-          acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc[t][j], 0, 0, 0);
-        }
-      }
-    __syncthreads();  // every lane has read this layer's input
-    for (int t = 0; t < 4; ++t)
-      for (int j = 0; j < nt; ++j)
-        for (int i = 0; i < 4; ++i) {
-          int row = t * 16 + lk + i, col = j * 16 + lr;
-          float v = acc[t][j][i] + bias[layer * 64 + col];
-          if (layer < 2) {
-            act[row * KP + col] = bf16_bits(v > 0.0f ? v : 0.0f);
-          } else if (col < 2 && base + row < n) {
-            out[(size_t)(base + row) * 2 + col] = v;
-          }
-        }
-    __syncthreads();
+  const float b30 = B3[0], b31 = B3[1];
+  for (uint32_t t = blockIdx.x; t < (n + 15) / 16; t += gridDim.x) {
+    const uint32_t a = t * 16 + lr;
+    v4s x[K1];
+#pragma unroll
+    for (int ks = 0; ks < K1; ++ks) {
+      const float* row = feat + (size_t)(a < n ? a : n - 1) * COST_FEATURES + ks * 16 + lk;
+      for (int i = 0; i < 4; ++i) x[ks][i] = (short)bf16_bits(row[i]);
+    }
+    v4s h1[4], h2[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      v4f acc = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int ks = 0; ks < K1; ++ks) acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w1[j][ks], x[ks], acc, 0, 0, 0);
+      h1[j] = hidden_frag(acc, b1[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      v4f acc = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w2[j][ks], h1[ks], acc, 0, 0, 0);
+      h2[j] = hidden_frag(acc, b2[j]);
+    }
+    v4f y = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) y = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w3[ks], h2[ks], y, 0, 0, 0);
+    if (l < 16 && a < n) {
+      out[(size_t)a * 2] = y[0] + b30;
+      out[(size_t)a * 2 + 1] = y[1] + b31;
+    }
   }
 }
 
@@ -335,25 +351,71 @@ __global__ void __launch_bounds__(256) k_scatter_words(const uint32_t* __restric
   uint32_t j = perm[i];
   if (j < n) dst[(size_t)j * words + w] = src[e];
 }
-// AoSoA-64 states: arena i of dst (n arenas) = arena perm[i] of src (n_src arenas), the persistent words (the tail is zero at a tick boundary). The
-// grid's y dimension walks the words, so all arenas of one word are copied together and the source lines they share
-// are read from HBM once.
+// AoSoA-64 states: arena i of dst (n arenas) = arena perm[i] of src (n_src arenas); an index past src leaves that arena of
+// dst as it was. The grid walks the words, so all arenas of one word are copied together and the source lines they share
+// are read from HBM once; word w's work-groups are all w % 8 modulo 8, on one XCD and its L2.
 __global__ void __launch_bounds__(256) k_gather_states(const uint32_t* __restrict__ src, uint32_t n_src,
                                                        const uint32_t* __restrict__ perm, uint32_t* __restrict__ dst, uint32_t n) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  uint32_t w = blockIdx.y;
+  const uint32_t groups = (n + 255u) / 256u, q = blockIdx.x / 8u;
+  const uint32_t w = q / groups * 8u + blockIdx.x % 8u, i = q % groups * 256u + threadIdx.x;
   if (i >= n || w >= (uint32_t)ARENA_WORDS) return;
   uint32_t a = perm[i];
   if (a < n_src) dst[aosoa_index(i, w)] = src[aosoa_index(a, w)];
+}
+// The same row by row: 4-byte reads at random places, one L2 request each, bound the kernel above (65,536 arenas: 1,148 us
+// without its XCD mapping, 971 us with it). Here a work-group takes one word of all of dst's arenas (up to ROW_DST): the
+// source's row of that word passes through LDS in parts of ROW_PART arenas, read from HBM as whole lines, and every thread
+// picks its arenas' values there, holds them in registers over the parts and writes whole lines at the end (65,536 arenas:
+// 758 us; a copy of the buffer 292 us). The group has read the whole row before it writes any of it, so dst may be src.
+constexpr uint32_t ROW_PART = 32768, ROW_THREADS = 1024, ROW_EACH = 64, ROW_DST = ROW_THREADS * ROW_EACH;
+constexpr uint32_t ROW_LOADS = ROW_PART / (4 * ROW_THREADS);
+// Rows from here on: a smaller row stays in L2 and fills few of a group's threads (16,384 arenas: rows 172 us, words 219 us;
+// 8,192 arenas: words 71 us). A sample of a source is gathered word by word too, and a batch past ROW_DST, where every group
+// would read several parts for each of several chunks (131,072 arenas: rows 2,473 us, words 1,897 us).
+constexpr uint32_t ROW_MIN = 12288;
+__global__ void __launch_bounds__(ROW_THREADS) k_gather_rows(const uint32_t* src, uint32_t n_src,
+                                                             const uint32_t* __restrict__ perm, uint32_t* dst, uint32_t n) {
+  extern __shared__ uint4 row4[];  // ROW_PART words
+  const uint32_t* row = (const uint32_t*)row4;
+  const uint32_t tid = threadIdx.x, w = blockIdx.x;
+  const uint32_t quads = (n_src + AOSOA_LANES - 1) / AOSOA_LANES * (AOSOA_LANES / 4);  // of the row, padding lanes included
+  uint32_t v[ROW_EACH];
+  const uint32_t parts = (n_src + ROW_PART - 1) / ROW_PART;
+  for (uint32_t part = 0; part < parts; ++part) {
+#pragma unroll
+    for (uint32_t k = 0; k < ROW_LOADS; ++k) {
+      const uint32_t g = part * (ROW_PART / 4) + k * ROW_THREADS + tid;  // arenas 4 g .. 4 g + 3
+      row4[k * ROW_THREADS + tid] = g < quads ? *(const uint4*)(src + aosoa_index(4 * g, w)) : uint4{0u, 0u, 0u, 0u};
+    }
+    __syncthreads();
+    uint32_t first = tid;
+    asm volatile("" : "+v"(first));  // not the same in every round to the compiler: 64 addresses kept over the rounds would spill
+#pragma unroll
+    for (uint32_t k = 0; k < ROW_EACH; ++k) {
+      const uint32_t i = first + k * ROW_THREADS;
+      if (k % 8 == 0) asm volatile("" ::: "memory");  // at most eight indices in flight: more would spill the values
+      if (k * ROW_THREADS < n) {  // the same for the whole work-group
+        const uint32_t at = (i < n ? perm[i] : 0u) - part * ROW_PART;
+        if (at < ROW_PART) v[k] = row[at];
+      }
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < ROW_EACH; ++k) {
+    const uint32_t i = k * ROW_THREADS + tid;
+    if (k % 8 == 0) asm volatile("" ::: "memory");
+    if (i < n && perm[i] < n_src) dst[aosoa_index(i, w)] = v[k];
+  }
 }
 
 // ---- the order by predicted cost ---------------------------------------------------------------------------------------------
 // A stable counting sort on the device: each arena's predicted normalised log cost falls into one of ORDER_BUCKETS
 // buckets (bucket 0 the most expensive); ranks are stable within a bucket (slot order), so the order is deterministic.
-// k_order_count: per-block bucket histograms, stored bucket-major (counts[b * blocks + block]) so that one exclusive scan
-// of the whole array (k_order_scan) gives every (bucket, block) pair its first rank. k_order_place: each arena's rank =
-// that base + its rank among the block's earlier arenas of the same bucket (wave ballots, then the earlier waves' counts),
-// mapped to a slot by the mode.
+// k_order_count: per-block bucket histograms, stored bucket-major (counts[b * blocks + block]). k_order_scan: each bucket's
+// row scanned. k_order_place: each arena's rank = the buckets before its own (their totals scanned by every work-group) + its
+// bucket's arenas in earlier blocks + its rank among the block's earlier arenas of the same bucket (wave ballots, then the
+// earlier waves' counts), mapped to a slot by the mode.
 __device__ inline uint32_t order_bucket(float p) {
   float q = (ORDER_HI - p) * ORDER_SCALE;
   return q != q ? ORDER_BUCKETS - 1u : q <= 0.0f ? 0u : q >= (float)(ORDER_BUCKETS - 1) ? ORDER_BUCKETS - 1u : (uint32_t)q;
@@ -379,36 +441,48 @@ __global__ void __launch_bounds__(ORDER_BLOCK) k_order_count(const float* __rest
   for (uint32_t b = t; b < ORDER_BUCKETS; b += ORDER_BLOCK) counts[(size_t)b * blocks + blockIdx.x] = h[b];
 }
 
-// Exclusive scan of m words in place, one work-group of ORDER_SCAN threads: each thread sums a contiguous chunk, the
-// chunk sums are scanned in LDS, then each thread rewrites its chunk.
-__global__ void __launch_bounds__(ORDER_SCAN) k_order_scan(uint32_t* __restrict__ v, uint32_t m) {
-  __shared__ uint32_t s[ORDER_SCAN];
-  const uint32_t t = threadIdx.x, chunk = (m + ORDER_SCAN - 1) / ORDER_SCAN;
-  const uint32_t lo = t * chunk < m ? t * chunk : m, hi = lo + chunk < m ? lo + chunk : m;
-  uint32_t sum = 0;
-  for (uint32_t i = lo; i < hi; ++i) sum += v[i];
-  s[t] = sum;
-  __syncthreads();
-  for (uint32_t d = 1; d < ORDER_SCAN; d <<= 1) {  // Hillis-Steele inclusive scan
-    uint32_t x = t >= d ? s[t - d] : 0u;
+// One work-group per bucket: the inclusive scan of its row of block counts, in place, ORDER_BLOCK at a time. A bucket's total
+// is then its row's last word, and a block's first rank within the bucket the word before its own. (A scan of the whole
+// array by one work-group took 109 us of the order's 120 at 65,536 arenas.)
+__global__ void __launch_bounds__(ORDER_BLOCK) k_order_scan(uint32_t* __restrict__ counts, uint32_t blocks) {
+  __shared__ uint32_t s[ORDER_BLOCK];
+  const uint32_t t = threadIdx.x;
+  uint32_t* v = counts + (size_t)blockIdx.x * blocks;
+  uint32_t carry = 0;
+  for (uint32_t lo = 0; lo < blocks; lo += ORDER_BLOCK) {
+    s[t] = lo + t < blocks ? v[lo + t] : 0u;
     __syncthreads();
-    s[t] += x;
+    for (uint32_t d = 1; d < ORDER_BLOCK; d <<= 1) {  // Hillis-Steele inclusive scan
+      const uint32_t x = t >= d ? s[t - d] : 0u;
+      __syncthreads();
+      s[t] += x;
+      __syncthreads();
+    }
+    if (lo + t < blocks) v[lo + t] = carry + s[t];
+    carry += s[ORDER_BLOCK - 1];
     __syncthreads();
-  }
-  uint32_t run = s[t] - sum;  // exclusive prefix of this chunk
-  for (uint32_t i = lo; i < hi; ++i) {
-    uint32_t c = v[i];
-    v[i] = run;
-    run += c;
   }
 }
 
-__global__ void __launch_bounds__(ORDER_BLOCK) k_order_place(const float* __restrict__ pred, uint32_t n, const uint32_t* __restrict__ base,
+__global__ void __launch_bounds__(ORDER_BLOCK) k_order_place(const float* __restrict__ pred, uint32_t n, const uint32_t* __restrict__ counts,
                                                              int mode, uint32_t* __restrict__ perm) {
   constexpr uint32_t WAVES = ORDER_BLOCK / AOSOA_LANES;
   __shared__ uint32_t wc[WAVES][ORDER_BUCKETS];
   const uint32_t t = threadIdx.x, lane = t % AOSOA_LANES, wave = t / AOSOA_LANES;
+  __shared__ uint32_t first[ORDER_BUCKETS];  // the rank of the bucket's first arena in this block
+  static_assert(ORDER_BUCKETS == ORDER_BLOCK, "one thread per bucket");
   for (uint32_t e = t; e < WAVES * ORDER_BUCKETS; e += ORDER_BLOCK) wc[e / ORDER_BUCKETS][e % ORDER_BUCKETS] = 0;
+  const uint32_t* mine = counts + (size_t)t * gridDim.x;
+  const uint32_t total = mine[gridDim.x - 1], earlier = blockIdx.x ? mine[blockIdx.x - 1] : 0u;
+  first[t] = total;
+  __syncthreads();
+  for (uint32_t d = 1; d < ORDER_BUCKETS; d <<= 1) {
+    const uint32_t x = t >= d ? first[t - d] : 0u;
+    __syncthreads();
+    first[t] += x;
+    __syncthreads();
+  }
+  first[t] += earlier - total;
   __syncthreads();
   const uint32_t a = blockIdx.x * ORDER_BLOCK + t;
   const bool valid = a < n;
@@ -426,7 +500,7 @@ __global__ void __launch_bounds__(ORDER_BLOCK) k_order_place(const float* __rest
   if (!valid) return;
   uint32_t rank = rank_in_wave;
   for (uint32_t w = 0; w < wave; ++w) rank += wc[w][b];
-  const uint32_t s = base[(size_t)b * gridDim.x + blockIdx.x] + rank;
+  const uint32_t s = first[b] + rank;
   if (s < n) perm[order_slot(s, n, mode)] = a;  // s < n always (the counts sum to n); the check keeps a stray rank out
 }
 
@@ -459,7 +533,7 @@ hipError_t order_scratch_address(uint32_t** out) { return hipGetSymbolAddress((v
 hipError_t launch_cost_order(hipStream_t st, const float* pred, uint32_t n, int mode, uint32_t* work, uint32_t* perm) {
   const unsigned blocks = blocks_of(n, ORDER_BLOCK);
   k_order_count<<<blocks, ORDER_BLOCK, 0, st>>>(pred, n, work);
-  k_order_scan<<<1, ORDER_SCAN, 0, st>>>(work, (uint32_t)order_work_words(n));
+  k_order_scan<<<ORDER_BUCKETS, ORDER_BLOCK, 0, st>>>(work, blocks);
   k_order_place<<<blocks, ORDER_BLOCK, 0, st>>>(pred, n, work, mode, perm);
   return hipGetLastError();
 }
@@ -474,11 +548,12 @@ hipError_t launch_block_order(hipStream_t st, const float* pred, uint32_t n, uin
   return launch_cost_order(st, block_pred, nb, ORDER_SORTED, work + 2ull * nb, order);
 }
 hipError_t launch_features(hipStream_t st, const uint32_t* states, uint32_t n, float* feat) {
-  k_features<<<blocks_of(n, 256), 256, 0, st>>>(states, n, feat);
+  k_features<<<blocks_of(n, AOSOA_LANES), AOSOA_LANES, 0, st>>>(states, n, feat);
   return hipGetLastError();
 }
 hipError_t launch_mlp_infer(hipStream_t st, const float* params, const float* feat, uint32_t n, float* out) {
-  k_mlp_infer<<<blocks_of(n, 64), 64, 0, st>>>(params, feat, n, out);
+  const uint32_t tiles = blocks_of(n, 16);
+  k_mlp_infer<<<tiles < INFER_WAVES ? tiles : INFER_WAVES, 64, 0, st>>>(params, feat, n, out);
   return hipGetLastError();
 }
 hipError_t launch_mlp_train(hipStream_t st, const float* params, const float* feat, const float* target, const float* contact,
@@ -507,8 +582,21 @@ hipError_t launch_gather_words(hipStream_t st, const uint32_t* src, const uint32
 }
 hipError_t launch_gather_states(hipStream_t st, const uint32_t* src, uint32_t n_src, const uint32_t* perm, uint32_t* dst,
                                 uint32_t n) {
-  k_gather_states<<<dim3(blocks_of(n, 256), ARENA_WORDS), 256, 0, st>>>(src, n_src, perm, dst, n);
+  static_assert(ARENA_WORDS % 8 == 0, "eight words in flight, one per XCD");
+  if (n_src >= ROW_MIN && n_src <= ROW_DST && n >= n_src / 2 && n <= ROW_DST)
+    k_gather_rows<<<ARENA_WORDS, ROW_THREADS, ROW_PART * sizeof(uint32_t), st>>>(src, n_src, perm, dst, n);
+  else
+    k_gather_states<<<blocks_of(n, 256) * ARENA_WORDS, 256, 0, st>>>(src, n_src, perm, dst, n);
   return hipGetLastError();
+}
+
+hipError_t launch_permute_states(hipStream_t st, uint32_t* states, uint32_t* spare, const uint32_t* perm, uint32_t n) {
+  if (n >= ROW_MIN && n <= ROW_DST) {
+    k_gather_rows<<<ARENA_WORDS, ROW_THREADS, ROW_PART * sizeof(uint32_t), st>>>(states, n, perm, states, n);
+    return hipGetLastError();
+  }
+  hipError_t e = launch_gather_states(st, states, n, perm, spare, n);
+  return e == hipSuccess ? launch_copy_words(st, spare, states, aosoa_words(n)) : e;
 }
 
 }  // namespace dev

@@ -607,6 +607,16 @@ int rsim_gather_states(rsim_device* dev, const rsim_states* src, const rsim_word
   RSIM_HIP(rs::dev::launch_gather_states(dev->stream, src->d, src->n, perm->d, dst->d, dst->n), "gather states");
   return RSIM_OK;
 }
+int rsim_permute_states(rsim_device* dev, rsim_states* states, const rsim_words* perm, rsim_states* spare) {
+  int rc = use(dev);
+  if (rc) return rc;
+  if (!states || !perm || !spare || states == spare || states->n != spare->n)
+    return fail(RSIM_ERR_INVALID, "rsim_permute_states: bad buffers");
+  if (perm->n < states->n) return fail(RSIM_ERR_SHORT, "rsim_permute_states: index list too short");
+  if (!states->n) return RSIM_OK;
+  RSIM_HIP(rs::dev::launch_permute_states(dev->stream, states->d, spare->d, perm->d, states->n), "permute states");
+  return RSIM_OK;
+}
 uint64_t rsim_cost_order_work_words(uint32_t n) { return rs::dev::order_work_words(n); }
 int rsim_cost_order(rsim_device* dev, const rsim_words* pred, uint32_t n, int mode, rsim_words* work, rsim_words* perm) {
   int rc = use(dev);

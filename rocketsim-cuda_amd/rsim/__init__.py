@@ -81,6 +81,7 @@ def lib():
             "rsim_capture_begin": ([_vp], ctypes.c_int), "rsim_capture_end": ([_vp, ctypes.POINTER(_vp)], ctypes.c_int),
             "rsim_graph_launch": ([_vp, _vp], ctypes.c_int), "rsim_graph_free": ([_vp], ctypes.c_int),
             "rsim_gather_states": ([_vp, _vp, _vp, _vp], ctypes.c_int),
+            "rsim_permute_states": ([_vp, _vp, _vp, _vp], ctypes.c_int),
             "rsim_permute_words": ([_vp, _vp, _vp, u32, u32, ctypes.c_int, _vp], ctypes.c_int),
             "rsim_upload_states": ([_vp, _vp, u32, ctypes.POINTER(_vp)], ctypes.c_int),
             "rsim_alloc_states": ([_vp, u32, ctypes.POINTER(_vp)], ctypes.c_int),

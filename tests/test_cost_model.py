@@ -431,3 +431,63 @@ def test_regrouped_full_size(rsim, oracle, world, device, dev_world):
         assert np.array_equal(oracle.sim8(cpu, world, c, threads=16), res[k]), "oracle decision %d" % k
     fd = first_diff(got[:, :2567], cpu[:, :2567])
     assert fd is None, "arena %d word %d" % fd
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 65, 12287, 12288, 12353, 32769, 65535, 65536, 65537])
+def test_gather_and_permute_states(rsim, device, n):
+    """Every word of every arena at its new place, at the edges of the word-wise and row-wise gathers: into another buffer
+    (with indices past the source, which leave their arenas as they were) and in place."""
+    note("gather_states and permute_states, %d arenas" % n)
+    rng = np.random.default_rng(n)
+    words, other = (rng.integers(0, 2**32, rsim.aosoa_words(n), dtype=np.uint32) for _ in range(2))
+    view = lambda w: w.reshape(-1, rsim.ARENA_WORDS, 64)  # [block, word, lane]
+    at = lambda w, i: view(w)[i // 64, :, i % 64]
+    put = lambda w: device.upload_states(rsim.aosoa_unpack(w, n))
+    perm = rng.permutation(n).astype(np.uint32)
+    src, dst, p = put(words), put(other), device.upload_words(perm)
+    some = rng.choice(n, min(n, 300), replace=False)
+    holes = perm.copy()
+    holes[some[::3]] = n + 5
+    device.gather_states(src, device.upload_words(holes), dst)
+    got = device.download_words(dst)
+    for i in some:
+        assert np.array_equal(at(got, i), at(other, i) if holes[i] >= n else at(words, int(holes[i]))), i
+    rsim._check(rsim.lib().rsim_permute_states(device.handle, src.handle, p.handle, dst.handle), "permute")
+    got = rsim.aosoa_unpack(device.download_words(src), n)
+    assert np.array_equal(got, rsim.aosoa_unpack(words, n)[perm])
+    assert rsim.lib().rsim_permute_states(device.handle, src.handle, p.handle, src.handle) != 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 4097, 32768 + 16])
+def test_prediction_tiles(rsim, device, n):
+    """The prediction at the edges of its 16-arena tiles and past one tile per wave. Bound: the float64 network's own sums in
+    fp32 (65 terms below 64 in size: 65 x 64 x 2^-24 = 2.5e-4) plus a bf16 unit on the few activations that such a
+    difference rounds the other way (2^-8 of an activation below 16, times a weight below 1)."""
+    note("cost prediction, %d arenas" % n)
+    feat = np.clip(np.random.default_rng(n).standard_normal((n, cm.FEATURES)), -4, 4).astype(np.float32)
+    model = cm.CostModel(device, seed=21)
+    got = device.read_words(model.predict(device.upload_words(feat.view(np.uint32).ravel()), n)).view(np.float32).reshape(n, 2)
+    want = ref_forward(model.host_params(), feat)[3]
+    assert np.abs(got - want).max() < 2.5e-4 + 16 / 256
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b", [1, 24, 25, 31, 33, 49, 63, 65, 8192 + 33])
+def test_gradient_groups(rsim, device, b):
+    """The gradient at the edges of its 32-row groups, of what the scratch has room for, and past one group of rows per
+    work-group; against the float64 gradient with the same rounding points. Bound: 2^-7 of a block's largest entry (an
+    activation whose fp32 sum rounds to the other bf16 neighbour moves the entries it enters by up to 2^-8 of them)."""
+    note("cost gradients, batch %d" % b)
+    rng = np.random.default_rng(b)
+    feat = np.clip(rng.standard_normal((b, cm.FEATURES)), -4, 4).astype(np.float32)
+    target, contact = rng.standard_normal(b).astype(np.float32), (rng.random(b) < 0.4).astype(np.float32)
+    model = cm.CostModel(device, seed=22)
+    up = [device.upload_words(np.ascontiguousarray(x).view(np.uint32).ravel()) for x in (feat, target, contact)]
+    scratch, loss = model.gradients(*up, b)
+    want_loss, want = ref_loss_grad(model.host_params(), feat, target, contact)
+    got = device.read_words(model.grad).view(np.float32)
+    assert np.abs(device.read_words(loss).view(np.float32) - want_loss).max() <= 2.0**-7 * np.abs(want_loss).max()
+    for lo, hi in ((cm.W1, cm.B1), (cm.B1, cm.W2), (cm.W2, cm.B2), (cm.B2, cm.W3), (cm.W3, cm.B3), (cm.B3, cm.PARAMS)):
+        assert np.abs(got[lo:hi] - want[lo:hi]).max() <= 2.0**-7 * np.abs(want[lo:hi]).max(), lo
