@@ -87,7 +87,8 @@ uint32_t rsim_world_count(const rsim_world* world);
 const void* rsim_world_device_ptr(const rsim_world* world);
 int rsim_world_free(rsim_world* world);
 
-/* upload_states / alloc_states (device.rs:73-80): n ArenaStates packed to AoSoA-64 on the host and uploaded; alloc zeroes. */
+/* upload_states / alloc_states (device.rs:73-80): n ArenaStates uploaded and packed to AoSoA-64 on the device; alloc
+ * zeroes. */
 int rsim_upload_states(rsim_device* dev, const void* states, uint32_t n, rsim_states** out);
 int rsim_alloc_states(rsim_device* dev, uint32_t n, rsim_states** out);
 /* Overwrites the n states of an existing buffer (same n) without reallocating. */

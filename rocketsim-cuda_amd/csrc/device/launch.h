@@ -18,6 +18,9 @@ RS_HD inline size_t aosoa_index(uint32_t a, uint32_t w) {
 
 hipError_t launch_identity(hipStream_t st, const uint32_t* in, uint32_t* out, uint32_t n, bool tick_only);
 hipError_t launch_copy_words(hipStream_t st, const uint32_t* in, uint32_t* out, size_t words);  // words % 4 == 0
+// n > 0 arenas between ArenaStates back to back and the AoSoA blocks from `blocks` on, both in device memory.
+hipError_t launch_pack_states(hipStream_t st, const uint32_t* aos, uint32_t* blocks, uint32_t n);
+hipError_t launch_unpack_states(hipStream_t st, const uint32_t* blocks, uint32_t* aos, uint32_t n);
 hipError_t launch_phase(hipStream_t st, int k, uint32_t* buf, const StaticData* w, uint32_t n, int32_t* status);
 hipError_t launch_step_tick(hipStream_t st, uint32_t* buf, const StaticData* w, uint32_t n, int32_t* status);
 // The result-word bit of an arena whose variant index is past the world table (the arena is not stepped).

@@ -14,6 +14,7 @@
 //   k_run                           several decisions per launch, the arena held in the lane from first to last
 //   k_run_queue                     k_run with persistent work-groups taking AoSoA blocks from a queue
 //   k_small (small_kernels.hip)     k_sim8 and k_run for small batches, the states in LDS
+//   k_pack_states / k_unpack_states the host's ArenaStates to and from AoSoA blocks
 //   k_copy_words                    a streaming copy of a state buffer (restores between timed runs)
 #include "device/launch.h"
 #include "device/aosoa.h"
@@ -193,6 +194,35 @@ __global__ void __launch_bounds__(256) k_copy_words(const uint4* __restrict__ in
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n16; i += stride) out[i] = in[i];
 }
 
+// Between n ArenaStates back to back (the host's format, staged in device memory) and AoSoA-64 blocks: a tile of 64 arenas x
+// 64 words per wave through LDS, whole lines on both sides. Lanes past n of the last block are written as zeros. Bound by
+// HBM and far below the transfer over PCIe that precedes or follows it; the host's own transposition of 2,048 arenas took
+// about 7 ms, a strided 4-byte access per word.
+constexpr uint32_t TILE_STRIDE = AOSOA_LANES + 1;  // odd: a column of the tile lies in distinct banks
+__global__ void __launch_bounds__(64) k_pack_states(const uint32_t* __restrict__ aos, uint32_t* __restrict__ out, uint32_t n) {
+  __shared__ uint32_t tile[AOSOA_LANES * TILE_STRIDE];
+  const uint32_t l = threadIdx.x, a0 = blockIdx.x * AOSOA_LANES, w0 = blockIdx.y * 64u;
+  const uint32_t words = (uint32_t)ARENA_WORDS - w0 < 64u ? (uint32_t)ARENA_WORDS - w0 : 64u;
+#pragma unroll 16
+  for (uint32_t r = 0; r < AOSOA_LANES; ++r)
+    tile[r * TILE_STRIDE + l] = a0 + r < n && l < words ? aos[(size_t)(a0 + r) * ARENA_WORDS + w0 + l] : 0u;
+  __syncthreads();
+#pragma unroll 16
+  for (uint32_t k = 0; k < words; ++k) out[block_base(a0) + (size_t)(w0 + k) * AOSOA_LANES + l] = tile[l * TILE_STRIDE + k];
+}
+__global__ void __launch_bounds__(64) k_unpack_states(const uint32_t* __restrict__ in, uint32_t* __restrict__ aos, uint32_t n) {
+  __shared__ uint32_t tile[AOSOA_LANES * TILE_STRIDE];
+  const uint32_t l = threadIdx.x, a0 = blockIdx.x * AOSOA_LANES, w0 = blockIdx.y * 64u;
+  const uint32_t words = (uint32_t)ARENA_WORDS - w0 < 64u ? (uint32_t)ARENA_WORDS - w0 : 64u;
+  const uint32_t arenas = n - a0 < AOSOA_LANES ? n - a0 : AOSOA_LANES;
+#pragma unroll 16
+  for (uint32_t k = 0; k < words; ++k) tile[l * TILE_STRIDE + k] = in[block_base(a0) + (size_t)(w0 + k) * AOSOA_LANES + l];
+  __syncthreads();
+#pragma unroll 16
+  for (uint32_t r = 0; r < arenas; ++r)
+    if (l < words) aos[(size_t)(a0 + r) * ARENA_WORDS + w0 + l] = tile[r * TILE_STRIDE + l];
+}
+
 // ---- launchers ------------------------------------------------------------------------------------------------------------------
 static dim3 grid_of(uint32_t n, uint32_t block) { return dim3((n + block - 1) / block > 0 ? (n + block - 1) / block : 1); }
 
@@ -207,6 +237,15 @@ hipError_t launch_copy_words(hipStream_t st, const uint32_t* in, uint32_t* out, 
   if (blocks > 8192) blocks = 8192;
   if (blocks == 0) blocks = 1;
   k_copy_words<<<dim3((unsigned)blocks), 256, 0, st>>>(reinterpret_cast<const uint4*>(in), reinterpret_cast<uint4*>(out), n16);
+  return hipGetLastError();
+}
+static dim3 tiles_of(uint32_t n) { return dim3((n + AOSOA_LANES - 1) / AOSOA_LANES, ((uint32_t)ARENA_WORDS + 63u) / 64u); }
+hipError_t launch_pack_states(hipStream_t st, const uint32_t* aos, uint32_t* blocks, uint32_t n) {
+  k_pack_states<<<tiles_of(n), 64, 0, st>>>(aos, blocks, n);
+  return hipGetLastError();
+}
+hipError_t launch_unpack_states(hipStream_t st, const uint32_t* blocks, uint32_t* aos, uint32_t n) {
+  k_unpack_states<<<tiles_of(n), 64, 0, st>>>(blocks, aos, n);
   return hipGetLastError();
 }
 hipError_t launch_phase(hipStream_t st, int k, uint32_t* buf, const StaticData* w, uint32_t n, int32_t* status) {

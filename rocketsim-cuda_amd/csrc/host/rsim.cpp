@@ -29,6 +29,8 @@ struct rsim_device {
   uint32_t status_cap;
   uint64_t live;  // worlds, state and word buffers (views included) and graphs not yet freed: rsim_close refuses while > 0
   uint32_t* order_scratch;  // this GPU's copy of the allocation-free order's fixed workspace (rsim_cost_order_noalloc)
+  uint32_t* stage;          // ArenaStates on their way to or from the host, at most STAGE_ARENAS (state uploads and downloads)
+  uint32_t stage_cap;       // its size in arenas
   uint32_t* queue;          // the block queue's counter of rsim_run_queued (one word, reset on the stream by each launch)
 };
 struct rsim_world {
@@ -116,6 +118,20 @@ void unpack(const uint32_t* in, uint32_t n, ArenaState* states) {
   }
 }
 
+// The staging buffer of state uploads and downloads: allocated by the first such call, sized to the largest batch seen up
+// to STAGE_ARENAS (65 MB), freed with the device. Every call that uses it ends synchronised, so it is never in use here.
+constexpr uint32_t STAGE_ARENAS = 6144;
+int ensure_stage(rsim_device* dev, uint32_t n) {
+  const uint32_t want = n < STAGE_ARENAS ? n : STAGE_ARENAS;
+  if (dev->stage_cap >= want) return RSIM_OK;
+  if (dev->stage) (void)hipFree(dev->stage);
+  dev->stage = nullptr;
+  dev->stage_cap = 0;
+  RSIM_HIP(hipMalloc((void**)&dev->stage, (size_t)want * sizeof(ArenaState)), "hipMalloc(stage)");
+  dev->stage_cap = want;
+  return RSIM_OK;
+}
+
 int ensure_status(rsim_device* dev, uint32_t n) {
   if (dev->status_cap >= n && dev->status) return RSIM_OK;
   if (dev->status) (void)hipFree(dev->status);
@@ -201,6 +217,7 @@ int rsim_close(rsim_device* dev) {
     return fail(RSIM_ERR_INVALID, "rsim_close: worlds, buffers or graphs of this device are still open (free them first)");
   (void)hipStreamSynchronize(dev->stream);
   if (dev->status) (void)hipFree(dev->status);
+  if (dev->stage) (void)hipFree(dev->stage);
   if (dev->queue) (void)hipFree(dev->queue);
   (void)hipEventDestroy(dev->t0);
   (void)hipEventDestroy(dev->t1);
@@ -292,14 +309,14 @@ int rsim_write_states(rsim_device* dev, rsim_states* dst, const void* states) {
   int rc = use_outside_capture(dev, "rsim_write_states");
   if (rc) return rc;
   if (!dst || (!states && dst->n)) return fail(RSIM_ERR_INVALID, "rsim_write_states: null argument");
-  std::vector<uint32_t> host;
-  try {
-    host.resize(rs::dev::aosoa_words(dst->n));
-  } catch (...) {
-    return fail(RSIM_ERR_INVALID, "rsim_write_states: out of host memory");
+  if (!dst->n) return RSIM_OK;
+  if ((rc = ensure_stage(dev, dst->n))) return rc;
+  const ArenaState* src = static_cast<const ArenaState*>(states);
+  for (uint32_t a = 0; a < dst->n; a += STAGE_ARENAS) {  // whole blocks but for the last, packed on the device
+    const uint32_t m = dst->n - a < STAGE_ARENAS ? dst->n - a : STAGE_ARENAS;
+    RSIM_HIP(hipMemcpyAsync(dev->stage, src + a, (size_t)m * sizeof(ArenaState), hipMemcpyHostToDevice, dev->stream), "state upload");
+    RSIM_HIP(rs::dev::launch_pack_states(dev->stream, dev->stage, dst->d + rs::dev::aosoa_index(a, 0), m), "state upload");
   }
-  pack(static_cast<const ArenaState*>(states), dst->n, host.data());
-  RSIM_HIP(hipMemcpyAsync(dst->d, host.data(), host.size() * 4, hipMemcpyHostToDevice, dev->stream), "state upload");
   RSIM_HIP(hipStreamSynchronize(dev->stream), "state upload");
   return RSIM_OK;
 }
@@ -344,15 +361,18 @@ int rsim_download_words(rsim_device* dev, const rsim_states* s, uint32_t* out) {
 }
 int rsim_download_states(rsim_device* dev, const rsim_states* s, void* out) {
   if (!s) return fail(RSIM_ERR_INVALID, "rsim_download_states: null states");
-  std::vector<uint32_t> host;
-  try {
-    host.resize(rs::dev::aosoa_words(s->n));
-  } catch (...) {
-    return fail(RSIM_ERR_INVALID, "rsim_download_states: out of host memory");
-  }
-  int rc = rsim_download_words(dev, s, host.data());
+  int rc = use_outside_capture(dev, "rsim_download_states");
   if (rc) return rc;
-  unpack(host.data(), s->n, static_cast<ArenaState*>(out));
+  if (!out && s->n) return fail(RSIM_ERR_INVALID, "rsim_download_states: null argument");
+  if (!s->n) return RSIM_OK;
+  if ((rc = ensure_stage(dev, s->n))) return rc;
+  ArenaState* dst = static_cast<ArenaState*>(out);
+  for (uint32_t a = 0; a < s->n; a += STAGE_ARENAS) {
+    const uint32_t m = s->n - a < STAGE_ARENAS ? s->n - a : STAGE_ARENAS;
+    RSIM_HIP(rs::dev::launch_unpack_states(dev->stream, s->d + rs::dev::aosoa_index(a, 0), dev->stage, m), "state download");
+    RSIM_HIP(hipMemcpyAsync(dst + a, dev->stage, (size_t)m * sizeof(ArenaState), hipMemcpyDeviceToHost, dev->stream), "state download");
+  }
+  RSIM_HIP(hipStreamSynchronize(dev->stream), "state download");
   return RSIM_OK;
 }
 

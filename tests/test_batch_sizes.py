@@ -86,3 +86,17 @@ def test_trace_goals_and_overflow(rsim, oracle, world, device, dev_world, n, var
         got = rsim.aosoa_unpack(slabs[t - 1], n)
         same(got[idx], ticks[idx], "trace tick %d" % t)
         assert not got[~live].any(), "ticks after a goal are not written"
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 6143, 6144, 6145, 12289])
+def test_states_to_the_device_and_back(rsim, device, n):
+    """The device's packing against the host's (rsim_aosoa_pack / unpack), at the edges of a block and of the staging
+    buffer; the padding lanes come out zero whatever the buffer held."""
+    print("[case] states up and down, %d arenas" % n, flush=True)
+    rng = np.random.default_rng(n)
+    states, before = (rng.integers(0, 2**32, (n, rsim.ARENA_WORDS), dtype=np.uint32) for _ in range(2))
+    d = device.upload_states(before)
+    device.write_states(d, states)
+    words = device.download_words(d)
+    assert np.array_equal(words, rsim.aosoa_pack(states))
+    assert np.array_equal(device.download_states(d), rsim.aosoa_unpack(words, n))
