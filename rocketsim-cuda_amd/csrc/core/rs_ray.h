@@ -48,6 +48,9 @@ RS_FN BodyView body_view(const ArenaState& s, const StaticData& w, uint32_t body
   }
   return v;
 }
+RS_FN BodyView dyn_body_view(const Body& b, const BodyConst& c) {  // of a dynamic body's own state
+  return BodyView{b.world, b.lin_vel, b.ang_vel, b.inv_inertia_world, c.inv_mass, b.collision_flags, c.user_idx};
+}
 RS_FN bool view_static(const BodyView& v) { return (v.flags & k::CF_STATIC) != 0; }
 RS_FN V3 vel_at(const BodyView& v, V3 rel) { return v.lin_vel + cross(v.ang_vel, rel); }
 RS_FN float impulse_denom(const BodyView& v, V3 pos, V3 n) {  // rigid_body_p1.cuh:66-71

@@ -9,49 +9,94 @@
 
 namespace rs {
 
+// P0, P2, P6 and P8 touch a few fields of every body or car: they read them all first and write them all last, so that the
+// bodies' reads are in flight together instead of each body's behind the branches and stores of the one before.
+
 // ---- P0 (arena_base.cuh:21-38) ---------------------------------------------------------------------------------------------------
 RS_INLINE void phase_p0(ArenaState& s, const StaticData& w) {
   s.events = 0;
-  for (int d = 0; d < NUM_DYN; ++d) clear_accum(s.bodies[d]);
-  for (int ci = 0; ci < NUM_CARS; ++ci) {
-    Body& rb = s.bodies[1 + ci];
-    limit_vels(rb, k::CAR_MAX_SPEED * k::UU_TO_BT, k::CAR_MAX_ANG_SPEED);
-    quantize_body(&rb.world.t, &rb.lin_vel, &rb.ang_vel);
-    s.cars[ci].vel = rb.lin_vel * k::BT_TO_UU;
-    s.cars[ci].ang_vel = rb.ang_vel;
+  Body b[NUM_DYN];
+  RS_UNROLL
+  for (int d = 0; d < NUM_DYN; ++d) {
+    b[d].world.t = s.bodies[d].world.t;
+    b[d].lin_vel = s.bodies[d].lin_vel;
+    b[d].ang_vel = s.bodies[d].ang_vel;
   }
-  Body& ball = s.bodies[0];
-  limit_vels(ball, w.mut_f[MF_BALL_MAX_SPEED] * k::UU_TO_BT, k::BALL_MAX_ANG_SPEED);
-  quantize_body(&ball.world.t, &ball.lin_vel, &ball.ang_vel);
-  s.ball.vel = ball.lin_vel * k::BT_TO_UU;
-  s.ball.ang_vel = ball.ang_vel;
+  RS_UNROLL
+  for (int d = 0; d < NUM_DYN; ++d) {  // the ball (0), then the cars: their limits and the quantisation
+    if (d == 0) limit_vels(b[d], w.mut_f[MF_BALL_MAX_SPEED] * k::UU_TO_BT, k::BALL_MAX_ANG_SPEED);
+    else limit_vels(b[d], k::CAR_MAX_SPEED * k::UU_TO_BT, k::CAR_MAX_ANG_SPEED);
+    quantize_body(&b[d].world.t, &b[d].lin_vel, &b[d].ang_vel);
+  }
+  RS_UNROLL
+  for (int d = 0; d < NUM_DYN; ++d) {
+    clear_accum(s.bodies[d]);
+    s.bodies[d].world.t = b[d].world.t;
+    s.bodies[d].lin_vel = b[d].lin_vel;
+    s.bodies[d].ang_vel = b[d].ang_vel;
+  }
+  s.ball.vel = b[0].lin_vel * k::BT_TO_UU;
+  s.ball.ang_vel = b[0].ang_vel;
+  RS_UNROLL
+  for (int ci = 0; ci < NUM_CARS; ++ci) {
+    s.cars[ci].vel = b[1 + ci].lin_vel * k::BT_TO_UU;
+    s.cars[ci].ang_vel = b[1 + ci].ang_vel;
+  }
 }
 
 // ---- P2 / P6 (discrete_dynamics_world.cuh) ---------------------------------------------------------------------------------------
 RS_INLINE void phase_p2(ArenaState& s, const StaticData& w) {
   const float dt = 1.0f / 120.0f;
   V3 g = w.gravity_bt * dt;
-  for (int d = 0; d < NUM_DYN; ++d)
-    if (body_active(s.bodies[d])) add_lin_impulse(s.bodies[d], g, true);
+  Body b[NUM_DYN];
+  RS_UNROLL
+  for (int d = 0; d < NUM_DYN; ++d) b[d] = s.bodies[d];
+  RS_UNROLL
   for (int d = 0; d < NUM_DYN; ++d) {
-    Body& b = s.bodies[d];
-    if (b.activation == k::ACT_SLEEPING) {
-      b.interp_world = b.world;
+    if (body_active(b[d])) add_lin_impulse(b[d], g, true);
+    if (b[d].activation == k::ACT_SLEEPING) {
+      b[d].interp_world = b[d].world;
       continue;
     }
-    apply_damping(b, w.bodies[w.dyn_body[d]], dt);
-    b.interp_world = predict_trans(b, dt);
+    apply_damping(b[d], w.bodies[w.dyn_body[d]], dt);
+    b[d].interp_world = predict_trans(b[d], dt);
+  }
+  RS_UNROLL
+  for (int d = 0; d < NUM_DYN; ++d) {
+    Body& o = s.bodies[d];
+    o.interp_world = b[d].interp_world;
+    o.lin_vel = b[d].lin_vel;
+    o.accum_lin_vel = b[d].accum_lin_vel;
+    o.accum_ang_vel = b[d].accum_ang_vel;
+    o.cached_linear_damping = b[d].cached_linear_damping;
+    o.cached_damping_time_step = b[d].cached_damping_time_step;
+    o.cached_linear_damping_value = b[d].cached_linear_damping_value;
   }
 }
 RS_INLINE void phase_p6(ArenaState& s, const StaticData& w) {
   const float dt = 1.0f / 120.0f;
+  Body b[NUM_DYN];
+  RS_UNROLL
+  for (int d = 0; d < NUM_DYN; ++d) b[d] = s.bodies[d];
+  bool moved[NUM_DYN];
+  RS_UNROLL
   for (int d = 0; d < NUM_DYN; ++d) {
-    Body& b = s.bodies[d];
-    if (!body_active(b)) continue;
-    Aff t = predict_trans(b, dt);
-    set_com_trans(b, w.bodies[w.dyn_body[d]], t);
+    const BodyConst& c = w.bodies[w.dyn_body[d]];
+    moved[d] = body_active(b[d]);
+    if (moved[d]) set_com_trans(b[d], c, predict_trans(b[d], dt));
+    update_activation(b[d], c, dt);
   }
-  for (int d = 0; d < NUM_DYN; ++d) update_activation(s.bodies[d], w.bodies[w.dyn_body[d]], dt);
+  RS_UNROLL
+  for (int d = 0; d < NUM_DYN; ++d) {
+    Body& o = s.bodies[d];
+    o.activation = b[d].activation;
+    o.deactivation_time = b[d].deactivation_time;
+    if (!moved[d]) continue;
+    o.world = b[d].world;
+    o.world_quat = b[d].world_quat;
+    o.interp_world = b[d].interp_world;
+    o.inv_inertia_world = b[d].inv_inertia_world;
+  }
 }
 
 // ---- P7 (arena_base.cuh:43-205, ball_base.cuh:22-48) ------------------------------------------------------------------------------
@@ -333,16 +378,40 @@ RS_FN void boost_pads_tick(ArenaState& s, const StaticData& w) {  // boost_pad_g
   }
 }
 RS_INLINE void phase_p8(ArenaState& s, const StaticData& w) {
+  Car car[NUM_CARS];
+  Body rb[NUM_CARS];
+  RS_UNROLL
   for (int ci = 0; ci < NUM_CARS; ++ci) {
-    car_post_tick(s.cars[ci], s.bodies[1 + ci]);
-    car_finish_tick(s.cars[ci], s.bodies[1 + ci]);
+    car[ci] = s.cars[ci];
+    rb[ci] = s.bodies[1 + ci];
+  }
+  const Body ball = s.bodies[0];
+  RS_UNROLL
+  for (int ci = 0; ci < NUM_CARS; ++ci) {
+    car_post_tick(car[ci], rb[ci]);
+    car_finish_tick(car[ci], rb[ci]);
+  }
+  RS_UNROLL
+  for (int ci = 0; ci < NUM_CARS; ++ci) {
+    Car& o = s.cars[ci];
+    if (car[ci].is_demoed) continue;  // a demoed car keeps its state
+    o.vel_impulse_cache = car[ci].vel_impulse_cache;
+    o.pos = car[ci].pos;
+    o.rot = car[ci].rot;
+    o.vel = car[ci].vel;
+    o.ang_vel = car[ci].ang_vel;
+    o.has_jumped = car[ci].has_jumped;
+    o.is_supersonic = car[ci].is_supersonic;
+    o.supersonic_grace_timer = car[ci].supersonic_grace_timer;
+    o.bump_cooldown_timer = car[ci].bump_cooldown_timer;
+    o.prev_controls = car[ci].prev_controls;
+    s.bodies[1 + ci].lin_vel = rb[ci].lin_vel;
   }
   if (w.boost_pads_enabled) boost_pads_tick(s, w);
-  const Body& rb = s.bodies[0];  // ball finish_physics_tick
-  s.ball.vel = rb.lin_vel * k::BT_TO_UU;
-  s.ball.ang_vel = rb.ang_vel;
-  s.ball.pos = rb.world.t * k::BT_TO_UU;
-  s.ball.rot = rb.world.m;
+  s.ball.vel = ball.lin_vel * k::BT_TO_UU;  // ball finish_physics_tick
+  s.ball.ang_vel = ball.ang_vel;
+  s.ball.pos = ball.world.t * k::BT_TO_UU;
+  s.ball.rot = ball.world.m;
   s.ball.tick_count_since_kickoff = u64w(u64(s.ball.tick_count_since_kickoff) + 1);
   s.tick_count = u64w(u64(s.tick_count) + 1);
 }
