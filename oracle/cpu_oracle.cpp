@@ -76,6 +76,67 @@ void rsim_cpu_static_layout(uint64_t* out) {
 uint64_t rsim_cpu_controls_word(int car) { return (offsetof(ArenaState, cars) + car * sizeof(Car) + offsetof(Car, controls)) / 4; }
 // Brute force: move_cells against the remove-then-push sequence it replaces, on `iters` random sorted lists (lengths up
 // to the cap, so overflow is exercised) and random block moves in the given world's grid. Returns the mismatch count.
+// The literal form of P4's island sort (simulation_island_manager.cuh:43-66 and the ascending sort before it) against the
+// register form, over random active lists, some with repeated entries; returns the number of differing lists.
+uint64_t rsim_cpu_check_island_sort(uint64_t seed, uint64_t iters) {
+  uint64_t bad = 0, x = seed | 1;
+  auto rnd = [&x]() {
+    x ^= x << 13;
+    x ^= x >> 7;
+    x ^= x << 17;
+    return x;
+  };
+  struct Rec {
+    static void sort(uint32_t* idx, int lo, int hi, const int* keys) {
+      int i = lo, j = hi, pivot = keys[idx[(lo + hi) / 2]];
+      for (;;) {
+        while (keys[idx[i]] < pivot) ++i;
+        while (pivot < keys[idx[j]]) --j;
+        if (i > j) break;
+        uint32_t t = idx[i];
+        idx[i] = idx[j];
+        idx[j] = t;
+        ++i;
+        if (j == 0) break;
+        --j;
+        if (i > j) break;
+      }
+      if (lo < j) sort(idx, lo, j, keys);
+      if (i < hi) sort(idx, i, hi, keys);
+    }
+  };
+  for (uint64_t it = 0; it < iters; ++it) {
+    uint32_t list[16], idx[16];
+    int keys[16], n = (int)(rnd() % 17);
+    uint32_t packed = 0;
+    for (int m = 0; m < 16; ++m) {
+      keys[m] = (int)(rnd() % 4) - 1;
+      packed |= (uint32_t)(keys[m] + 1) << (2 * m);
+    }
+    for (uint32_t i = 0; i < 16; ++i) list[i] = i;
+    for (uint32_t i = 15; i > 0; --i) {
+      const uint32_t j = (uint32_t)(rnd() % (i + 1)), t = list[i];
+      list[i] = list[j];
+      list[j] = t;
+    }
+    if (it % 8 == 0 && n > 1) list[rnd() % (uint64_t)n] = list[rnd() % (uint64_t)n];
+    for (int i = 0; i < n; ++i) {
+      int j = i - 1;
+      while (j >= 0 && idx[j] > list[i]) {
+        idx[j + 1] = idx[j];
+        --j;
+      }
+      idx[j + 1] = list[i];
+    }
+    if (n > 1) Rec::sort(idx, 0, n - 1, keys);
+    Nibbles got = sorted_nibbles(list, n);
+    hoare_sort(got, n, packed);
+    bool same = true;
+    for (int i = 0; i < n; ++i) same = same && got.get(i) == idx[i];
+    bad += same ? 0 : 1;
+  }
+  return bad;
+}
 uint64_t rsim_cpu_check_move_cells(const StaticData* w, uint64_t seed, uint64_t iters) {
   uint64_t bad = 0, x = seed | 1;
   auto rnd = [&x]() {

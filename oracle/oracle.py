@@ -57,6 +57,8 @@ class Oracle:
         L.rsim_sample_controls.argtypes = [_u64, _u32, _u32, _u32, _vp]
         L.rsim_cpu_check_move_cells.argtypes = [_vp, _u64, _u64]
         L.rsim_cpu_check_move_cells.restype = _u64
+        L.rsim_cpu_check_island_sort.argtypes = [_u64, _u64]
+        L.rsim_cpu_check_island_sort.restype = _u64
         for f in ("rsim_cpu_arena_words", "rsim_cpu_tick_words", "rsim_cpu_static_words", "rsim_cpu_controls_word"):
             getattr(L, f).restype = _u64
         self.L = L
@@ -116,6 +118,9 @@ class Oracle:
         b[nodes + used * nsize:nodes + (used + count) * nsize] = b[nodes + first * nsize:nodes + (first + count) * nsize]
         b[rec(mesh, nf_off):rec(mesh, nf_off) + 4] = np.array([used], np.uint32).view(np.uint8)
         return b.view(np.uint32)
+
+    def check_island_sort(self, seed, iters):
+        return int(self.L.rsim_cpu_check_island_sort(seed, iters))
 
     def check_move_cells(self, world, seed, iters):
         """Mismatches of the one-pass cell move against remove-then-push on random lists (brute force)."""

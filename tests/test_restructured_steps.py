@@ -9,3 +9,9 @@ def test_move_cells_equals_remove_then_push(oracle):
     for p in ((0, 0), (6, 2)):
         w = oracle.build_world(*p)
         assert oracle.check_move_cells(w, 12345 + p[0], 100000) == 0
+
+
+def test_island_sort_in_a_register_equals_the_literal_sort(oracle):
+    """simulation_island_manager.cuh:43-66 and the ascending sort before it, over active lists of 0 to 16 entries with
+    every mix of keys, some with repeated entries."""
+    assert oracle.check_island_sort(99, 2000000) == 0
