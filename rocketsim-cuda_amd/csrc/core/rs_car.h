@@ -771,7 +771,7 @@ RS_FN void wheel_rays_prepare(const ArenaState& s, const StaticData& w, WheelRay
   prep.tb.n_jobs = prep.tb.n_leaves = prep.tb.next = 0;
   prep.tb.leaves = 1;
   for (int ci = 0; ci < NUM_CARS; ++ci) {
-    prep.ncand[ci] = 0;
+    prep.cand[ci].clear();
     prep.first_job[ci] = prep.tb.n_jobs;
     if (!s.cars[ci].is_demoed) {
       const CarConst& cc = w.cars[ci];
@@ -780,8 +780,8 @@ RS_FN void wheel_rays_prepare(const ArenaState& s, const StaticData& w, WheelRay
       for (int i = 0; i < NUM_WHEELS; ++i) wheel_ray_ends(cc.wheels[i], ct, &src[i], &dst[i]);
       ClosestHits hits;
       wheel_hits_init(hits, src, dst, cc.body_idx);
-      prep.ncand[ci] = ray_screen(s, w, hits, prep.cand[ci]);
-      ray_jobs(s, w, hits, prep.cand[ci], prep.ncand[ci], prep.tb);
+      ray_screen(s, w, hits, prep.cand[ci]);
+      ray_jobs(s, w, hits, prep.cand[ci], prep.tb);
     }
     prep.end_job[ci] = prep.tb.n_jobs;
   }

@@ -554,12 +554,32 @@ RS_FN void ray_candidate(const ArenaState& s, const StaticData& w, uint32_t h, C
 // ray order; in each cell its static handles, then its dynamic ones; every handle at most once, kept if its box overlaps
 // the rays' box. The screen runs over all cells before any candidate's ray test: a ray test changes only the hits, which
 // the screen does not read, so this is the sequence of screening and testing entry by entry, with the screen's loads no
-// longer waiting behind the tests. Returns the number of candidates written to cand (at most 32).
+// longer waiting behind the tests.
 // A handle's box test does not depend on the cell it is met in, so every handle is tested once, up front, into a mask (the
 // world's box for a static handle, the proxy's for a dynamic one); the cells' ranges, their runs in the dynamic list
 // (bisections side by side) and their static entries (eight at a time) are then read as independent loads, and only the
-// walk in entry order, with its at-most-once rule, stays sequential.
-RS_FN int ray_screen(const ArenaState& s, const StaticData& w, const ClosestHits& hits, uint32_t* cand) {
+// walk in entry order, with its at-most-once rule, stays sequential. The casting car's own handle, which every candidate
+// test refuses, is left out, and the dynamic list is read only where another dynamic body's box overlaps: for a car on its
+// own, none. The candidates are kept in a register.
+struct HandleList {  // at most 32 handles of 5 bits, twelve to a word
+  uint64_t v[3];
+  int n;
+  RS_FN void clear() { v[0] = v[1] = v[2] = 0, n = 0; }
+  RS_FN void push(uint32_t h) {
+    const int word = n >= 24 ? 2 : n >= 12 ? 1 : 0;
+    const uint64_t bits = (uint64_t)h << (5 * (n - 12 * word));
+    v[0] |= word == 0 ? bits : 0ull;
+    v[1] |= word == 1 ? bits : 0ull;
+    v[2] |= word == 2 ? bits : 0ull;
+    ++n;
+  }
+  RS_FN uint32_t get(int i) const {
+    const uint64_t v0 = v[0], v1 = v[1], v2 = v[2];
+    const int word = i >= 24 ? 2 : i >= 12 ? 1 : 0;
+    return (uint32_t)((word == 2 ? v2 : word == 1 ? v1 : v0) >> (5 * (i - 12 * word))) & 31u;
+  }
+};
+RS_FN void ray_screen(const ArenaState& s, const StaticData& w, const ClosestHits& hits, HandleList& cand) {
   static_assert(NUM_HANDLES <= 32, "one bit per handle");
   Aabb rb;
   rb.min = vmin(hits.from[0], hits.to[0]);
@@ -579,14 +599,22 @@ RS_FN int ray_screen(const ArenaState& s, const StaticData& w, const ClosestHits
   uint32_t over = 0;
   RS_UNROLL
   for (int h = 0; h < NUM_HANDLES; ++h) over |= overlaps(rb, w.proxies[h].aabb) ? 1u << h : 0u;
+  uint32_t dynamic = 0;
   RS_UNROLL
   for (int d = NUM_DYN - 1; d >= 0; --d) {  // a handle's first dynamic slot gives its box
     const uint32_t bit = 1u << w.dyn_handle[d];
     over = overlaps(rb, s.dyn_proxy[d].aabb) ? over | bit : over & ~bit;
+    dynamic |= bit;
   }
+  RS_UNROLL
+  for (int h = 0; h < NUM_HANDLES; ++h)
+    if (w.proxies[h].client_body == hits.ignore_body) over &= ~(1u << h);
+  cand.clear();
+  if (over == 0) return;
   // the cell's dynamic entries: the list is sorted by cell (an invariant of the format, dump.rs:683-685), so its run
   // is found by bisection and walked in list order, the entries a full scan would visit, in the same order
-  const uint32_t nd = s.n_dyn_cells < (uint32_t)MAX_DYN_CELLS ? s.n_dyn_cells : (uint32_t)MAX_DYN_CELLS;
+  uint32_t nd = 0;
+  if (over & dynamic) nd = s.n_dyn_cells < (uint32_t)MAX_DYN_CELLS ? s.n_dyn_cells : (uint32_t)MAX_DYN_CELLS;
   CellRange cr[4];
   uint32_t lo[4], hi[4];
   RS_UNROLL
@@ -608,7 +636,6 @@ RS_FN int ray_screen(const ArenaState& s, const StaticData& w, const ClosestHits
     }
   }
   uint32_t seen = 0;  // distinct handles: at most one per bit of `seen`, so at most 32 candidates
-  int ncand = 0;
   RS_UNROLL
   for (int q = 0; q < 4; ++q) {
     if (q >= nc) break;
@@ -623,25 +650,23 @@ RS_FN int ray_screen(const ArenaState& s, const StaticData& w, const ClosestHits
         const uint32_t bit = 1u << hs[j];
         if (seen & bit) continue;
         seen |= bit;
-        if (over & bit) cand[ncand++] = hs[j];
+        if (over & bit) cand.push(hs[j]);
       }
     }
     for (uint32_t e = lo[q]; e < nd && s.dyn_cells[e].cell == cells[q]; ++e) {
       const uint32_t h = s.dyn_cells[e].handle, bit = 1u << h;
       if (seen & bit) continue;
       seen |= bit;
-      if (over & bit) cand[ncand++] = h;
+      if (over & bit) cand.push(h);
     }
   }
-  return ncand;
 }
 // The candidates' mesh walks, in the order ray_tests reaches them, appended to tb (as many as fit); a walk's node test reads
 // only the packet's box in the mesh frame, which the hits do not change, so the walks can run before the tests (on the GPU
 // pooled across the wave's lanes).
-RS_FN void ray_jobs(const ArenaState& s, const StaticData& w, ClosestHits& hits, const uint32_t* cand, int ncand,
-                    TravBatch& tb) {
-  for (int k = 0; k < ncand && tb.n_jobs < (uint32_t)TJ_MAX; ++k) {
-    const ProxyConst& p = w.proxies[cand[k]];
+RS_FN void ray_jobs(const ArenaState& s, const StaticData& w, ClosestHits& hits, const HandleList& cand, TravBatch& tb) {
+  for (int k = 0; k < cand.n && tb.n_jobs < (uint32_t)TJ_MAX; ++k) {
+    const ProxyConst& p = w.proxies[cand.get(k)];
     const uint32_t body = p.client_body;
     if (!ray_candidate_passes(p, hits) || !rays_walk_mesh(w.bodies[body].shape_kind)) continue;
     BodyRays br;
@@ -657,10 +682,10 @@ RS_FN void ray_jobs(const ArenaState& s, const StaticData& w, ClosestHits& hits,
   }
 }
 // The candidates' ray tests in screen order, mesh candidates taking their walked leaves from tb[first_job, end_job).
-RS_FN void ray_tests(const ArenaState& s, const StaticData& w, ClosestHits& hits, const uint32_t* cand, int ncand,
-                     const TravBatch& tb, uint32_t first_job, uint32_t end_job) {
+RS_FN void ray_tests(const ArenaState& s, const StaticData& w, ClosestHits& hits, const HandleList& cand, const TravBatch& tb,
+                     uint32_t first_job, uint32_t end_job) {
   uint32_t next_job = first_job;
-  for (int k = 0; k < ncand; ++k) ray_candidate(s, w, cand[k], hits, &tb, &next_job, end_job);
+  for (int k = 0; k < cand.n; ++k) ray_candidate(s, w, cand.get(k), hits, &tb, &next_job, end_job);
 }
 
 struct WheelHit {
@@ -679,8 +704,7 @@ RS_FN void wheel_hits_init(ClosestHits& hits, const V3* from, const V3* to, uint
 // respawning car casts no rays that tick), so the screen and the walks done early are the ones done at the cast.
 struct WheelRayPrep {
   TravBatch tb;
-  uint32_t cand[NUM_CARS][32];
-  int ncand[NUM_CARS];
+  HandleList cand[NUM_CARS];
   uint32_t first_job[NUM_CARS], end_job[NUM_CARS];
 };
 // vehicle/raycaster.rs cast_rays (raycaster.cuh:153-176), the screen and walks taken from the car's share of `prep`
@@ -688,7 +712,7 @@ RS_FN void cast_wheel_rays(const ArenaState& s, const StaticData& w, const V3* f
                            const WheelRayPrep& prep, int ci, WheelHit out[4]) {
   ClosestHits hits;
   wheel_hits_init(hits, from, to, ignore);
-  ray_tests(s, w, hits, prep.cand[ci], prep.ncand[ci], prep.tb, prep.first_job[ci], prep.end_job[ci]);
+  ray_tests(s, w, hits, prep.cand[ci], prep.tb, prep.first_job[ci], prep.end_job[ci]);
   RS_UNROLL for (int i = 0; i < 4; ++i) {
     out[i].some = 0;
     out[i].point = splat(0.0f);
