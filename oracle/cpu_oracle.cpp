@@ -137,6 +137,100 @@ uint64_t rsim_cpu_check_island_sort(uint64_t seed, uint64_t iters) {
   }
   return bad;
 }
+// The literal broadphase update (grid_broadphase.cuh:68-84, axis_sweep.cuh:49-127: every swap made in the state's own lists,
+// body by body and axis by axis, the cell block removed and pushed) against phase_p3a, from the given sampled state on
+// through `iters` random moves of its bodies: small steps, jumps across the arena, and moves onto another body's place.
+// Returns the number of moves after which the two states differ.
+uint64_t rsim_cpu_check_sweep(const StaticData* w, const uint32_t* state, uint64_t seed, uint64_t iters) {
+  struct Lit {
+    static void shift(ArenaState& s, uint32_t h, int ax, bool max, int by) {
+      HandleEdges& e = s.handle_edges[h];
+      if (max) e.max[ax] = (uint16_t)(e.max[ax] + by);
+      else e.min[ax] = (uint16_t)(e.min[ax] + by);
+    }
+    // the edge at i moves one way while it is out of order; passing an edge of the other kind adds or removes the pair
+    static void sort(ArenaState& s, const StaticData& w, int ax, uint32_t i, int dir, bool max, bool add) {
+      Edge* e = s.edges[ax];
+      for (;;) {
+        if (dir < 0 ? i == 0 : i + 1 >= (uint32_t)NUM_EDGES) return;
+        const uint32_t o = i + (uint32_t)dir;
+        const bool out = dir < 0 ? e[i].pos < e[o].pos : e[o].handle != 0 && e[i].pos >= e[o].pos;
+        if (!out) return;
+        const bool omax = (e[o].pos & 1u) != 0;
+        if (omax != max && overlap_2d(s, e[i].handle, e[o].handle, ax)) {
+          if (add) add_pair(s, w, e[i].handle, e[o].handle);
+          else remove_pair(s, w, e[i].handle, e[o].handle);
+        }
+        shift(s, e[o].handle, ax, omax, -dir);
+        shift(s, e[i].handle, ax, max, dir);
+        const Edge t = e[i];
+        e[i] = e[o];
+        e[o] = t;
+        i = o;
+      }
+    }
+  };
+  static ArenaState a, b;
+  memcpy(&a, state, sizeof a);
+  uint64_t bad = 0, x = seed | 1;
+  auto rnd = [&x]() {
+    x ^= x << 13;
+    x ^= x >> 7;
+    x ^= x << 17;
+    return x;
+  };
+  auto uni = [&rnd]() { return (float)(rnd() % 20001) * 1e-4f - 1.0f; };
+  for (uint64_t it = 0; it < iters; ++it) {
+    for (int d = 0; d < NUM_DYN; ++d) {
+      Body& m = a.bodies[d];
+      const uint64_t kind = rnd() % 8;
+      if (kind == 0) m.world.t = V3{uni() * 80.0f, uni() * 100.0f, uni() * 20.0f + 20.0f};
+      else if (kind == 1) m.world.t = a.bodies[rnd() % NUM_DYN].world.t + V3{uni(), uni(), uni()};
+      else if (kind < 6) m.world.t = m.world.t + V3{uni() * 2.0f, uni() * 2.0f, uni()};
+      m.interp_world.t = rnd() % 4 ? m.world.t + V3{uni(), uni(), uni()} : m.world.t;
+    }
+    b = a;
+    const V3 cbt = splat(k::CONTACT_BREAKING_THRESHOLD);
+    for (int d = 0; d < NUM_DYN; ++d) {
+      const BodyConst& bc = w->bodies[w->dyn_body[d]];
+      const Body& m = a.bodies[d];
+      if (m.collision_flags & k::CF_STATIC) continue;
+      const bool ball = bc.shape_kind == k::SHAPE_SPHERE;
+      Aabb p = ball ? sphere_box(bc.sphere_margin, m.world.t) : compound_box(bc, m.world);
+      Aabb n = ball ? sphere_box(bc.sphere_margin, m.interp_world.t) : compound_box(bc, m.interp_world);
+      p.min = vmin(p.min - cbt, n.min - cbt);
+      p.max = vmax(p.max + cbt, n.max + cbt);
+      const uint32_t h = w->dyn_handle[d];
+      DynProxy& dp = a.dyn_proxy[d];
+      dp.aabb = p;
+      uint16_t qmin[3], qmax[3];
+      sap_quantize(*w, p.min, 0, qmin);
+      sap_quantize(*w, p.max, 1, qmax);
+      for (int ax = 0; ax < 3; ++ax) {
+        const uint32_t mn = a.handle_edges[h].min[ax], mx = a.handle_edges[h].max[ax];
+        const int dmin = (int)qmin[ax] - (int)a.edges[ax][mn].pos, dmax = (int)qmax[ax] - (int)a.edges[ax][mx].pos;
+        a.edges[ax][mn].pos = qmin[ax];
+        a.edges[ax][mx].pos = qmax[ax];
+        if (dmin < 0) Lit::sort(a, *w, ax, mn, -1, false, true);
+        if (dmax > 0) Lit::sort(a, *w, ax, mx, 1, true, true);
+        if (dmin > 0) Lit::sort(a, *w, ax, mn, 1, false, false);
+        if (dmax < 0) Lit::sort(a, *w, ax, mx, -1, true, false);
+      }
+      uint32_t ni[3];
+      cell_indices(*w, p.min, ni);
+      const uint32_t nidx = cell_index(*w, ni), old = dp.cell_idx;
+      dp.cell_idx = nidx;
+      if (nidx != old) {
+        update_cells(a, *w, false, h, dp.indices);
+        for (int k = 0; k < 3; ++k) dp.indices[k] = ni[k];
+        update_cells(a, *w, true, h, ni);
+      }
+    }
+    phase_p3a(b, *w);
+    if (memcmp(&a, &b, sizeof a) != 0) ++bad;
+  }
+  return bad;
+}
 uint64_t rsim_cpu_check_move_cells(const StaticData* w, uint64_t seed, uint64_t iters) {
   uint64_t bad = 0, x = seed | 1;
   auto rnd = [&x]() {

@@ -57,6 +57,8 @@ class Oracle:
         L.rsim_sample_controls.argtypes = [_u64, _u32, _u32, _u32, _vp]
         L.rsim_cpu_check_move_cells.argtypes = [_vp, _u64, _u64]
         L.rsim_cpu_check_move_cells.restype = _u64
+        L.rsim_cpu_check_sweep.argtypes = [_vp, _vp, _u64, _u64]
+        L.rsim_cpu_check_sweep.restype = _u64
         L.rsim_cpu_check_island_sort.argtypes = [_u64, _u64]
         L.rsim_cpu_check_island_sort.restype = _u64
         for f in ("rsim_cpu_arena_words", "rsim_cpu_tick_words", "rsim_cpu_static_words", "rsim_cpu_controls_word"):
@@ -125,6 +127,10 @@ class Oracle:
     def check_move_cells(self, world, seed, iters):
         """Mismatches of the one-pass cell move against remove-then-push on random lists (brute force)."""
         return int(self.L.rsim_cpu_check_move_cells(_p(world), seed, iters))
+
+    def check_sweep(self, world, state, seed, iters):
+        """Mismatches of the broadphase phase against the literal swaps, body by body and axis by axis, over random moves."""
+        return int(self.L.rsim_cpu_check_sweep(_p(world), _p(state), seed, iters))
 
     # -- workloads (the same builder source as the product's) --
     def build_world(self, p0=0, p1=0, gravity_z=-650.0, boost_accel_scale=1.0, ball_radius=91.25):

@@ -103,8 +103,9 @@ RS_FN void remove_pair(ArenaState& s, const StaticData& w, uint32_t ha, uint32_t
 // and one axis's edge list at a time (48 words) in a copy: on the GPU the lane's LDS slice, which no other phase uses
 // between P1's wheel-ray walks and P3b's narrowphase walks; on the host a local array. A sort step is then a chain of LDS
 // reads and writes, where in private memory it was a chain of dependent round trips that also waited on the step's own
-// stores. The edge indices are copied in at the start of P3a and written back at its end for the handles whose indices
-// changed; an axis's edges are copied in when that axis's sort starts and written back over the slots the sorts wrote.
+// stores. The edge indices are copied in where a lane has a sort to run and written back after its last one for the handles
+// whose indices changed; an axis's edges are copied in when a sort of that axis starts and written back over the slots it
+// wrote.
 // Indices are masked to the copy's extent (a malformed state stays within its own lane's words).
 constexpr uint32_t SAP_HE_WORDS = 3u * NUM_HANDLES;  // then the axis's edges, at most 64 slots (NUM_EDGES of them used)
 static_assert(sizeof(HandleEdges) == 12 && sizeof(Edge) == 4 && sizeof(((ArenaState*)nullptr)->handle_edges) == 4 * SAP_HE_WORDS,
@@ -352,106 +353,133 @@ RS_FN void cell_block(const StaticData& w, const uint32_t idx[3], uint32_t lo[3]
     n[a] = (top < p ? top : p) - lo[a] + 1;
   }
 }
-// Values v of [lo, lo + n) with v < x.
-RS_FN uint32_t count_below(uint32_t x, uint32_t lo, uint32_t n) { return x <= lo ? 0u : (x - lo < n ? x - lo : n); }
+// The block's cell after `cell` in ascending order, (j, k) its row and place in the row.
+RS_FN void next_cell(uint32_t& cell, uint32_t& j, uint32_t& k, const uint32_t n[3], uint32_t nz, uint32_t nyz) {
+  ++cell, ++k;
+  if (k < n[2]) return;
+  k = 0, cell += nz - n[2], ++j;
+  if (j < n[1]) return;
+  j = 0, cell += nyz - n[1] * nz;
+}
 
 // A dynamic handle's move from the cell block around `from` to the block around `to`: the same list as removing (cell, h)
 // for every cell of the old block (first match each) and then pushing (cell, h) for every cell of the new block in
 // ascending order (each after the last entry of a cell <= it; pushes past MAX_DYN_CELLS count as overflow), computed in
-// one pass. The list is read once into registers and every entry written once to its final slot: the remove/push loops
-// shift the list through memory once per cell, a chain of dependent accesses a wave pays whenever any of its lanes moves.
+// one pass. The list is read once, the entries that stay are packed into the lane's LDS slice (a local array on the host),
+// and one loop merges the new cells into them, writing every entry once to its final slot: the remove/push loops shift the
+// list through memory once per cell, a chain of dependent accesses a wave pays whenever any of its lanes moves.
+// No division by the grid's strides: an old block's entry is found by comparing against at most three layers and rows, and
+// the new cells come by stepping. With the quotients, and the merge unrolled over the list's 64 slots, a move took 57K
+// cycles of its wave, wherever its state lay: instructions and taken branches; now 33K with the state in LDS, 44K without.
+struct CellCopy {
+#if !defined(__HIP_DEVICE_COMPILE__)
+  uint32_t words[2 * MAX_DYN_CELLS + 4];
+#endif
+  RS_FN uint32_t* word(uint32_t k) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return lane_word(k);
+#else
+    return &words[k];
+#endif
+  }
+  RS_FN DynCell get(uint32_t i) { return DynCell{*word(2 * i), *word(2 * i + 1)}; }
+  RS_FN void set(uint32_t i, DynCell e) { *word(2 * i) = e.cell, *word(2 * i + 1) = e.handle; }
+};
+static_assert(2 * MAX_DYN_CELLS + 4 <= SWEEP_WORDS, "the list and the two entries read ahead of its end fit the lane's slice");
 RS_FN void move_cells(ArenaState& s, const StaticData& w, uint32_t h, const uint32_t from[3], const uint32_t to[3]) {
   const uint32_t nz = w.grid_num_cells[2], nyz = w.grid_num_cells[1] * nz;
   uint32_t olo[3], on[3], nlo[3], nn[3];
   cell_block(w, from, olo, on);
   cell_block(w, to, nlo, nn);
-  const uint32_t total = nn[0] * nn[1] * nn[2], plane = nn[1] * nn[2];
+  const uint32_t total = nn[0] * nn[1] * nn[2];
   const uint32_t n = s.n_dyn_cells < (uint32_t)MAX_DYN_CELLS ? s.n_dyn_cells : (uint32_t)MAX_DYN_CELLS;
   DynCell e[MAX_DYN_CELLS];
-  bool keep[MAX_DYN_CELLS];
   uint32_t removed = 0, kept = 0;
+  CellCopy c;
 RS_UNROLL
   for (int i = 0; i < MAX_DYN_CELLS; ++i) e[i] = (uint32_t)i < n ? s.dyn_cells[i] : DynCell{0, 0};
 RS_UNROLL
   for (int i = 0; i < MAX_DYN_CELLS; ++i) {
-    uint32_t c = e[i].cell, ci = c / nyz, cj = (c - ci * nyz) / nz, ck = c - ci * nyz - cj * nz;
-    uint32_t di = ci - olo[0], dj = cj - olo[1], dk = ck - olo[2];  // unsigned: out of the block wraps high
-    bool in_old = e[i].handle == h && di < on[0] && dj < on[1] && dk < on[2];
-    uint32_t bit = in_old ? 1u << ((di * 3 + dj) * 3 + dk) : 0u;
-    bool drop = in_old && (removed & bit) == 0;
-    if (drop) removed |= bit;
-    keep[i] = (uint32_t)i < n && !drop;
-    kept += keep[i] ? 1u : 0u;
+    // the entry's place in the old block, if it has one: unsigned differences from the block's first layer, row and cell,
+    // each below the block's extent (at most three) times its stride; below it the difference wraps high
+    uint32_t r = e[i].cell - olo[0] * nyz;
+    bool in_old = e[i].handle == h && r < on[0] * nyz;
+    const uint32_t di = (r >= nyz ? 1u : 0u) + (r >= 2 * nyz ? 1u : 0u);
+    r = r - di * nyz - olo[1] * nz;
+    in_old = in_old && r < on[1] * nz;
+    const uint32_t dj = (r >= nz ? 1u : 0u) + (r >= 2 * nz ? 1u : 0u);
+    r = r - dj * nz - olo[2];
+    in_old = in_old && r < on[2];
+    const uint32_t bit = in_old ? 1u << (((di * 3 + dj) * 3 + r) & 31u) : 0u;
+    const bool drop = in_old && (removed & bit) == 0;
+    removed |= bit;
+    c.set(kept, e[i]);  // kept <= i; an entry that goes is written over by the next
+    kept += (uint32_t)i < n && !drop ? 1u : 0u;
   }
   const uint32_t room = (uint32_t)MAX_DYN_CELLS - kept, placed = total < room ? total : room;
-  uint32_t m = 0, done = 0;  // old entries written, new entries written
-RS_UNROLL
-  for (int i = 0; i < MAX_DYN_CELLS; ++i) {
-    if (!keep[i]) continue;
-    // new cells below this entry's cell (new cells are visited in ascending index order, which is (i, j, k) order)
-    uint32_t c = e[i].cell, ci = c / nyz, cj = (c - ci * nyz) / nz, ck = c - ci * nyz - cj * nz;
-    uint32_t below = count_below(ci, nlo[0], nn[0]) * plane;
-    if (ci - nlo[0] < nn[0]) {
-      below += count_below(cj, nlo[1], nn[1]) * nn[2];
-      if (cj - nlo[1] < nn[1]) below += count_below(ck, nlo[2], nn[2]);
+  uint32_t next = nlo[0] * nyz + nlo[1] * nz + nlo[2], nj = 0, nk = 0;  // the next new cell (ascending in (i, j, k) order)
+  DynCell cur = c.get(0), ahead = c.get(1);
+  for (uint32_t m = 0, done = 0; m + done < kept + placed;) {  // a new cell goes before the first entry of a higher cell
+    const bool fresh = done < placed && (m >= kept || next < cur.cell);
+    s.dyn_cells[m + done] = DynCell{fresh ? next : cur.cell, fresh ? h : cur.handle};
+    if (fresh) {
+      ++done;
+      next_cell(next, nj, nk, nn, nz, nyz);
+    } else {
+      ++m;
+      cur = ahead;
+      ahead = c.get(m + 1);
     }
-    if (below > placed) below = placed;
-    for (; done < below; ++done) {
-      uint32_t a = done / plane, r = done - a * plane, b = r / nn[2], k2 = r - b * nn[2];
-      s.dyn_cells[done + m] = DynCell{(nlo[0] + a) * nyz + (nlo[1] + b) * nz + nlo[2] + k2, h};
-    }
-    s.dyn_cells[done + m] = e[i];
-    ++m;
-  }
-  for (; done < placed; ++done) {
-    uint32_t a = done / plane, r = done - a * plane, b = r / nn[2], k2 = r - b * nn[2];
-    s.dyn_cells[done + m] = DynCell{(nlo[0] + a) * nyz + (nlo[1] + b) * nz + nlo[2] + k2, h};
   }
   for (uint32_t i = kept + placed; i < n; ++i) s.dyn_cells[i] = DynCell{0, 0};
   s.n_dyn_cells = kept + placed;
   s.overflow[OVF_DYN_CELLS] += total - placed;
 }
-RS_FN void grid_set_aabb(ArenaState& s, const StaticData& w, SapCopy& c, uint32_t d, Aabb box) {  // grid_broadphase.cuh:68-84
-  uint32_t h = w.dyn_handle[d];
-  s.dyn_proxy[d].aabb = box;
-  uint16_t qmin[3], qmax[3];
-  sap_quantize(w, box.min, 0, qmin);
-  sap_quantize(w, box.max, 1, qmax);
-  // the handle's six edge positions read together; an axis whose edges keep their positions is left alone, as
-  // update_axis would. Sorting one axis changes only that axis's edges and edge indices, so the other axes' reads stand.
-  uint32_t hmin[3], hmax[3];
-  for (int ax = 0; ax < 3; ++ax) {
-    hmin[ax] = c.he_get(h, (uint32_t)ax);
-    hmax[ax] = c.he_get(h, 3u + ax);
-  }
-  uint16_t pmin[3], pmax[3];
-  for (int ax = 0; ax < 3; ++ax) {
-    pmin[ax] = s.edges[ax][hmin[ax]].pos;
-    pmax[ax] = s.edges[ax][hmax[ax]].pos;
-  }
-  for (int ax = 0; ax < 3; ++ax)
-    if (qmin[ax] != pmin[ax] || qmax[ax] != pmax[ax]) update_axis(s, w, c, ax, h, qmin[ax], qmax[ax]);
-  uint32_t old = s.dyn_proxy[d].cell_idx, ni[3];
-  cell_indices(w, box.min, ni);
-  uint32_t nidx = cell_index(w, ni);
-  s.dyn_proxy[d].cell_idx = nidx;
-  if (nidx != old) {
-    uint32_t from[3] = {s.dyn_proxy[d].indices[0], s.dyn_proxy[d].indices[1], s.dyn_proxy[d].indices[2]};
-    for (int a = 0; a < 3; ++a) s.dyn_proxy[d].indices[a] = ni[a];
-    move_cells(s, w, h, from, ni);  // = update_cells(remove, from) then update_cells(add, ni)
-  }
+// An axis's new edge positions leave the edge order as it is (no sort step would swap), read from the state's lists. Each
+// compare is the first one of the sort that dmin or dmax starts, against the two edges' new positions; edge indices that
+// are out of range or out of order (a malformed state) are left to the sorts.
+RS_FN bool edges_stay(const ArenaState& s, int ax, uint32_t mn, uint32_t mx, uint16_t qmin, uint16_t qmax, bool* same) {
+  constexpr uint32_t TOP = (uint32_t)NUM_EDGES - 1u;
+  const bool valid = mn < mx && mx <= TOP;
+  const uint32_t a = valid ? mn : 0u, b = valid ? mx : 0u;
+  const Edge emn = s.edges[ax][a], emx = s.edges[ax][b];
+  const Edge before_mn = s.edges[ax][a > 0 ? a - 1 : 0], after_mx = s.edges[ax][b < TOP ? b + 1 : TOP];
+  const Edge after_mn = s.edges[ax][a < TOP ? a + 1 : TOP], before_mx = s.edges[ax][b > 0 ? b - 1 : 0];
+  *same = valid && qmin == emn.pos && qmax == emx.pos;
+  const bool apart = b > a + 1;  // else the two edges are each other's neighbours: their order is that of qmin and qmax
+  const bool min_down = qmin < emn.pos && a > 0 && qmin < before_mn.pos;
+  const bool max_up = qmax > emx.pos && b < TOP && after_mx.handle != 0 && qmax >= after_mx.pos;
+  const bool min_up = qmin > emn.pos && (apart ? after_mn.handle != 0 && qmin >= after_mn.pos : qmin >= qmax);
+  const bool max_down = qmax < emx.pos && (apart ? qmax < before_mx.pos : qmax < qmin);
+  return valid && !min_down && !max_up && !min_up && !max_down;
 }
 
-// P3a (collision_world.cuh:34-50): the dynamic bodies' swept boxes (current and predicted transform, each grown by the
-// contact breaking threshold) into the broadphase, the sweep working on its copy (SapCopy).
+// P3a (collision_world.cuh:34-50, grid_broadphase.cuh:68-84): the dynamic bodies' swept boxes (current and predicted
+// transform, each grown by the contact breaking threshold) into the broadphase.
+// Of a body's axis updates about one in twenty moves an edge past another; the rest only write positions. So the updates
+// run in two steps. First, in body and axis order, every update that leaves its axis's order as it is writes its two
+// positions in place, from six loads; one that does not is put off, and so are the later bodies' updates of that axis.
+// Then each lane runs its own put-off updates in order, the sweep working on its copy (SapCopy), so a wave pays for the
+// most that one of its lanes has (two or three) and not for all nine. The order that matters is kept: an update in place
+// changes no edge index and no pair, and reads and writes its own axis's edges only, so it commutes with the other axes'
+// sorts (whose overlap tests read edge indices); and a body's sorts and its cell list share no data, so the cell moves
+// come last, again each lane its own. With every update copying its axis in and out, P3a took 183K cycles per wave and
+// tick of contact play at 65,536 arenas, 91K at kickoff and 38K for one arena a wave in LDS; now 140K, 82K and 23K.
 RS_INLINE void phase_p3a(ArenaState& s, const StaticData& w) {
-  SapCopy c;
-  sap_copy_in(s, c);
   const V3 cbt = splat(k::CONTACT_BREAKING_THRESHOLD);
+  // everything that the bodies' moves are computed from, read together before the first store
+  uint32_t put_off = 0, moved = 0, live = 0;  // bit 3 d + axis; bit d
+  uint32_t q[3 * NUM_DYN];                    // new positions, the min edge's low
+  Aabb box[NUM_DYN];
+  HandleEdges he[NUM_DYN];
+  uint32_t cell[NUM_DYN];
+  RS_UNROLL
   for (uint32_t d = 0; d < (uint32_t)NUM_DYN; ++d) {
     const BodyConst& bc = w.bodies[w.dyn_body[d]];
     const Body& b = s.bodies[d];
-    if (b.collision_flags & k::CF_STATIC) continue;
+    he[d] = s.handle_edges[w.dyn_handle[d]];
+    cell[d] = s.dyn_proxy[d].cell_idx;
+    if (!(b.collision_flags & k::CF_STATIC)) live |= 1u << d;
     Aabb a = bc.shape_kind == k::SHAPE_SPHERE ? sphere_box(bc.sphere_margin, b.world.t) : compound_box(bc, b.world);
     a.min -= cbt;
     a.max += cbt;
@@ -460,9 +488,59 @@ RS_INLINE void phase_p3a(ArenaState& s, const StaticData& w) {
     a2.max += cbt;
     a.min = vmin(a.min, a2.min);
     a.max = vmax(a.max, a2.max);
-    grid_set_aabb(s, w, c, d, a);
+    box[d] = a;
+    uint16_t qmin[3], qmax[3];
+    sap_quantize(w, a.min, 0, qmin);
+    sap_quantize(w, a.max, 1, qmax);
+    RS_UNROLL
+    for (int ax = 0; ax < 3; ++ax) q[3 * d + ax] = (uint32_t)qmax[ax] << 16 | qmin[ax];
+    uint32_t ni[3];
+    cell_indices(w, a.min, ni);
+    const uint32_t nidx = cell_index(w, ni);
+    if (nidx != cell[d]) moved |= 1u << d;
+    cell[d] = nidx;
   }
-  sap_copy_out(s, c);
+  moved &= live;
+  RS_UNROLL
+  for (uint32_t d = 0; d < (uint32_t)NUM_DYN; ++d) {
+    if (!(live & (1u << d))) continue;
+    bool stay[3], same[3];
+    RS_UNROLL
+    for (int ax = 0; ax < 3; ++ax)
+      stay[ax] = edges_stay(s, ax, he[d].min[ax], he[d].max[ax], (uint16_t)q[3 * d + ax], (uint16_t)(q[3 * d + ax] >> 16), &same[ax]);
+    RS_UNROLL
+    for (int ax = 0; ax < 3; ++ax) {
+      if (put_off & (0x49u << ax) || !stay[ax]) {
+        put_off |= 1u << (3 * d + ax);
+      } else if (!same[ax]) {
+        s.edges[ax][he[d].min[ax]].pos = (uint16_t)q[3 * d + ax];
+        s.edges[ax][he[d].max[ax]].pos = (uint16_t)(q[3 * d + ax] >> 16);
+      }
+    }
+    s.dyn_proxy[d].aabb = box[d];
+    if (moved & (1u << d)) s.dyn_proxy[d].cell_idx = cell[d];
+  }
+  if (put_off) {
+    SapCopy c;
+    sap_copy_in(s, c);
+    do {
+      const int o = __builtin_ctz(put_off), d = o >= 6 ? 2 : o >= 3 ? 1 : 0;
+      put_off &= put_off - 1;
+      uint32_t qo = q[0];
+      RS_UNROLL
+      for (int i = 1; i < 3 * NUM_DYN; ++i) qo = i == o ? q[i] : qo;
+      update_axis(s, w, c, o - 3 * d, w.dyn_handle[d], (uint16_t)qo, (uint16_t)(qo >> 16));
+    } while (put_off);
+    sap_copy_out(s, c);
+  }
+  while (moved) {
+    const int d = __builtin_ctz(moved);
+    moved &= moved - 1;
+    uint32_t from[3] = {s.dyn_proxy[d].indices[0], s.dyn_proxy[d].indices[1], s.dyn_proxy[d].indices[2]}, to[3];
+    cell_indices(w, s.dyn_proxy[d].aabb.min, to);
+    for (int a = 0; a < 3; ++a) s.dyn_proxy[d].indices[a] = to[a];
+    move_cells(s, w, w.dyn_handle[d], from, to);  // = update_cells(remove, from) then update_cells(add, to)
+  }
 }
 
 }  // namespace rs
