@@ -761,41 +761,67 @@ template <bool UW, class M>
 RS_NOINL void car_pre_tick_in(typename M::template Ptr<ArenaState> sp, const RS_CONST_AS StaticData* wp, int ci,
                               const RS_PRIVATE_AS WheelRayPrep* pp) {
   if (UW) wp = rs_uniform_ptr(wp);
-  RS_UNIFORM_INDEX(ci);
+  if (!M::SPLIT) RS_UNIFORM_INDEX(ci);
   car_pre_tick(*(ArenaState*)sp, *(const StaticData*)wp, ci, *(const WheelRayPrep*)pp);
 }
-// Both cars' wheel-ray screens and mesh walks, before either car's pre-tick (exact: see WheelRayPrep). A demoed car casts
-// no rays this tick (its pre-tick respawns it at most); its share is empty.
-template <class M>
-RS_FN void wheel_rays_prepare(const ArenaState& s, const StaticData& w, WheelRayPrep& prep) {
-  prep.tb.n_jobs = prep.tb.n_leaves = prep.tb.next = 0;
-  prep.tb.leaves = 1;
-  for (int ci = 0; ci < NUM_CARS; ++ci) {
-    prep.cand[ci].clear();
-    prep.first_job[ci] = prep.tb.n_jobs;
-    if (!s.cars[ci].is_demoed) {
-      const CarConst& cc = w.cars[ci];
-      const Aff ct = s.bodies[dyn_slot(w, cc.body_idx)].world;
-      V3 src[NUM_WHEELS], dst[NUM_WHEELS];
-      for (int i = 0; i < NUM_WHEELS; ++i) wheel_ray_ends(cc.wheels[i], ct, &src[i], &dst[i]);
-      ClosestHits hits;
-      wheel_hits_init(hits, src, dst, cc.body_idx);
-      ray_screen(s, w, hits, prep.cand[ci]);
-      ray_jobs(s, w, hits, prep.cand[ci], prep.tb);
-    }
-    prep.end_job[ci] = prep.tb.n_jobs;
+// Car ci's wheel-ray screen and mesh jobs. Returns whether its rays may hit a dynamic body. A demoed car casts no rays this
+// tick (its pre-tick respawns it at most); its share is empty.
+RS_FN bool wheel_rays_collect(const ArenaState& s, const StaticData& w, int ci, WheelRayPrep& prep) {
+  bool dynamic = false;
+  prep.cand[ci].clear();
+  prep.first_job[ci] = prep.tb.n_jobs;
+  if (!s.cars[ci].is_demoed) {
+    const CarConst& cc = w.cars[ci];
+    const Aff ct = s.bodies[dyn_slot(w, cc.body_idx)].world;
+    V3 src[NUM_WHEELS], dst[NUM_WHEELS];
+    for (int i = 0; i < NUM_WHEELS; ++i) wheel_ray_ends(cc.wheels[i], ct, &src[i], &dst[i]);
+    ClosestHits hits;
+    wheel_hits_init(hits, src, dst, cc.body_idx);
+    dynamic = ray_screen(s, w, hits, prep.cand[ci]);
+    ray_jobs(s, w, hits, prep.cand[ci], prep.tb);
   }
-  trav_run<M>(w, prep.tb);
+  prep.end_job[ci] = prep.tb.n_jobs;
+  return dynamic;
 }
+// Both cars' screens and walks come before either car's pre-tick (exact: see WheelRayPrep).
+// Where a state is split over lanes, each car has a lane of its own. The cars' pre-ticks then run side by side when neither
+// car's rays can meet a dynamic body and neither car is demoed: a pre-tick reads and writes its own car and chassis, the
+// bodies its rays hit, and, at a respawn, the random state. Otherwise the first car's lane goes first, then the second's.
 template <bool UW = false, class M = InPrivate>
 RS_INLINE void phase_p1(ArenaState& s, const StaticData& w) {
-  for (int ci = 0; ci < NUM_CARS; ++ci) car_flip_zdamp(s, w, ci);
+  using SP = typename M::template Ptr<ArenaState>;
   WheelRayPrep prep;
-  wheel_rays_prepare<M>(s, w, prep);
+  prep.tb.n_jobs = prep.tb.n_leaves = prep.tb.next = 0;
+  prep.tb.leaves = 1;
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (M::SPLIT) {
+    const uint32_t arena = split_arena(), ci = split_role();
+    if (ci < (uint32_t)NUM_CARS) {
+      car_flip_zdamp(s, w, (int)ci);
+      const bool dynamic = wheel_rays_collect(s, w, (int)ci, prep);
+      trav_run<M>(w, prep.tb);
+      const bool was = s.cars[ci].is_on_ground != 0;
+      const uint64_t tied = __ballot(dynamic || s.cars[ci].is_demoed != 0);
+      const bool in_order = ((tied >> arena | tied >> (arena + InLds::ARENAS)) & 1u) != 0;
+      for (uint32_t turn = 0; turn < (uint32_t)NUM_CARS; ++turn) {
+        if (turn == (in_order ? ci : 0u))
+          car_pre_tick_in<UW, M>((SP)&s, (const RS_CONST_AS StaticData*)&w, (int)ci, (const RS_PRIVATE_AS WheelRayPrep*)&prep);
+        wave_lds_sync();
+      }
+      const uint64_t landed = __ballot(!was && s.cars[ci].is_on_ground);
+      const uint32_t bits = (uint32_t)(landed >> arena & 1u) << EV_LANDED |
+                            (uint32_t)(landed >> (arena + InLds::ARENAS) & 1u) << (EV_LANDED + 1);
+      if (ci == 0 && bits != 0) s.events |= bits;
+    }
+    return;
+  }
+#endif
+  for (int ci = 0; ci < NUM_CARS; ++ci) car_flip_zdamp(s, w, ci);
+  for (int ci = 0; ci < NUM_CARS; ++ci) wheel_rays_collect(s, w, ci, prep);
+  trav_run<M>(w, prep.tb);
   for (int ci = 0; ci < NUM_CARS; ++ci) {
     uint32_t was = s.cars[ci].is_on_ground;
-    car_pre_tick_in<UW, M>((typename M::template Ptr<ArenaState>)&s, (const RS_CONST_AS StaticData*)&w, ci,
-                           (const RS_PRIVATE_AS WheelRayPrep*)&prep);
+    car_pre_tick_in<UW, M>((SP)&s, (const RS_CONST_AS StaticData*)&w, ci, (const RS_PRIVATE_AS WheelRayPrep*)&prep);
     if (!was && s.cars[ci].is_on_ground) s.events |= 1u << (EV_LANDED + ci);
   }
 }

@@ -85,12 +85,14 @@ namespace rs {
 // Where the lanes' ArenaStates live, and how many arenas a wave steps at most: private memory, one arena per lane, or LDS,
 // a few arenas per wave.
 struct InPrivate {
-  static constexpr uint32_t ARENAS = 64;
+  static constexpr uint32_t ARENAS = 64, WALKERS = 64;
+  static constexpr bool SPLIT = false;
   template <class T>
   using Ptr = RS_PRIVATE_AS T*;
 };
 struct InLds {
-  static constexpr uint32_t ARENAS = 3;
+  static constexpr uint32_t ARENAS = 3, ROLES = 3, WALKERS = 2 * ARENAS;
+  static constexpr bool SPLIT = true;
   template <class T>
   using Ptr = RS_LDS_AS T*;
 };

@@ -554,7 +554,7 @@ RS_FN void ray_candidate(const ArenaState& s, const StaticData& w, uint32_t h, C
 // ray order; in each cell its static handles, then its dynamic ones; every handle at most once, kept if its box overlaps
 // the rays' box. The screen runs over all cells before any candidate's ray test: a ray test changes only the hits, which
 // the screen does not read, so this is the sequence of screening and testing entry by entry, with the screen's loads no
-// longer waiting behind the tests.
+// longer waiting behind the tests. Returns whether a dynamic body may be hit (its box overlaps the rays' box).
 // A handle's box test does not depend on the cell it is met in, so every handle is tested once, up front, into a mask (the
 // world's box for a static handle, the proxy's for a dynamic one); the cells' ranges, their runs in the dynamic list
 // (bisections side by side) and their static entries (eight at a time) are then read as independent loads, and only the
@@ -579,7 +579,7 @@ struct HandleList {  // at most 32 handles of 5 bits, twelve to a word
     return (uint32_t)((word == 2 ? v2 : word == 1 ? v1 : v0) >> (5 * (i - 12 * word))) & 31u;
   }
 };
-RS_FN void ray_screen(const ArenaState& s, const StaticData& w, const ClosestHits& hits, HandleList& cand) {
+RS_FN bool ray_screen(const ArenaState& s, const StaticData& w, const ClosestHits& hits, HandleList& cand) {
   static_assert(NUM_HANDLES <= 32, "one bit per handle");
   Aabb rb;
   rb.min = vmin(hits.from[0], hits.to[0]);
@@ -610,7 +610,7 @@ RS_FN void ray_screen(const ArenaState& s, const StaticData& w, const ClosestHit
   for (int h = 0; h < NUM_HANDLES; ++h)
     if (w.proxies[h].client_body == hits.ignore_body) over &= ~(1u << h);
   cand.clear();
-  if (over == 0) return;
+  if (over == 0) return false;
   // the cell's dynamic entries: the list is sorted by cell (an invariant of the format, dump.rs:683-685), so its run
   // is found by bisection and walked in list order, the entries a full scan would visit, in the same order
   uint32_t nd = 0;
@@ -660,6 +660,7 @@ RS_FN void ray_screen(const ArenaState& s, const StaticData& w, const ClosestHit
       if (over & bit) cand.push(h);
     }
   }
+  return (over & dynamic) != 0;
 }
 // The candidates' mesh walks, in the order ray_tests reaches them, appended to tb (as many as fit); a walk's node test reads
 // only the packet's box in the mesh frame, which the hits do not change, so the walks can run before the tests (on the GPU

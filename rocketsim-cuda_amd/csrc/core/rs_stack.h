@@ -44,6 +44,9 @@ __device__ inline uint32_t* wave_lds() {
 // Word k of this lane's slice, and word k of lane `slot`'s slice of the same wave.
 __device__ inline uint32_t* lane_word(uint32_t k) { return wave_lds() + ((threadIdx.x & 63u) * (uint32_t)LANE_LDS_WORDS + k); }
 __device__ inline uint32_t* wave_lane_word(uint32_t slot, uint32_t k) { return wave_lds() + (slot * (uint32_t)LANE_LDS_WORDS + k); }
+// The lane's arena of the wave and its part in it, where a state is split over lanes (SPLIT): lane = arena + 3 * role.
+__device__ inline uint32_t split_arena() { return (threadIdx.x & 63u) % InLds::ARENAS; }
+__device__ inline uint32_t split_role() { return (threadIdx.x & 63u) / InLds::ARENAS; }
 struct TravStack {
   uint32_t spill[TRAV_CAP - TRAV_LDS];
   int n;

@@ -12,8 +12,42 @@ namespace rs {
 // P0, P2, P6 and P8 touch a few fields of every body or car: they read them all first and write them all last, so that the
 // bodies' reads are in flight together instead of each body's behind the branches and stores of the one before.
 
+// Where a state is split over lanes (SPLIT), lane role d takes body d (and its car), every lane the one of its role.
+
 // ---- P0 (arena_base.cuh:21-38) ---------------------------------------------------------------------------------------------------
+// The body's limits and the quantisation: the ball is body 0, then the cars.
+RS_FN void limit_and_quantize(Body& b, const StaticData& w, uint32_t d) {
+  const float lin = d == 0 ? w.mut_f[MF_BALL_MAX_SPEED] * k::UU_TO_BT : k::CAR_MAX_SPEED * k::UU_TO_BT;
+  limit_vels(b, lin, d == 0 ? k::BALL_MAX_ANG_SPEED : k::CAR_MAX_ANG_SPEED);
+  quantize_body(&b.world.t, &b.lin_vel, &b.ang_vel);
+}
+template <class M>
 RS_INLINE void phase_p0(ArenaState& s, const StaticData& w) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (M::SPLIT) {
+    const uint32_t d = split_role();
+    Body& o = s.bodies[d];
+    Body b;
+    b.world.t = o.world.t;
+    b.lin_vel = o.lin_vel;
+    b.ang_vel = o.ang_vel;
+    limit_and_quantize(b, w, d);
+    clear_accum(o);
+    o.world.t = b.world.t;
+    o.lin_vel = b.lin_vel;
+    o.ang_vel = b.ang_vel;
+    const V3 vel = b.lin_vel * k::BT_TO_UU;
+    if (d == 0) {
+      s.events = 0;
+      s.ball.vel = vel;
+      s.ball.ang_vel = b.ang_vel;
+    } else {
+      s.cars[d - 1].vel = vel;
+      s.cars[d - 1].ang_vel = b.ang_vel;
+    }
+    return;
+  }
+#endif
   s.events = 0;
   Body b[NUM_DYN];
   RS_UNROLL
@@ -23,11 +57,7 @@ RS_INLINE void phase_p0(ArenaState& s, const StaticData& w) {
     b[d].ang_vel = s.bodies[d].ang_vel;
   }
   RS_UNROLL
-  for (int d = 0; d < NUM_DYN; ++d) {  // the ball (0), then the cars: their limits and the quantisation
-    if (d == 0) limit_vels(b[d], w.mut_f[MF_BALL_MAX_SPEED] * k::UU_TO_BT, k::BALL_MAX_ANG_SPEED);
-    else limit_vels(b[d], k::CAR_MAX_SPEED * k::UU_TO_BT, k::CAR_MAX_ANG_SPEED);
-    quantize_body(&b[d].world.t, &b[d].lin_vel, &b[d].ang_vel);
-  }
+  for (int d = 0; d < NUM_DYN; ++d) limit_and_quantize(b[d], w, (uint32_t)d);
   RS_UNROLL
   for (int d = 0; d < NUM_DYN; ++d) {
     clear_accum(s.bodies[d]);
@@ -45,58 +75,81 @@ RS_INLINE void phase_p0(ArenaState& s, const StaticData& w) {
 }
 
 // ---- P2 / P6 (discrete_dynamics_world.cuh) ---------------------------------------------------------------------------------------
+RS_FN void predict_motion(Body& b, const StaticData& w, uint32_t d, V3 g, float dt) {
+  if (body_active(b)) add_lin_impulse(b, g, true);
+  if (b.activation == k::ACT_SLEEPING) {
+    b.interp_world = b.world;
+    return;
+  }
+  apply_damping(b, w.bodies[w.dyn_body[d]], dt);
+  b.interp_world = predict_trans(b, dt);
+}
+RS_FN void predict_motion_store(Body& o, const Body& b) {
+  o.interp_world = b.interp_world;
+  o.lin_vel = b.lin_vel;
+  o.accum_lin_vel = b.accum_lin_vel;
+  o.accum_ang_vel = b.accum_ang_vel;
+  o.cached_linear_damping = b.cached_linear_damping;
+  o.cached_damping_time_step = b.cached_damping_time_step;
+  o.cached_linear_damping_value = b.cached_linear_damping_value;
+}
+template <class M>
 RS_INLINE void phase_p2(ArenaState& s, const StaticData& w) {
   const float dt = 1.0f / 120.0f;
   V3 g = w.gravity_bt * dt;
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (M::SPLIT) {
+    const uint32_t d = split_role();
+    Body b = s.bodies[d];
+    predict_motion(b, w, d, g, dt);
+    predict_motion_store(s.bodies[d], b);
+    return;
+  }
+#endif
   Body b[NUM_DYN];
   RS_UNROLL
   for (int d = 0; d < NUM_DYN; ++d) b[d] = s.bodies[d];
   RS_UNROLL
-  for (int d = 0; d < NUM_DYN; ++d) {
-    if (body_active(b[d])) add_lin_impulse(b[d], g, true);
-    if (b[d].activation == k::ACT_SLEEPING) {
-      b[d].interp_world = b[d].world;
-      continue;
-    }
-    apply_damping(b[d], w.bodies[w.dyn_body[d]], dt);
-    b[d].interp_world = predict_trans(b[d], dt);
-  }
+  for (int d = 0; d < NUM_DYN; ++d) predict_motion(b[d], w, (uint32_t)d, g, dt);
   RS_UNROLL
-  for (int d = 0; d < NUM_DYN; ++d) {
-    Body& o = s.bodies[d];
-    o.interp_world = b[d].interp_world;
-    o.lin_vel = b[d].lin_vel;
-    o.accum_lin_vel = b[d].accum_lin_vel;
-    o.accum_ang_vel = b[d].accum_ang_vel;
-    o.cached_linear_damping = b[d].cached_linear_damping;
-    o.cached_damping_time_step = b[d].cached_damping_time_step;
-    o.cached_linear_damping_value = b[d].cached_linear_damping_value;
-  }
+  for (int d = 0; d < NUM_DYN; ++d) predict_motion_store(s.bodies[d], b[d]);
 }
+RS_FN bool integrate(Body& b, const StaticData& w, uint32_t d, float dt) {  // whether the body moved
+  const BodyConst& c = w.bodies[w.dyn_body[d]];
+  const bool moved = body_active(b);
+  if (moved) set_com_trans(b, c, predict_trans(b, dt));
+  update_activation(b, c, dt);
+  return moved;
+}
+RS_FN void integrate_store(Body& o, const Body& b, bool moved) {
+  o.activation = b.activation;
+  o.deactivation_time = b.deactivation_time;
+  if (!moved) return;
+  o.world = b.world;
+  o.world_quat = b.world_quat;
+  o.interp_world = b.interp_world;
+  o.inv_inertia_world = b.inv_inertia_world;
+}
+template <class M>
 RS_INLINE void phase_p6(ArenaState& s, const StaticData& w) {
   const float dt = 1.0f / 120.0f;
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (M::SPLIT) {
+    const uint32_t d = split_role();
+    Body b = s.bodies[d];
+    const bool moved = integrate(b, w, d, dt);
+    integrate_store(s.bodies[d], b, moved);
+    return;
+  }
+#endif
   Body b[NUM_DYN];
   RS_UNROLL
   for (int d = 0; d < NUM_DYN; ++d) b[d] = s.bodies[d];
   bool moved[NUM_DYN];
   RS_UNROLL
-  for (int d = 0; d < NUM_DYN; ++d) {
-    const BodyConst& c = w.bodies[w.dyn_body[d]];
-    moved[d] = body_active(b[d]);
-    if (moved[d]) set_com_trans(b[d], c, predict_trans(b[d], dt));
-    update_activation(b[d], c, dt);
-  }
+  for (int d = 0; d < NUM_DYN; ++d) moved[d] = integrate(b[d], w, (uint32_t)d, dt);
   RS_UNROLL
-  for (int d = 0; d < NUM_DYN; ++d) {
-    Body& o = s.bodies[d];
-    o.activation = b[d].activation;
-    o.deactivation_time = b[d].deactivation_time;
-    if (!moved[d]) continue;
-    o.world = b[d].world;
-    o.world_quat = b[d].world_quat;
-    o.interp_world = b[d].interp_world;
-    o.inv_inertia_world = b[d].inv_inertia_world;
-  }
+  for (int d = 0; d < NUM_DYN; ++d) integrate_store(s.bodies[d], b[d], moved[d]);
 }
 
 // ---- P7 (arena_base.cuh:43-205, ball_base.cuh:22-48) ------------------------------------------------------------------------------
@@ -377,7 +430,50 @@ RS_FN void boost_pads_tick(ArenaState& s, const StaticData& w) {  // boost_pad_g
       if (touching[cj] == i) win[cj] = nw;
   }
 }
+RS_FN void car_tick_store(ArenaState& s, uint32_t ci, const Car& car, const Body& rb) {
+  if (car.is_demoed) return;  // a demoed car keeps its state
+  Car& o = s.cars[ci];
+  o.vel_impulse_cache = car.vel_impulse_cache;
+  o.pos = car.pos;
+  o.rot = car.rot;
+  o.vel = car.vel;
+  o.ang_vel = car.ang_vel;
+  o.has_jumped = car.has_jumped;
+  o.is_supersonic = car.is_supersonic;
+  o.supersonic_grace_timer = car.supersonic_grace_timer;
+  o.bump_cooldown_timer = car.bump_cooldown_timer;
+  o.prev_controls = car.prev_controls;
+  s.bodies[1 + ci].lin_vel = rb.lin_vel;
+}
+RS_FN void ball_finish_tick(ArenaState& s, const Body& ball) {  // ball finish_physics_tick
+  s.ball.vel = ball.lin_vel * k::BT_TO_UU;
+  s.ball.ang_vel = ball.ang_vel;
+  s.ball.pos = ball.world.t * k::BT_TO_UU;
+  s.ball.rot = ball.world.m;
+  s.ball.tick_count_since_kickoff = u64w(u64(s.ball.tick_count_since_kickoff) + 1);
+}
+template <class M>
 RS_INLINE void phase_p8(ArenaState& s, const StaticData& w) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (M::SPLIT) {
+    const uint32_t d = split_role();
+    if (d == 0) {
+      ball_finish_tick(s, s.bodies[0]);
+    } else {
+      Car car = s.cars[d - 1];
+      Body rb = s.bodies[d];
+      car_post_tick(car, rb);
+      car_finish_tick(car, rb);
+      car_tick_store(s, d - 1, car, rb);
+    }
+    wave_lds_sync();
+    if (d == 0) {
+      if (w.boost_pads_enabled) boost_pads_tick(s, w);
+      s.tick_count = u64w(u64(s.tick_count) + 1);
+    }
+    return;
+  }
+#endif
   Car car[NUM_CARS];
   Body rb[NUM_CARS];
   RS_UNROLL
@@ -392,27 +488,9 @@ RS_INLINE void phase_p8(ArenaState& s, const StaticData& w) {
     car_finish_tick(car[ci], rb[ci]);
   }
   RS_UNROLL
-  for (int ci = 0; ci < NUM_CARS; ++ci) {
-    Car& o = s.cars[ci];
-    if (car[ci].is_demoed) continue;  // a demoed car keeps its state
-    o.vel_impulse_cache = car[ci].vel_impulse_cache;
-    o.pos = car[ci].pos;
-    o.rot = car[ci].rot;
-    o.vel = car[ci].vel;
-    o.ang_vel = car[ci].ang_vel;
-    o.has_jumped = car[ci].has_jumped;
-    o.is_supersonic = car[ci].is_supersonic;
-    o.supersonic_grace_timer = car[ci].supersonic_grace_timer;
-    o.bump_cooldown_timer = car[ci].bump_cooldown_timer;
-    o.prev_controls = car[ci].prev_controls;
-    s.bodies[1 + ci].lin_vel = rb[ci].lin_vel;
-  }
+  for (int ci = 0; ci < NUM_CARS; ++ci) car_tick_store(s, (uint32_t)ci, car[ci], rb[ci]);
   if (w.boost_pads_enabled) boost_pads_tick(s, w);
-  s.ball.vel = ball.lin_vel * k::BT_TO_UU;  // ball finish_physics_tick
-  s.ball.ang_vel = ball.ang_vel;
-  s.ball.pos = ball.world.t * k::BT_TO_UU;
-  s.ball.rot = ball.world.m;
-  s.ball.tick_count_since_kickoff = u64w(u64(s.ball.tick_count_since_kickoff) + 1);
+  ball_finish_tick(s, ball);
   s.tick_count = u64w(u64(s.tick_count) + 1);
 }
 
@@ -429,17 +507,23 @@ RS_NOINL int run_phase_in(int kk, typename M::template Ptr<ArenaState> sp, const
   RS_UNIFORM_INDEX(kk);
   ArenaState& s = *(ArenaState*)sp;
   const StaticData& w = *(const StaticData*)wp;
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (M::SPLIT) {  // the phases that are not split run on the arena's first lane
+    const bool split = kk == 0 || kk == 1 || kk == 2 || kk == 7 || kk == 9;
+    if (!split && split_role() != 0) return PHASE_OK;
+  }
+#endif
   switch (kk) {
-    case 0: phase_p0(s, w); return PHASE_OK;
+    case 0: phase_p0<M>(s, w); return PHASE_OK;
     case 1: phase_p1<UW, M>(s, w); return PHASE_OK;
-    case 2: phase_p2(s, w); return PHASE_OK;
+    case 2: phase_p2<M>(s, w); return PHASE_OK;
     case 3: phase_p3a(s, w); return PHASE_OK;
     case 4: return phase_p3b<UW, M>(s, w) == 0 ? PHASE_OK : PHASE_UNIMPLEMENTED;
     case 5: phase_p4(s, w); return PHASE_OK;
     case 6: phase_p5(s, w); return PHASE_OK;
-    case 7: phase_p6(s, w); return PHASE_OK;
+    case 7: phase_p6<M>(s, w); return PHASE_OK;
     case 8: phase_p7(s, w); return PHASE_OK;
-    case 9: phase_p8(s, w); return PHASE_OK;
+    case 9: phase_p8<M>(s, w); return PHASE_OK;
     default: return PHASE_BAD_INDEX;
   }
 }

@@ -93,10 +93,10 @@ RS_FN void trav_walk(const StaticData& w, TravBatch& tb) {  // each job's own de
 }
 #if defined(__HIP_DEVICE_COMPILE__)
 // The pooled walk's LDS area (the wave's slices taken together): job records, per-job leaf counts and first slots, the
-// control words, two frontiers and the leaf list, for waves of ARENAS arenas.
-template <uint32_t ARENAS>
+// control words, two frontiers and the leaf list, for waves whose first WALKERS lanes bring walks.
+template <uint32_t WALKERS>
 struct PoolArea {
-  static constexpr uint32_t JOBS = ARENAS * TJ_MAX, Q = ARENAS == 64 ? 940 : 256, L = ARENAS == 64 ? 960 : 256;
+  static constexpr uint32_t JOBS = WALKERS * TJ_MAX, Q = WALKERS == 64 ? 940 : 232, L = WALKERS == 64 ? 960 : 232;
   static constexpr uint32_t REC = 10;  // a job record: box (6 words), the address of its mesh's first node (2), the mesh's node count
   static constexpr uint32_t JOB_W = 0, CNT_W = JOB_W + REC * JOBS, START_W = CNT_W + JOBS, CTRL_W = START_W + JOBS, Q_W = CTRL_W + 4,
                             L_W = Q_W + 4 * Q, WORDS = L_W + 2 * L;
@@ -105,9 +105,9 @@ static_assert(PoolArea<64>::WORDS <= WAVE_LDS_WORDS, "the pooled walk fits the w
 constexpr uint32_t PT_DEPTH = 15;
 __device__ inline uint32_t* wave_word(uint32_t j) { return wave_lds() + j; }
 
-template <uint32_t ARENAS>
+template <uint32_t WALKERS>
 __device__ inline bool trav_pooled(const StaticData& w, TravBatch& tb) {
-  using A = PoolArea<ARENAS>;
+  using A = PoolArea<WALKERS>;
   constexpr uint32_t PT_JOBS = A::JOBS, PT_Q = A::Q, PT_L = A::L, PT_REC = A::REC, PT_JOB_W = A::JOB_W, PT_CNT_W = A::CNT_W,
                      PT_START_W = A::START_W, PT_CTRL_W = A::CTRL_W, PT_L_W = A::L_W;
   auto pt_q = [](uint32_t which, uint32_t i, uint32_t k) { return wave_word(A::Q_W + which * 2 * A::Q + 2 * i + k); };
@@ -274,7 +274,7 @@ __device__ inline bool trav_pooled(const StaticData& w, TravBatch& tb) {
 template <class M>
 RS_FN void trav_run(const StaticData& w, TravBatch& tb) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  if (trav_pooled<M::ARENAS>(w, tb)) return;
+  if (trav_pooled<M::WALKERS>(w, tb)) return;
 #endif
   trav_walk(w, tb);
 }

@@ -6,9 +6,14 @@
 // per word however few lanes use it, so that spread-out waves would also crowd each other out of the caches). The lanes
 // past the wave's arenas help with the copies in and out, where each instruction moves 64 words of one arena.
 //
-// What bounds it: the tick's own instruction chain (about 25,000 instructions of one wave per tick at a kickoff) and its
-// remaining waits. Measured, ms per decision over four decisions, against one arena per lane in private memory: contact
-// mix 64 arenas 2.71 -> 1.53, 1,000 arenas 3.55 -> 2.23, 3,072 arenas 3.89 -> 2.96; kickoffs 1,024 arenas 1.26 -> 1.14.
+// An arena's two cars and its ball are lanes of their own in the phases that treat them alike (P0, P1, P2, P6, P8: SPLIT):
+// with the state in LDS another lane reaches it as well, and a phase that did three bodies or two cars in turn takes the
+// time of one. Ms per decision, one lane an arena -> split: kickoffs 1,024 arenas 1.01 -> 0.72 (P1 109K -> 68K cycles per
+// wave and tick); contact mix 64 arenas 1.36 -> 1.29, 1,000 arenas 2.05 -> 1.76.
+//
+// What bounds it: the tick's own instruction chain and its remaining waits, one wave a SIMD. When it was introduced, still
+// one lane an arena, ms per decision over four decisions against one arena per lane in private memory: contact mix 64
+// arenas 2.71 -> 1.53, 1,000 arenas 3.55 -> 2.23, 3,072 arenas 3.89 -> 2.96; kickoffs 1,024 arenas 1.26 -> 1.14.
 #include "device/launch.h"
 #include "device/aosoa.h"
 
@@ -16,9 +21,9 @@ namespace rs {
 namespace dev {
 
 // The wave's LDS: the stepper's lane slices and the pooled walks' area (which share the words from 0), then the states.
-constexpr uint32_t SMALL_SLICE_WORDS = InLds::ARENAS * (uint32_t)LANE_LDS_WORDS;
+constexpr uint32_t SMALL_SLICE_WORDS = InLds::ARENAS * InLds::ROLES * (uint32_t)LANE_LDS_WORDS;
 #if defined(__HIP_DEVICE_COMPILE__)
-static_assert(PoolArea<InLds::ARENAS>::WORDS <= 1728, "the pooled walk fits below the states");
+static_assert(PoolArea<InLds::WALKERS>::WORDS <= 1728, "the pooled walk fits below the states");
 #endif
 constexpr uint32_t SMALL_STATE_W = 1728;
 static_assert(SMALL_SLICE_WORDS <= SMALL_STATE_W && SMALL_STATE_W % 4 == 0, "the slices fit below the states");
@@ -60,13 +65,15 @@ __global__ void __launch_bounds__(64) k_small(Sim8Args p, uint32_t per_wave, uin
 #if defined(__HIP_DEVICE_COMPILE__)
   const uint32_t a0 = blockIdx.x * per_wave, lane = threadIdx.x;
   const uint32_t cnt = p.n - a0 < per_wave ? p.n - a0 : per_wave;
-  const uint32_t a = a0 + (lane < cnt ? lane : 0u);
+  // lane = arena + 3 * role: role 0 is the arena's own lane, the others take a body or car of their own (see SPLIT)
+  const bool part = lane < InLds::ARENAS * InLds::ROLES && split_arena() < cnt, mine = lane < cnt;
+  const uint32_t slot = part ? split_arena() : 0u, a = a0 + slot;
   const uint32_t v = p.variant ? p.variant[a] : 0u;
-  const bool bad = v >= p.nworlds, mine = lane < cnt;
+  const bool bad = v >= p.nworlds;
   const StaticData& w = p.worlds[bad ? 0u : v];
   for (uint32_t j = 0; j < cnt; ++j) small_load(j, p.buf, a0 + j);
   wave_lds_sync();
-  ArenaState& s = *(ArenaState*)(RS_LDS_AS ArenaState*)small_state(mine ? lane : 0u);
+  ArenaState& s = *(ArenaState*)(RS_LDS_AS ArenaState*)small_state(slot);
   for (uint32_t d = 0; d < decisions; ++d) {
     if (d > 0) {  // the mid-tick tail is clear at a decision's start, as the copy clears it
       for (uint32_t j = 0; j < cnt; ++j)
@@ -74,11 +81,12 @@ __global__ void __launch_bounds__(64) k_small(Sim8Args p, uint32_t per_wave, uin
       wave_lds_sync();
     }
     uint32_t word = 0u;
-    bool live = mine && !bad;
+    bool live = part && !bad;
     for (uint32_t t = 1; t <= TICKS_PER_DECISION; ++t) {  // run_decision, with the wave's copies out between the ticks
       if (live) {
         const Controls* c = p.ctl + ((size_t)d * p.n + a) * NUM_CARS;
-        for (int i = 0; i < NUM_CARS; ++i) s.cars[i].controls = c[i];
+        if (mine)
+          for (int i = 0; i < NUM_CARS; ++i) s.cars[i].controls = c[i];
         if (step_tick<UW, InLds>(s, w) != PHASE_OK) word |= SIM8_UNIMPLEMENTED;
       }
       const uint64_t stepped = __ballot(live);
