@@ -796,10 +796,14 @@ RS_INLINE void phase_p1(ArenaState& s, const StaticData& w) {
 #if defined(__HIP_DEVICE_COMPILE__)
   if constexpr (M::SPLIT) {
     const uint32_t arena = split_arena(), ci = split_role();
-    if (ci < (uint32_t)NUM_CARS) {
+    const bool mine = ci < (uint32_t)NUM_CARS;
+    bool dynamic = false;
+    if (mine) {
       car_flip_zdamp(s, w, (int)ci);
-      const bool dynamic = wheel_rays_collect(s, w, (int)ci, prep);
-      trav_run<M>(w, prep.tb);
+      dynamic = wheel_rays_collect(s, w, (int)ci, prep);
+    }
+    trav_run<M>(w, prep.tb);  // with every lane of the arena
+    if (mine) {
       const bool was = s.cars[ci].is_on_ground != 0;
       const uint64_t tied = __ballot(dynamic || s.cars[ci].is_demoed != 0);
       const bool in_order = ((tied >> arena | tied >> (arena + InLds::ARENAS)) & 1u) != 0;

@@ -822,6 +822,9 @@ RS_INLINE uint32_t phase_p3b_body(ArenaState& s, const StaticData& w) {
   const uint32_t n_records0 = s.n_records;
   Np c = {s, w, 0, nullptr, nullptr, 0u, n_records0};
   uint32_t n = s.n_pairs < (uint32_t)MAX_PAIRS ? s.n_pairs : (uint32_t)MAX_PAIRS;
+#if defined(__HIP_DEVICE_COMPILE__)
+  if (M::SPLIT && split_role() != 0) n = 0;  // the arena's own lane has its pairs, the others help with the pooled stages
+#endif
   TravBatch tb;
   tb.n_jobs = tb.n_leaves = tb.next = tb.leaves = 0;
   for (uint32_t i = 0; i < n && tb.n_jobs < (uint32_t)TJ_MAX; ++i) {  // the mesh jobs, in pair order

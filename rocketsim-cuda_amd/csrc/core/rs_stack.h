@@ -28,6 +28,8 @@ constexpr int SWEEP_WORDS = 3 * 24 + 64;
 constexpr int LANE_LDS_WORDS = SWEEP_WORDS | 1;
 static_assert(LANE_LDS_WORDS >= TRAV_LDS && LANE_LDS_WORDS >= BANK_WORDS, "every use fits the slice");
 constexpr uint32_t WAVE_LDS_WORDS = 64u * (uint32_t)LANE_LDS_WORDS;
+// The words that a stage pooled over all 64 lanes uses at most when the wave steps a few arenas (their states start here).
+constexpr uint32_t POOL_WORDS = 1728;
 RS_HD inline size_t trav_lds_bytes(uint32_t block) {
   return (size_t)WAVE_LDS_WORDS * ((block + 63u) / 64u) * sizeof(uint32_t);
 }
@@ -41,10 +43,10 @@ __device__ inline uint32_t* wave_lds() {
   const uint32_t byte = (threadIdx.x >> 6) * WAVE_LDS_WORDS * (uint32_t)sizeof(uint32_t);
   return (uint32_t*)(__attribute__((address_space(3))) uint32_t*)byte;
 }
-// Word k of this lane's slice, and word k of lane `slot`'s slice of the same wave.
+// Word k of this lane's slice.
 __device__ inline uint32_t* lane_word(uint32_t k) { return wave_lds() + ((threadIdx.x & 63u) * (uint32_t)LANE_LDS_WORDS + k); }
-__device__ inline uint32_t* wave_lane_word(uint32_t slot, uint32_t k) { return wave_lds() + (slot * (uint32_t)LANE_LDS_WORDS + k); }
-// The lane's arena of the wave and its part in it, where a state is split over lanes (SPLIT): lane = arena + 3 * role.
+// The lane's arena of the wave and its part in it, where a state is split over lanes (SPLIT): lane = arena + 3 * role. Role 0
+// is the arena's own lane, roles 0 to 2 take a body or car each, and every role of an arena takes part in pooled stages.
 __device__ inline uint32_t split_arena() { return (threadIdx.x & 63u) % InLds::ARENAS; }
 __device__ inline uint32_t split_role() { return (threadIdx.x & 63u) / InLds::ARENAS; }
 struct TravStack {
@@ -85,10 +87,10 @@ struct DeltaBank {
   __device__ float applied(int row) const { return *at((uint32_t)(BANK_BODIES * BANK_BODY_WORDS + row)); }
   __device__ void set_applied(int row, float v) { *at((uint32_t)(BANK_BODIES * BANK_BODY_WORDS + row)) = v; }
 };
-// Wave-wide staging through the same slices (the narrowphase's batched separating-axis tests, between the BVH walks): slot
-// r of a wave is the slice of the wave's lane r, so any lane of the wave can write or read any slot. LDS accesses of one
-// wave execute in order; the fences only keep the compiler from moving them across the hand-off points.
-__device__ inline float* wave_slot(uint32_t slot, uint32_t k) { return reinterpret_cast<float*>(wave_lane_word(slot, k)); }
+// Wave-wide staging through the same words (the narrowphase's batched separating-axis tests, between the BVH walks): slot
+// after slot from the first word on, so any lane of the wave can write or read any slot. LDS accesses of one wave execute
+// in order; the fences only keep the compiler from moving them across the hand-off points.
+__device__ inline float* wave_word_f(uint32_t j) { return reinterpret_cast<float*>(wave_lds() + j); }
 __device__ inline void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -100,7 +102,10 @@ __device__ inline void wave_lds_sync() {
 // from ballots (task order: lane order, then the owner's order); the records and results pass through the LDS slots.
 template <int REC, int OUT, int MAXT, class Stage, class Exec, class Collect>
 __device__ inline void wave_pool(uint32_t cnt, Stage stage, Exec exec, Collect collect) {
-  static_assert(OUT <= REC && REC <= LANE_LDS_WORDS, "a slot holds a record, then its result");
+  constexpr uint32_t STRIDE = REC | 1;  // odd: lanes reading the same word of their slots hit distinct banks
+  static_assert(OUT <= REC, "a slot holds a record, then its result");
+  static_assert(64u * STRIDE <= POOL_WORDS && POOL_WORDS <= WAVE_LDS_WORDS, "a full wave's slots fit the pooled words");
+  auto slot_word = [](uint32_t slot, int k) { return wave_word_f(slot * STRIDE + (uint32_t)k); };
   const uint32_t lane = threadIdx.x & 63u;
   const uint64_t below = lane ? (~0ull >> (64u - lane)) : 0ull;
   const uint64_t active = __ballot(1);
@@ -119,20 +124,20 @@ __device__ inline void wave_pool(uint32_t cnt, Stage stage, Exec exec, Collect c
     for (uint32_t t = lo; t < hi; ++t) {  // this lane's tasks in the window, into the slots their order gives
       stage(t, r);
       const uint32_t slot = pre + t - base;
-      for (int k = 0; k < REC; ++k) *wave_slot(slot, (uint32_t)k) = r[k];
+      for (int k = 0; k < REC; ++k) *slot_word(slot, k) = r[k];
     }
     wave_lds_sync();
     if (base + rank < total) {
-      for (int k = 0; k < REC; ++k) r[k] = *wave_slot(rank, (uint32_t)k);
+      for (int k = 0; k < REC; ++k) r[k] = *slot_word(rank, k);
       float o[OUT];
       exec(r, o);
-      for (int k = 0; k < OUT; ++k) *wave_slot(rank, (uint32_t)k) = o[k];
+      for (int k = 0; k < OUT; ++k) *slot_word(rank, k) = o[k];
     }
     wave_lds_sync();
     for (uint32_t t = lo; t < hi; ++t) {
       float o[OUT];
       const uint32_t slot = pre + t - base;
-      for (int k = 0; k < OUT; ++k) o[k] = *wave_slot(slot, (uint32_t)k);
+      for (int k = 0; k < OUT; ++k) o[k] = *slot_word(slot, k);
       collect(t, o);
     }
     wave_lds_sync();

@@ -508,9 +508,9 @@ RS_NOINL int run_phase_in(int kk, typename M::template Ptr<ArenaState> sp, const
   ArenaState& s = *(ArenaState*)sp;
   const StaticData& w = *(const StaticData*)wp;
 #if defined(__HIP_DEVICE_COMPILE__)
-  if constexpr (M::SPLIT) {  // the phases that are not split run on the arena's first lane
-    const bool split = kk == 0 || kk == 1 || kk == 2 || kk == 7 || kk == 9;
-    if (!split && split_role() != 0) return PHASE_OK;
+  if constexpr (M::SPLIT) {  // P1 and P3b pool stages over all lanes, P0, P2, P6 and P8 are split, the others whole
+    const uint32_t roles = kk == 1 || kk == 4 ? 64u : kk == 0 || kk == 2 || kk == 7 || kk == 9 ? M::ROLES : 1u;
+    if (split_role() >= roles) return PHASE_OK;
   }
 #endif
   switch (kk) {

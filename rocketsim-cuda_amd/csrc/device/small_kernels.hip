@@ -8,8 +8,10 @@
 //
 // An arena's two cars and its ball are lanes of their own in the phases that treat them alike (P0, P1, P2, P6, P8: SPLIT):
 // with the state in LDS another lane reaches it as well, and a phase that did three bodies or two cars in turn takes the
-// time of one. Ms per decision, one lane an arena -> split: kickoffs 1,024 arenas 1.01 -> 0.72 (P1 109K -> 68K cycles per
-// wave and tick); contact mix 64 arenas 1.36 -> 1.29, 1,000 arenas 2.05 -> 1.76.
+// time of one. The mesh walks and the batched separating-axis tests, whose work items any lane can take, are pooled over
+// every lane. Ms per decision, one lane an arena -> split -> split and pooled: kickoffs 1,024 arenas 1.01 -> 0.72 -> 0.66
+// (P1 109K -> 68K -> 64K cycles per wave and tick); contact mix 64 arenas 1.36 -> 1.29 -> 1.11, 1,000 arenas 2.05 -> 1.76 ->
+// 1.52 (P3b 77K -> 78K -> 66K).
 //
 // What bounds it: the tick's own instruction chain and its remaining waits, one wave a SIMD. When it was introduced, still
 // one lane an arena, ms per decision over four decisions against one arena per lane in private memory: contact mix 64
@@ -23,9 +25,9 @@ namespace dev {
 // The wave's LDS: the stepper's lane slices and the pooled walks' area (which share the words from 0), then the states.
 constexpr uint32_t SMALL_SLICE_WORDS = InLds::ARENAS * InLds::ROLES * (uint32_t)LANE_LDS_WORDS;
 #if defined(__HIP_DEVICE_COMPILE__)
-static_assert(PoolArea<InLds::WALKERS>::WORDS <= 1728, "the pooled walk fits below the states");
+static_assert(PoolArea<InLds::WALKERS>::WORDS <= POOL_WORDS, "the pooled walk fits below the states");
 #endif
-constexpr uint32_t SMALL_STATE_W = 1728;
+constexpr uint32_t SMALL_STATE_W = POOL_WORDS;
 static_assert(SMALL_SLICE_WORDS <= SMALL_STATE_W && SMALL_STATE_W % 4 == 0, "the slices fit below the states");
 static uint32_t small_lds_bytes(uint32_t per_wave) { return (SMALL_STATE_W + per_wave * (uint32_t)ARENA_WORDS) * 4u; }
 
@@ -65,8 +67,7 @@ __global__ void __launch_bounds__(64) k_small(Sim8Args p, uint32_t per_wave, uin
 #if defined(__HIP_DEVICE_COMPILE__)
   const uint32_t a0 = blockIdx.x * per_wave, lane = threadIdx.x;
   const uint32_t cnt = p.n - a0 < per_wave ? p.n - a0 : per_wave;
-  // lane = arena + 3 * role: role 0 is the arena's own lane, the others take a body or car of their own (see SPLIT)
-  const bool part = lane < InLds::ARENAS * InLds::ROLES && split_arena() < cnt, mine = lane < cnt;
+  const bool part = split_arena() < cnt, mine = lane < cnt;  // role 0 of an arena is its own lane
   const uint32_t slot = part ? split_arena() : 0u, a = a0 + slot;
   const uint32_t v = p.variant ? p.variant[a] : 0u;
   const bool bad = v >= p.nworlds;
@@ -113,8 +114,10 @@ __global__ void __launch_bounds__(64) k_small(Sim8Args p, uint32_t per_wave, uin
 
 // Arenas per wave: one while the waves fill at most two of a CU's four SIMDs, three (what a fourth of a CU's LDS holds)
 // above. Waves on one CU share its caches and instruction fetch, which from there on costs more than further arenas in the
-// wave (ms per decision with 1 / 2 / 3 per wave, contact mix: 256 arenas 1.80 / 1.87 / 2.01, 512 arenas 2.01 / 2.11 / 2.08,
-// 768 arenas 2.23 / 2.15 / 2.10, 1,536 arenas 3.09 / 2.46 / 2.44; kickoffs: 768 arenas 1.13 / 1.12 / 1.04).
+// wave (ms per decision with 1 / 2 / 3 per wave, contact mix: 256 arenas 1.23 / 1.29 / 1.38, 512 arenas 1.35 / 1.41 / 1.44,
+// 768 arenas 1.45 / 1.43 / 1.43, 1,536 arenas 1.97 / 1.61 / 1.59; kickoffs: 256 arenas 0.57 / 0.59 / 0.59, 768 arenas
+// 0.68 / 0.64 / 0.61). Past three on every SIMD a second round of waves follows: at 4,096 arenas contact mix takes 2.36 ms
+// here and 2.96 with the states in private memory, but kickoffs 1.42 and 1.07, and at 8,192 both are slower here.
 static uint32_t small_per_wave(uint32_t n) { return n <= 512 ? 1u : InLds::ARENAS; }
 hipError_t launch_small(hipStream_t st, const Sim8Args& p, uint32_t decisions) {
   const uint32_t per_wave = small_per_wave(p.n), lds = small_lds_bytes(per_wave);
