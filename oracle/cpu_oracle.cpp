@@ -226,7 +226,7 @@ uint64_t rsim_cpu_check_sweep(const StaticData* w, const uint32_t* state, uint64
         update_cells(a, *w, true, h, ni);
       }
     }
-    phase_p3a(b, *w);
+    phase_p3a<InPrivate>(b, *w);
     if (memcmp(&a, &b, sizeof a) != 0) ++bad;
   }
   return bad;

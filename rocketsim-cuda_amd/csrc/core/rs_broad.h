@@ -454,6 +454,41 @@ RS_FN bool edges_stay(const ArenaState& s, int ax, uint32_t mn, uint32_t mx, uin
   return valid && !min_down && !max_up && !min_up && !max_down;
 }
 
+// What a body's move is computed from, and its new box, edge positions (the min edge's low) and cell.
+struct SweptBody {
+  Aabb box;
+  HandleEdges he;
+  uint32_t q[3], cell;
+  uint32_t live, moved;
+};
+RS_FN SweptBody swept_body(const ArenaState& s, const StaticData& w, uint32_t d) {
+  const V3 cbt = splat(k::CONTACT_BREAKING_THRESHOLD);
+  const BodyConst& bc = w.bodies[w.dyn_body[d]];
+  const Body& b = s.bodies[d];
+  SweptBody o;
+  o.he = s.handle_edges[w.dyn_handle[d]];
+  const uint32_t old = s.dyn_proxy[d].cell_idx;
+  o.live = b.collision_flags & k::CF_STATIC ? 0u : 1u;
+  Aabb a = bc.shape_kind == k::SHAPE_SPHERE ? sphere_box(bc.sphere_margin, b.world.t) : compound_box(bc, b.world);
+  a.min -= cbt;
+  a.max += cbt;
+  Aabb a2 = bc.shape_kind == k::SHAPE_SPHERE ? sphere_box(bc.sphere_margin, b.interp_world.t) : compound_box(bc, b.interp_world);
+  a2.min -= cbt;
+  a2.max += cbt;
+  a.min = vmin(a.min, a2.min);
+  a.max = vmax(a.max, a2.max);
+  o.box = a;
+  uint16_t qmin[3], qmax[3];
+  sap_quantize(w, a.min, 0, qmin);
+  sap_quantize(w, a.max, 1, qmax);
+  RS_UNROLL
+  for (int ax = 0; ax < 3; ++ax) o.q[ax] = (uint32_t)qmax[ax] << 16 | qmin[ax];
+  uint32_t ni[3];
+  cell_indices(w, a.min, ni);
+  o.cell = cell_index(w, ni);
+  o.moved = o.live != 0 && o.cell != old ? 1u : 0u;
+  return o;
+}
 // P3a (collision_world.cuh:34-50, grid_broadphase.cuh:68-84): the dynamic bodies' swept boxes (current and predicted
 // transform, each grown by the contact breaking threshold) into the broadphase.
 // Of a body's axis updates about one in twenty moves an edge past another; the rest only write positions. So the updates
@@ -465,60 +500,54 @@ RS_FN bool edges_stay(const ArenaState& s, int ax, uint32_t mn, uint32_t mx, uin
 // sorts (whose overlap tests read edge indices); and a body's sorts and its cell list share no data, so the cell moves
 // come last, again each lane its own. With every update copying its axis in and out, P3a took 183K cycles per wave and
 // tick of contact play at 65,536 arenas, 91K at kickoff and 38K for one arena a wave in LDS; now 140K, 82K and 23K.
+template <class M>
 RS_INLINE void phase_p3a(ArenaState& s, const StaticData& w) {
-  const V3 cbt = splat(k::CONTACT_BREAKING_THRESHOLD);
   // everything that the bodies' moves are computed from, read together before the first store
-  uint32_t put_off = 0, moved = 0, live = 0;  // bit 3 d + axis; bit d
-  uint32_t q[3 * NUM_DYN];                    // new positions, the min edge's low
-  Aabb box[NUM_DYN];
-  HandleEdges he[NUM_DYN];
-  uint32_t cell[NUM_DYN];
-  RS_UNROLL
-  for (uint32_t d = 0; d < (uint32_t)NUM_DYN; ++d) {
-    const BodyConst& bc = w.bodies[w.dyn_body[d]];
-    const Body& b = s.bodies[d];
-    he[d] = s.handle_edges[w.dyn_handle[d]];
-    cell[d] = s.dyn_proxy[d].cell_idx;
-    if (!(b.collision_flags & k::CF_STATIC)) live |= 1u << d;
-    Aabb a = bc.shape_kind == k::SHAPE_SPHERE ? sphere_box(bc.sphere_margin, b.world.t) : compound_box(bc, b.world);
-    a.min -= cbt;
-    a.max += cbt;
-    Aabb a2 = bc.shape_kind == k::SHAPE_SPHERE ? sphere_box(bc.sphere_margin, b.interp_world.t) : compound_box(bc, b.interp_world);
-    a2.min -= cbt;
-    a2.max += cbt;
-    a.min = vmin(a.min, a2.min);
-    a.max = vmax(a.max, a2.max);
-    box[d] = a;
-    uint16_t qmin[3], qmax[3];
-    sap_quantize(w, a.min, 0, qmin);
-    sap_quantize(w, a.max, 1, qmax);
+  uint32_t put_off = 0, moved = 0;  // bit 3 d + axis; bit d
+  SweptBody b[NUM_DYN];
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (M::SPLIT) {  // a body a lane, handed to the arena's own lane through the lanes' slices
+    constexpr uint32_t WORDS = sizeof(SweptBody) / 4u;
+    static_assert(WORDS * NUM_DYN <= (uint32_t)LANE_LDS_WORDS, "the slice holds the arena's bodies");
+    const SweptBody own = swept_body(s, w, split_role());
+    const uint32_t first = split_arena() * (uint32_t)LANE_LDS_WORDS;
+    uint32_t v[WORDS];
+    __builtin_memcpy(v, &own, sizeof own);
+    for (uint32_t i = 0; i < WORDS; ++i) wave_lds()[first + split_role() * WORDS + i] = v[i];
+    wave_lds_sync();
+    if (split_role() != 0) return;
     RS_UNROLL
-    for (int ax = 0; ax < 3; ++ax) q[3 * d + ax] = (uint32_t)qmax[ax] << 16 | qmin[ax];
-    uint32_t ni[3];
-    cell_indices(w, a.min, ni);
-    const uint32_t nidx = cell_index(w, ni);
-    if (nidx != cell[d]) moved |= 1u << d;
-    cell[d] = nidx;
+    for (uint32_t d = 0; d < (uint32_t)NUM_DYN; ++d) {
+      RS_UNROLL
+      for (uint32_t i = 0; i < WORDS; ++i) v[i] = wave_lds()[first + d * WORDS + i];
+      __builtin_memcpy(&b[d], v, sizeof own);
+    }
+    wave_lds_sync();
   }
-  moved &= live;
+#endif
+  if constexpr (!M::SPLIT) {
+    RS_UNROLL
+    for (uint32_t d = 0; d < (uint32_t)NUM_DYN; ++d) b[d] = swept_body(s, w, d);
+  }
   RS_UNROLL
   for (uint32_t d = 0; d < (uint32_t)NUM_DYN; ++d) {
-    if (!(live & (1u << d))) continue;
+    moved |= b[d].moved << d;
+    if (!b[d].live) continue;
     bool stay[3], same[3];
     RS_UNROLL
     for (int ax = 0; ax < 3; ++ax)
-      stay[ax] = edges_stay(s, ax, he[d].min[ax], he[d].max[ax], (uint16_t)q[3 * d + ax], (uint16_t)(q[3 * d + ax] >> 16), &same[ax]);
+      stay[ax] = edges_stay(s, ax, b[d].he.min[ax], b[d].he.max[ax], (uint16_t)b[d].q[ax], (uint16_t)(b[d].q[ax] >> 16), &same[ax]);
     RS_UNROLL
     for (int ax = 0; ax < 3; ++ax) {
       if (put_off & (0x49u << ax) || !stay[ax]) {
         put_off |= 1u << (3 * d + ax);
       } else if (!same[ax]) {
-        s.edges[ax][he[d].min[ax]].pos = (uint16_t)q[3 * d + ax];
-        s.edges[ax][he[d].max[ax]].pos = (uint16_t)(q[3 * d + ax] >> 16);
+        s.edges[ax][b[d].he.min[ax]].pos = (uint16_t)b[d].q[ax];
+        s.edges[ax][b[d].he.max[ax]].pos = (uint16_t)(b[d].q[ax] >> 16);
       }
     }
-    s.dyn_proxy[d].aabb = box[d];
-    if (moved & (1u << d)) s.dyn_proxy[d].cell_idx = cell[d];
+    s.dyn_proxy[d].aabb = b[d].box;
+    if (b[d].moved) s.dyn_proxy[d].cell_idx = b[d].cell;
   }
   if (put_off) {
     SapCopy c;
@@ -526,9 +555,9 @@ RS_INLINE void phase_p3a(ArenaState& s, const StaticData& w) {
     do {
       const int o = __builtin_ctz(put_off), d = o >= 6 ? 2 : o >= 3 ? 1 : 0;
       put_off &= put_off - 1;
-      uint32_t qo = q[0];
+      uint32_t qo = b[0].q[0];
       RS_UNROLL
-      for (int i = 1; i < 3 * NUM_DYN; ++i) qo = i == o ? q[i] : qo;
+      for (int i = 1; i < 3 * NUM_DYN; ++i) qo = i == o ? b[i / 3].q[i % 3] : qo;
       update_axis(s, w, c, o - 3 * d, w.dyn_handle[d], (uint16_t)qo, (uint16_t)(qo >> 16));
     } while (put_off);
     sap_copy_out(s, c);

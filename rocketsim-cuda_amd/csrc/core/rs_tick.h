@@ -343,14 +343,53 @@ RS_FN int pad_winner(const ArenaState& s, int pad, float mx) {
 // The steps and their order are the reference's; the pad lists are read together (one bit per pad with a touching car),
 // a list is written back only when it changed, the discovery screen is one mask over the pads' boxes, and the winner is
 // computed for the (at most NUM_CARS) pads a car touches rather than for all 34: the same reads decide the same writes.
+// Where a state is split over lanes, the two passes over all pads take one pad a lane and the masks come from ballots.
+struct PadScreens {
+  uint64_t listed, in_boxes[NUM_CARS];  // pads with a touching car; pads whose box holds the car's position
+};
+#if defined(__HIP_DEVICE_COMPILE__)
+__device__ inline PadScreens pad_screens_split(const ArenaState& s, const StaticData& w) {
+  constexpr uint32_t ROUND = 64u / InLds::ARENAS;  // roles that every arena has
+  const uint32_t arena = split_arena(), role = split_role();
+  const V3 pos[NUM_CARS] = {s.cars[0].pos, s.cars[1].pos};
+  PadScreens o = {};
+  for (uint32_t p0 = 0; p0 < (uint32_t)NUM_PADS; p0 += ROUND) {
+    const bool mine = role < ROUND && p0 + role < (uint32_t)NUM_PADS;
+    const uint32_t i = mine ? p0 + role : 0u;
+    const Aabb b = w.pads[i].aabb;
+    // pad p0 + r of this arena is bit arena + 3 r; the few that are set are moved to bit p0 + r
+    auto pads = [&](bool set) {
+      uint64_t m = __ballot(mine && set) >> arena, out = 0;
+      for (m &= 0x9249249249249249ull; m != 0; m &= m - 1) out |= 1ull << (p0 + (uint32_t)__builtin_ctzll(m) / InLds::ARENAS);
+      return out;
+    };
+    o.listed |= pads(s.pad_touching[i].n != 0u);
+    for (int ci = 0; ci < NUM_CARS; ++ci) o.in_boxes[ci] |= pads(all3(cmple(b.min, pos[ci])) && all3(cmpge(b.max, pos[ci])));
+  }
+  return o;
+}
+#endif
+template <class M>
 RS_FN void boost_pads_tick(ArenaState& s, const StaticData& w) {  // boost_pad_grid.cuh:56-133
   static_assert(NUM_PADS <= 64, "one bit per pad");
+#if defined(__HIP_DEVICE_COMPILE__)
+  PadScreens screens = {};
+  if constexpr (M::SPLIT) {
+    screens = pad_screens_split(s, w);
+    if (split_role() != 0) return;
+  }
+#endif
   const float mx = w.mut_f[MF_CAR_MAX_BOOST_AMOUNT];
   int touching[NUM_CARS];
   for (int ci = 0; ci < NUM_CARS; ++ci) touching[ci] = -1;
   uint64_t listed_pads = 0;
-  RS_UNROLL
-  for (int i = 0; i < NUM_PADS; ++i) listed_pads |= (uint64_t)(s.pad_touching[i].n != 0u) << i;
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (M::SPLIT) listed_pads = screens.listed;
+#endif
+  if constexpr (!M::SPLIT) {
+    RS_UNROLL
+    for (int i = 0; i < NUM_PADS; ++i) listed_pads |= (uint64_t)(s.pad_touching[i].n != 0u) << i;
+  }
   for (uint64_t m = listed_pads; m != 0; m &= m - 1) {  // retention, pad order (a pad with no car keeps nothing)
     const int i = __builtin_ctzll(m);
     const PadConst& pad = w.pads[i];
@@ -380,7 +419,11 @@ RS_FN void boost_pads_tick(ArenaState& s, const StaticData& w) {  // boost_pad_g
     look[ci] = !(car.is_demoed || car.pos.z > w.max_pad_z || touching[ci] >= 0);
   }
   uint64_t in_boxes[NUM_CARS] = {};
-  if (look[0] || look[1]) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (M::SPLIT)
+    for (int ci = 0; ci < NUM_CARS; ++ci) in_boxes[ci] = screens.in_boxes[ci];
+#endif
+  if (!M::SPLIT && (look[0] || look[1])) {
     static_assert(NUM_CARS == 2, "the screens test two cars");
     RS_UNROLL
     for (int i = 0; i < NUM_PADS; ++i) {
@@ -459,7 +502,7 @@ RS_INLINE void phase_p8(ArenaState& s, const StaticData& w) {
     const uint32_t d = split_role();
     if (d == 0) {
       ball_finish_tick(s, s.bodies[0]);
-    } else {
+    } else if (d < M::ROLES) {
       Car car = s.cars[d - 1];
       Body rb = s.bodies[d];
       car_post_tick(car, rb);
@@ -467,10 +510,8 @@ RS_INLINE void phase_p8(ArenaState& s, const StaticData& w) {
       car_tick_store(s, d - 1, car, rb);
     }
     wave_lds_sync();
-    if (d == 0) {
-      if (w.boost_pads_enabled) boost_pads_tick(s, w);
-      s.tick_count = u64w(u64(s.tick_count) + 1);
-    }
+    if (w.boost_pads_enabled) boost_pads_tick<M>(s, w);
+    if (d == 0) s.tick_count = u64w(u64(s.tick_count) + 1);
     return;
   }
 #endif
@@ -489,7 +530,7 @@ RS_INLINE void phase_p8(ArenaState& s, const StaticData& w) {
   }
   RS_UNROLL
   for (int ci = 0; ci < NUM_CARS; ++ci) car_tick_store(s, (uint32_t)ci, car[ci], rb[ci]);
-  if (w.boost_pads_enabled) boost_pads_tick(s, w);
+  if (w.boost_pads_enabled) boost_pads_tick<M>(s, w);
   ball_finish_tick(s, ball);
   s.tick_count = u64w(u64(s.tick_count) + 1);
 }
@@ -508,8 +549,8 @@ RS_NOINL int run_phase_in(int kk, typename M::template Ptr<ArenaState> sp, const
   ArenaState& s = *(ArenaState*)sp;
   const StaticData& w = *(const StaticData*)wp;
 #if defined(__HIP_DEVICE_COMPILE__)
-  if constexpr (M::SPLIT) {  // P1 and P3b pool stages over all lanes, P0, P2, P6 and P8 are split, the others whole
-    const uint32_t roles = kk == 1 || kk == 4 ? 64u : kk == 0 || kk == 2 || kk == 7 || kk == 9 ? M::ROLES : 1u;
+  if constexpr (M::SPLIT) {  // P1, P3b and P8 have work for all lanes, P0, P2, P3a and P6 are split, the others whole
+    const uint32_t roles = kk == 1 || kk == 4 || kk == 9 ? 64u : kk == 0 || kk == 2 || kk == 3 || kk == 7 ? M::ROLES : 1u;
     if (split_role() >= roles) return PHASE_OK;
   }
 #endif
@@ -517,7 +558,7 @@ RS_NOINL int run_phase_in(int kk, typename M::template Ptr<ArenaState> sp, const
     case 0: phase_p0<M>(s, w); return PHASE_OK;
     case 1: phase_p1<UW, M>(s, w); return PHASE_OK;
     case 2: phase_p2<M>(s, w); return PHASE_OK;
-    case 3: phase_p3a(s, w); return PHASE_OK;
+    case 3: phase_p3a<M>(s, w); return PHASE_OK;
     case 4: return phase_p3b<UW, M>(s, w) == 0 ? PHASE_OK : PHASE_UNIMPLEMENTED;
     case 5: phase_p4(s, w); return PHASE_OK;
     case 6: phase_p5(s, w); return PHASE_OK;

@@ -6,12 +6,13 @@
 // per word however few lanes use it, so that spread-out waves would also crowd each other out of the caches). The lanes
 // past the wave's arenas help with the copies in and out, where each instruction moves 64 words of one arena.
 //
-// An arena's two cars and its ball are lanes of their own in the phases that treat them alike (P0, P1, P2, P6, P8: SPLIT):
-// with the state in LDS another lane reaches it as well, and a phase that did three bodies or two cars in turn takes the
-// time of one. The mesh walks and the batched separating-axis tests, whose work items any lane can take, are pooled over
-// every lane. Ms per decision, one lane an arena -> split -> split and pooled: kickoffs 1,024 arenas 1.01 -> 0.72 -> 0.66
-// (P1 109K -> 68K -> 64K cycles per wave and tick); contact mix 64 arenas 1.36 -> 1.29 -> 1.11, 1,000 arenas 2.05 -> 1.76 ->
-// 1.52 (P3b 77K -> 78K -> 66K).
+// An arena's two cars and its ball are lanes of their own in the phases that treat them alike (P0, P1, P2, P6, P8 and the
+// swept boxes of P3a: SPLIT): with the state in LDS another lane reaches it as well, and a phase that did three bodies or two
+// cars in turn takes the time of one. The mesh walks, the batched separating-axis tests and the passes over all boost pads,
+// whose work items any lane can take, are spread over every lane. Ms per decision, one lane an arena -> bodies and cars
+// split -> walks and tests over all lanes -> boxes and pads too: kickoffs 1,024 arenas 1.01 -> 0.72 -> 0.66 -> 0.61 (P1 109K ->
+// 64K cycles per wave and tick); contact mix 64 arenas 1.36 -> 1.29 -> 1.11 -> 1.07, 1,000 arenas 2.05 -> 1.76 -> 1.52 ->
+// 1.47.
 //
 // What bounds it: the tick's own instruction chain and its remaining waits, one wave a SIMD. When it was introduced, still
 // one lane an arena, ms per decision over four decisions against one arena per lane in private memory: contact mix 64
