@@ -21,13 +21,16 @@ constexpr int BANK_WORDS = BANK_BODIES * BANK_BODY_WORDS + BANK_ROWS;
 constexpr int SWEEP_WORDS = 3 * 24 + 64;
 // All three live in the same per-lane LDS slice: each is used in a phase of its own (the walks in P1 and P3b, the sweep in
 // P3a, the bank in P5). Each wave of the work-group owns 64 slices, lane-major: word k of lane l of wave v is at
-// (v * 64 + l) * LANE_LDS_WORDS + k. The slice is an odd number of words, so lanes reading the same k hit distinct banks,
+// v * WAVE_LDS_WORDS + l * LANE_LDS_WORDS + k. The slice is an odd number of words, so lanes reading the same k hit distinct banks,
 // and a wave that steps only a few arenas needs only as many slices. The layout does not depend on the work-group size (a
 // kernel allocates whole waves), so the device functions never read it: they need no dispatch-packet pointer, which every
 // call would otherwise carry.
 constexpr int LANE_LDS_WORDS = SWEEP_WORDS | 1;
 static_assert(LANE_LDS_WORDS >= TRAV_LDS && LANE_LDS_WORDS >= BANK_WORDS, "every use fits the slice");
-constexpr uint32_t WAVE_LDS_WORDS = 64u * (uint32_t)LANE_LDS_WORDS;
+// A wave's LDS: its 64 slices, and the words past them that the pooled walk uses too (rs_trav.h). A quarter of a CU's 160 KB
+// (10,240 words) is the most: four waves a CU.
+constexpr uint32_t WAVE_LDS_WORDS = 9232;
+static_assert(64u * (uint32_t)LANE_LDS_WORDS <= WAVE_LDS_WORDS && WAVE_LDS_WORDS <= 10240, "the slices fit, and four waves a CU");
 // The words that a stage pooled over all 64 lanes uses at most when the wave steps a few arenas (their states start here).
 constexpr uint32_t POOL_WORDS = 1728;
 RS_HD inline size_t trav_lds_bytes(uint32_t block) {

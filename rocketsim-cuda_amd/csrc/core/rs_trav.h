@@ -92,16 +92,17 @@ RS_FN void trav_walk(const StaticData& w, TravBatch& tb) {  // each job's own de
   }
 }
 #if defined(__HIP_DEVICE_COMPILE__)
-// The pooled walk's LDS area (the wave's slices taken together): job records, per-job leaf counts and first slots, the
+// The pooled walk's LDS area (the wave's slices and the words past them): job records, per-job leaf counts and first slots, the
 // control words, two frontiers and the leaf list, for waves whose first WALKERS lanes bring walks.
 template <uint32_t WALKERS>
 struct PoolArea {
-  static constexpr uint32_t JOBS = WALKERS * TJ_MAX, Q = WALKERS == 64 ? 940 : 232, L = WALKERS == 64 ? 960 : 232;
+  static constexpr uint32_t JOBS = WALKERS * TJ_MAX, Q = WALKERS == 64 ? 1024 : 232, L = Q;
   static constexpr uint32_t REC = 10;  // a job record: box (6 words), the address of its mesh's first node (2), the mesh's node count
   static constexpr uint32_t JOB_W = 0, CNT_W = JOB_W + REC * JOBS, START_W = CNT_W + JOBS, CTRL_W = START_W + JOBS, Q_W = CTRL_W + 4,
                             L_W = Q_W + 4 * Q, WORDS = L_W + 2 * L;
+  static_assert(L <= Q, "the leaves are sorted in the frontiers' space");
 };
-static_assert(PoolArea<64>::WORDS <= WAVE_LDS_WORDS, "the pooled walk fits the wave's LDS slices");
+static_assert(PoolArea<64>::WORDS <= WAVE_LDS_WORDS, "the pooled walk fits the wave's LDS");
 constexpr uint32_t PT_DEPTH = 15;
 __device__ inline uint32_t* wave_word(uint32_t j) { return wave_lds() + j; }
 

@@ -100,3 +100,18 @@ def test_states_to_the_device_and_back(rsim, device, n):
     words = device.download_words(d)
     assert np.array_equal(words, rsim.aosoa_pack(states))
     assert np.array_equal(device.download_states(d), rsim.aosoa_unpack(words, n))
+
+
+@pytest.mark.parametrize("block", [64, 128, 256])
+def test_full_waves_of_one_arena(rsim, oracle, world, device, dev_world, block):
+    """256 contact arenas, each in all 64 lanes of a wave of its own: every lane brings the same walks, so some waves fill the
+    pooled walk's queues to their last slots and some past them (a wave of 15 leaves a lane has 960)."""
+    print("[case] waves of one arena, block %d" % block, flush=True)
+    k, copies = 256, 256 if block == 64 else 64  # at block 64, enough arenas for full waves
+    states = rsim.sample_arenas(world, rsim.SCEN_CONTACT, 5, k)
+    d, r = device.upload_states(np.repeat(states, copies, axis=0)), device.alloc_words(copies * k)
+    for decision in range(4):
+        ctl = rsim.sample_controls(9, decision, k)
+        device.sim8(d, dev_world, device.upload_controls(np.repeat(ctl, copies, axis=0)), r, block=block)
+        assert np.array_equal(device.read_words(r), np.repeat(oracle.sim8(states, world, ctl, threads=8), copies)), decision
+    same(device.download_states(d), np.repeat(states, copies, axis=0), "waves of one arena, block %d" % block)
