@@ -119,17 +119,29 @@ void unpack(const uint32_t* in, uint32_t n, ArenaState* states) {
 }
 
 // The staging buffer of state uploads and downloads: allocated by the first such call, sized to the largest batch seen up
-// to STAGE_ARENAS (65 MB), freed with the device. Every call that uses it ends synchronised, so it is never in use here.
+// to STAGE_ARENAS (65 MB), freed with the device; where the device has no room for that, as much as it has, down to one
+// block. Every call that uses it ends synchronised, so it is never in use here.
 constexpr uint32_t STAGE_ARENAS = 6144;
 int ensure_stage(rsim_device* dev, uint32_t n) {
-  const uint32_t want = n < STAGE_ARENAS ? n : STAGE_ARENAS;
+  uint32_t want = n < STAGE_ARENAS ? n : STAGE_ARENAS;
   if (dev->stage_cap >= want) return RSIM_OK;
   if (dev->stage) (void)hipFree(dev->stage);
   dev->stage = nullptr;
   dev->stage_cap = 0;
-  RSIM_HIP(hipMalloc((void**)&dev->stage, (size_t)want * sizeof(ArenaState)), "hipMalloc(stage)");
+  hipError_t e;
+  while ((e = hipMalloc((void**)&dev->stage, (size_t)want * sizeof(ArenaState))) == hipErrorOutOfMemory && want > rs::dev::AOSOA_LANES) {
+    (void)hipGetLastError();  // tried again smaller
+    want = want / 2 > rs::dev::AOSOA_LANES ? want / 2 / rs::dev::AOSOA_LANES * rs::dev::AOSOA_LANES : rs::dev::AOSOA_LANES;
+  }
+  RSIM_HIP(e, "hipMalloc(stage)");
   dev->stage_cap = want;
   return RSIM_OK;
+}
+
+// Arenas staged at a time for a batch of n: all of them, or whole blocks.
+uint32_t stage_step(const rsim_device* dev, uint32_t n) {
+  const uint32_t cap = dev->stage_cap < STAGE_ARENAS ? dev->stage_cap : STAGE_ARENAS;
+  return n <= cap ? n : cap / rs::dev::AOSOA_LANES * rs::dev::AOSOA_LANES;
 }
 
 int ensure_status(rsim_device* dev, uint32_t n) {
@@ -312,8 +324,9 @@ int rsim_write_states(rsim_device* dev, rsim_states* dst, const void* states) {
   if (!dst->n) return RSIM_OK;
   if ((rc = ensure_stage(dev, dst->n))) return rc;
   const ArenaState* src = static_cast<const ArenaState*>(states);
-  for (uint32_t a = 0; a < dst->n; a += STAGE_ARENAS) {  // whole blocks but for the last, packed on the device
-    const uint32_t m = dst->n - a < STAGE_ARENAS ? dst->n - a : STAGE_ARENAS;
+  const uint32_t step = stage_step(dev, dst->n);
+  for (uint32_t a = 0; a < dst->n; a += step) {  // whole blocks but for the last, packed on the device
+    const uint32_t m = dst->n - a < step ? dst->n - a : step;
     RSIM_HIP(hipMemcpyAsync(dev->stage, src + a, (size_t)m * sizeof(ArenaState), hipMemcpyHostToDevice, dev->stream), "state upload");
     RSIM_HIP(rs::dev::launch_pack_states(dev->stream, dev->stage, dst->d + rs::dev::aosoa_index(a, 0), m), "state upload");
   }
@@ -367,8 +380,9 @@ int rsim_download_states(rsim_device* dev, const rsim_states* s, void* out) {
   if (!s->n) return RSIM_OK;
   if ((rc = ensure_stage(dev, s->n))) return rc;
   ArenaState* dst = static_cast<ArenaState*>(out);
-  for (uint32_t a = 0; a < s->n; a += STAGE_ARENAS) {
-    const uint32_t m = s->n - a < STAGE_ARENAS ? s->n - a : STAGE_ARENAS;
+  const uint32_t step = stage_step(dev, s->n);
+  for (uint32_t a = 0; a < s->n; a += step) {
+    const uint32_t m = s->n - a < step ? s->n - a : step;
     RSIM_HIP(rs::dev::launch_unpack_states(dev->stream, s->d + rs::dev::aosoa_index(a, 0), dev->stage, m), "state download");
     RSIM_HIP(hipMemcpyAsync(dst + a, dev->stage, (size_t)m * sizeof(ArenaState), hipMemcpyDeviceToHost, dev->stream), "state download");
   }
