@@ -259,8 +259,10 @@ hipError_t launch_step_tick(hipStream_t st, uint32_t* buf, const StaticData* w, 
 // The lanes of a work-group that asks for SIM8_BLOCK, the production size: one wave, of fewer arenas where the batch leaves
 // SIMDs idle, since a wave pays for the union of its arenas' paths. 32 lanes as long as they fill at most one wave per
 // SIMD; fewer lose more to the half-empty rows of private memory that crowd the caches than their shorter unions gain
-// (ms per decision at 16 / 32 / 64 lanes, contact mix: 4,096 arenas 3.26 / 3.55 / 4.07, 16,384 arenas 4.54 / 4.02 / 4.44,
-// 32,768 arenas 8.43 / 4.91 / 5.18; kickoffs: 3,500 arenas 1.47 / 1.33 / 1.35, 16,384 arenas 2.04 / 1.64 / 1.63). Any
+// (ms per decision at 16 / 32 lanes, contact mix: 4,096 arenas 2.75 / 2.96, 8,192 arenas 3.15 / 3.13, 16,384 arenas 3.66 /
+// 3.36, 32,768 arenas 6.67 / 4.06; kickoffs: 4,096 arenas 1.11 / 1.07, 16,384 arenas 1.50 / 1.25; with an earlier tick, at 32 /
+// 64 lanes, contact mix: 4,096 arenas 3.55 / 4.07, 16,384 arenas 4.02 / 4.44, 32,768 arenas 4.91 / 5.18; kickoffs: 3,500
+// arenas 1.33 / 1.35, 16,384 arenas 1.64 / 1.63). Any
 // other size is the caller's own choice.
 static uint32_t wave_lanes(uint32_t n, uint32_t block) { return block == SIM8_BLOCK && n <= SPREAD_MAX_N ? 32u : block; }
 hipError_t launch_run(hipStream_t st, const Sim8Args& p, uint32_t decisions, uint32_t block) {
