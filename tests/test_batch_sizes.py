@@ -8,6 +8,7 @@ import pytest
 import forced_cases as fc
 from conftest import first_diff
 from helpers import TICK_WORDS
+from rsim import layout
 
 pytestmark = pytest.mark.gpu
 
@@ -115,3 +116,41 @@ def test_full_waves_of_one_arena(rsim, oracle, world, device, dev_world, block):
         device.sim8(d, dev_world, device.upload_controls(np.repeat(ctl, copies, axis=0)), r, block=block)
         assert np.array_equal(device.read_words(r), np.repeat(oracle.sim8(states, world, ctl, threads=8), copies)), decision
     same(device.download_states(d), np.repeat(states, copies, axis=0), "waves of one arena, block %d" % block)
+
+
+@pytest.mark.parametrize("n", [3, 64, 700])
+def test_cars_tied_to_each_other(rsim, oracle, world, device, dev_world, n):
+    """A small batch gives each car a lane of its own; cars whose updates touch shared state take turns. Arena by arena:
+    both cars demoed and due in the same tick (they draw from one random state), the second car standing on the first
+    (its wheels push it), the first car standing on the ball, and a plain kickoff beside them in the same wave."""
+    print("[case] tied cars, %d arenas" % n, flush=True)
+    states = rsim.sample_arenas(world, rsim.SCEN_KICKOFF, 77, n)
+    a = layout.arena_view(states)
+    for i in range(n):
+        kind, cars, bodies = i % 4, a["cars"][i], a["bodies"][i]
+        if kind == 0:
+            cars["is_demoed"][:] = 1
+            cars["demo_respawn_timer"][:] = np.float32((1 + i % 7) / 120.0)
+            continue
+        if kind == 3:
+            continue
+        below = {f: float(cars[0]["pos"][f]) for f in "xyz"}  # kind 1: the second car over the first
+        if kind == 2:  # the first car over the ball
+            fc.place_ball(a, i, (below["x"], below["y"], 93.0), (0, 0, 0))
+            below["z"] = 93.0 + 91.0
+        top = 1 if kind == 1 else 0
+        for f in "xyz":
+            x = np.float32(below[f] + (40.0 if f == "z" else 0.0))
+            cars[top]["pos"][f] = x
+            for t in ("world_trans", "interp_world_trans"):
+                bodies[1 + top][t]["translation"][f] = x * fc.UU_TO_BT
+    d, r = device.upload_states(states), device.alloc_words(n)
+    stood = np.zeros(n, bool)
+    for k in range(3):
+        ctl = rsim.sample_controls(78, k, n)
+        device.sim8(d, dev_world, device.upload_controls(ctl), r)
+        assert np.array_equal(device.read_words(r), oracle.sim8(states, world, ctl, threads=8)), k
+        ray = a["cars"]["wheels"]["raycast_info"]
+        stood |= ((ray["some"] != 0) & (ray["v"]["ground_stick"]["some"] != 0)).any((1, 2))
+    assert stood[1::4].any() and (n < 4 or stood[2::4].any()), "some wheels stood on a car, some on the ball"
+    same(device.download_states(d), states, "tied cars %d" % n)
