@@ -353,11 +353,11 @@ __global__ void __launch_bounds__(256) k_scatter_words(const uint32_t* __restric
 }
 // AoSoA-64 states: arena i of dst (n arenas) = arena perm[i] of src (n_src arenas); an index past src leaves that arena of
 // dst as it was. The grid walks the words, so all arenas of one word are copied together and the source lines they share
-// are read from HBM once; word w's work-groups are all w % 8 modulo 8, on one XCD and its L2.
+// are read from HBM once; word w's work-groups are all w % 8 modulo 8, on one XCD and its L2. Eight words in x, their eights
+// in y: a launch takes fewer than 2^32 work-items in x, which one dimension for all words would pass at 1,542,657 arenas.
 __global__ void __launch_bounds__(256) k_gather_states(const uint32_t* __restrict__ src, uint32_t n_src,
                                                        const uint32_t* __restrict__ perm, uint32_t* __restrict__ dst, uint32_t n) {
-  const uint32_t groups = (n + 255u) / 256u, q = blockIdx.x / 8u;
-  const uint32_t w = q / groups * 8u + blockIdx.x % 8u, i = q % groups * 256u + threadIdx.x;
+  const uint32_t w = blockIdx.y * 8u + blockIdx.x % 8u, i = blockIdx.x / 8u * 256u + threadIdx.x;
   if (i >= n || w >= (uint32_t)ARENA_WORDS) return;
   uint32_t a = perm[i];
   if (a < n_src) dst[aosoa_index(i, w)] = src[aosoa_index(a, w)];
@@ -586,7 +586,7 @@ hipError_t launch_gather_states(hipStream_t st, const uint32_t* src, uint32_t n_
   if (n_src >= ROW_MIN && n_src <= ROW_DST && n >= n_src / 2 && n <= ROW_DST)
     k_gather_rows<<<ARENA_WORDS, ROW_THREADS, ROW_PART * sizeof(uint32_t), st>>>(src, n_src, perm, dst, n);
   else
-    k_gather_states<<<blocks_of(n, 256) * ARENA_WORDS, 256, 0, st>>>(src, n_src, perm, dst, n);
+    k_gather_states<<<dim3(blocks_of(n, 256) * 8u, ARENA_WORDS / 8), 256, 0, st>>>(src, n_src, perm, dst, n);
   return hipGetLastError();
 }
 

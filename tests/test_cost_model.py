@@ -491,3 +491,25 @@ def test_gradient_groups(rsim, device, b):
     assert np.abs(device.read_words(loss).view(np.float32) - want_loss).max() <= 2.0**-7 * np.abs(want_loss).max()
     for lo, hi in ((cm.W1, cm.B1), (cm.B1, cm.W2), (cm.W2, cm.B2), (cm.B2, cm.W3), (cm.W3, cm.B3), (cm.B3, cm.PARAMS)):
         assert np.abs(got[lo:hi] - want[lo:hi]).max() <= 2.0**-7 * np.abs(want[lo:hi]).max(), lo
+
+
+@pytest.mark.gpu
+def test_gather_states_past_a_one_dimensional_grid(rsim, device):
+    """One arena more than 2^32 work-items of one per word and arena, in groups of 256, allow in one dimension (17 GB): the
+    arenas at the edges of the batch and some of those between, gathered back into a small buffer."""
+    n = 2**32 // (256 * rsim.ARENA_WORDS) * 256 + 1
+    note("gather_states, %d arenas" % n)
+    rng = np.random.default_rng(3)
+    states = rng.integers(0, 2**32, (64, rsim.ARENA_WORDS), dtype=np.uint32)
+    src, dst = device.upload_states(states), device.alloc_states(n)
+    try:
+        perm = rng.integers(0, 70, n, dtype=np.uint32)  # 64..69 are past the source: those arenas stay zero
+        device.gather_states(src, device.upload_words(perm), dst)
+        some = np.unique(np.concatenate([[0, 63, 64, 65, n // 2, n - 258, n - 257, n - 256, n - 2, n - 1],
+                                         rng.integers(0, n, 500)])).astype(np.uint32)
+        got = device.alloc_states(len(some))
+        device.gather_states(dst, device.upload_words(some), got)
+        want = np.concatenate([states, np.zeros((6, rsim.ARENA_WORDS), np.uint32)])[perm[some]]
+        assert np.array_equal(device.download_states(got), want)
+    finally:
+        dst.free()
