@@ -120,7 +120,7 @@ void unpack(const uint32_t* in, uint32_t n, ArenaState* states) {
 
 // The staging buffer of state uploads and downloads: allocated by the first such call, sized to the largest batch seen up
 // to STAGE_ARENAS (65 MB), freed with the device; where the device has no room for that, as much as it has, down to one
-// block. Every call that uses it ends synchronised, so it is never in use here.
+// block. Every call that uses it ends synchronised (finish_transfer), so it is never in use here.
 constexpr uint32_t STAGE_ARENAS = 6144;
 int ensure_stage(rsim_device* dev, uint32_t n) {
   uint32_t want = n < STAGE_ARENAS ? n : STAGE_ARENAS;
@@ -142,6 +142,14 @@ int ensure_stage(rsim_device* dev, uint32_t n) {
 uint32_t stage_step(const rsim_device* dev, uint32_t n) {
   const uint32_t cap = dev->stage_cap < STAGE_ARENAS ? dev->stage_cap : STAGE_ARENAS;
   return n <= cap ? n : cap / rs::dev::AOSOA_LANES * rs::dev::AOSOA_LANES;
+}
+
+// The end of a transfer whose steps were queued up to the first error e: waited for in any case, since what is queued reads
+// or writes the caller's memory and the staging buffer.
+int finish_transfer(rsim_device* dev, hipError_t e, const char* what) {
+  const hipError_t done = hipStreamSynchronize(dev->stream);
+  RSIM_HIP(e != hipSuccess ? e : done, what);
+  return RSIM_OK;
 }
 
 int ensure_status(rsim_device* dev, uint32_t n) {
@@ -325,13 +333,13 @@ int rsim_write_states(rsim_device* dev, rsim_states* dst, const void* states) {
   if ((rc = ensure_stage(dev, dst->n))) return rc;
   const ArenaState* src = static_cast<const ArenaState*>(states);
   const uint32_t step = stage_step(dev, dst->n);
-  for (uint32_t a = 0; a < dst->n; a += step) {  // whole blocks but for the last, packed on the device
+  hipError_t e = hipSuccess;
+  for (uint32_t a = 0; e == hipSuccess && a < dst->n; a += step) {  // whole blocks but for the last, packed on the device
     const uint32_t m = dst->n - a < step ? dst->n - a : step;
-    RSIM_HIP(hipMemcpyAsync(dev->stage, src + a, (size_t)m * sizeof(ArenaState), hipMemcpyHostToDevice, dev->stream), "state upload");
-    RSIM_HIP(rs::dev::launch_pack_states(dev->stream, dev->stage, dst->d + rs::dev::aosoa_index(a, 0), m), "state upload");
+    e = hipMemcpyAsync(dev->stage, src + a, (size_t)m * sizeof(ArenaState), hipMemcpyHostToDevice, dev->stream);
+    if (e == hipSuccess) e = rs::dev::launch_pack_states(dev->stream, dev->stage, dst->d + rs::dev::aosoa_index(a, 0), m);
   }
-  RSIM_HIP(hipStreamSynchronize(dev->stream), "state upload");
-  return RSIM_OK;
+  return finish_transfer(dev, e, "state upload");
 }
 int rsim_upload_states(rsim_device* dev, const void* states, uint32_t n, rsim_states** out) {
   int rc = rsim_alloc_states(dev, n, out);
@@ -381,13 +389,13 @@ int rsim_download_states(rsim_device* dev, const rsim_states* s, void* out) {
   if ((rc = ensure_stage(dev, s->n))) return rc;
   ArenaState* dst = static_cast<ArenaState*>(out);
   const uint32_t step = stage_step(dev, s->n);
-  for (uint32_t a = 0; a < s->n; a += step) {
+  hipError_t e = hipSuccess;
+  for (uint32_t a = 0; e == hipSuccess && a < s->n; a += step) {
     const uint32_t m = s->n - a < step ? s->n - a : step;
-    RSIM_HIP(rs::dev::launch_unpack_states(dev->stream, s->d + rs::dev::aosoa_index(a, 0), dev->stage, m), "state download");
-    RSIM_HIP(hipMemcpyAsync(dst + a, dev->stage, (size_t)m * sizeof(ArenaState), hipMemcpyDeviceToHost, dev->stream), "state download");
+    e = rs::dev::launch_unpack_states(dev->stream, s->d + rs::dev::aosoa_index(a, 0), dev->stage, m);
+    if (e == hipSuccess) e = hipMemcpyAsync(dst + a, dev->stage, (size_t)m * sizeof(ArenaState), hipMemcpyDeviceToHost, dev->stream);
   }
-  RSIM_HIP(hipStreamSynchronize(dev->stream), "state download");
-  return RSIM_OK;
+  return finish_transfer(dev, e, "state download");
 }
 
 // ---- word buffers ------------------------------------------------------------------------------------------------------------
