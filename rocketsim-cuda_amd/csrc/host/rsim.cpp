@@ -120,7 +120,7 @@ void unpack(const uint32_t* in, uint32_t n, ArenaState* states) {
 
 // The staging buffer of state uploads and downloads: allocated by the first such call, sized to the largest batch seen up
 // to STAGE_ARENAS (65 MB), freed with the device; where the device has no room for that, as much as it has, down to one
-// block. Every call that uses it ends synchronised (finish_transfer), so it is never in use here.
+// block, and without room for that none (stage_cap 0): the host then transposes the whole batch itself. Every call that uses it ends synchronised (finish_transfer), so it is never in use here.
 constexpr uint32_t STAGE_ARENAS = 6144;
 int ensure_stage(rsim_device* dev, uint32_t n) {
   uint32_t want = n < STAGE_ARENAS ? n : STAGE_ARENAS;
@@ -129,8 +129,10 @@ int ensure_stage(rsim_device* dev, uint32_t n) {
   dev->stage = nullptr;
   dev->stage_cap = 0;
   hipError_t e;
-  while ((e = hipMalloc((void**)&dev->stage, (size_t)want * sizeof(ArenaState))) == hipErrorOutOfMemory && want > rs::dev::AOSOA_LANES) {
+  while ((e = hipMalloc((void**)&dev->stage, (size_t)want * sizeof(ArenaState))) == hipErrorOutOfMemory) {
     (void)hipGetLastError();  // tried again smaller
+    dev->stage = nullptr;
+    if (want <= rs::dev::AOSOA_LANES) return RSIM_OK;
     want = want / 2 > rs::dev::AOSOA_LANES ? want / 2 / rs::dev::AOSOA_LANES * rs::dev::AOSOA_LANES : rs::dev::AOSOA_LANES;
   }
   RSIM_HIP(e, "hipMalloc(stage)");
@@ -149,6 +151,15 @@ uint32_t stage_step(const rsim_device* dev, uint32_t n) {
 int finish_transfer(rsim_device* dev, hipError_t e, const char* what) {
   const hipError_t done = hipStreamSynchronize(dev->stream);
   RSIM_HIP(e != hipSuccess ? e : done, what);
+  return RSIM_OK;
+}
+// A batch's words in the host's memory, for the transfers without a staging buffer.
+int host_words(uint32_t n, std::vector<uint32_t>& v) {
+  try {
+    v.resize(rs::dev::aosoa_words(n));
+  } catch (...) {
+    return fail(RSIM_ERR_INVALID, "state transfer: out of host memory");
+  }
   return RSIM_OK;
 }
 
@@ -332,6 +343,12 @@ int rsim_write_states(rsim_device* dev, rsim_states* dst, const void* states) {
   if (!dst->n) return RSIM_OK;
   if ((rc = ensure_stage(dev, dst->n))) return rc;
   const ArenaState* src = static_cast<const ArenaState*>(states);
+  if (!dev->stage) {
+    std::vector<uint32_t> words;
+    if ((rc = host_words(dst->n, words))) return rc;
+    pack(src, dst->n, words.data());
+    return finish_transfer(dev, hipMemcpyAsync(dst->d, words.data(), words.size() * 4, hipMemcpyHostToDevice, dev->stream), "state upload");
+  }
   const uint32_t step = stage_step(dev, dst->n);
   hipError_t e = hipSuccess;
   for (uint32_t a = 0; e == hipSuccess && a < dst->n; a += step) {  // whole blocks but for the last, packed on the device
@@ -388,6 +405,12 @@ int rsim_download_states(rsim_device* dev, const rsim_states* s, void* out) {
   if (!s->n) return RSIM_OK;
   if ((rc = ensure_stage(dev, s->n))) return rc;
   ArenaState* dst = static_cast<ArenaState*>(out);
+  if (!dev->stage) {
+    std::vector<uint32_t> words;
+    if ((rc = host_words(s->n, words)) || (rc = rsim_download_words(dev, s, words.data()))) return rc;
+    unpack(words.data(), s->n, dst);
+    return RSIM_OK;
+  }
   const uint32_t step = stage_step(dev, s->n);
   hipError_t e = hipSuccess;
   for (uint32_t a = 0; e == hipSuccess && a < s->n; a += step) {

@@ -113,6 +113,19 @@ void failing_copy(rsim_device* dev) {
   round_trip(dev, s, n, 2);
   CHECK(rsim_states_free(s) == RSIM_OK);
 }
+// A device that has room for the caller's buffers and no more: transfers work all the same.
+void full_device(rsim_device* dev) {
+  for (uint32_t n : {1u, 200u, 6500u}) {
+    rsim_states* s = nullptr;
+    g_room = rsim_aosoa_words(n) * 4;
+    CHECK(rsim_alloc_states(dev, n, &s) == RSIM_OK);
+    round_trip(dev, s, n, 3);
+    CHECK(rsim_states_free(s) == RSIM_OK);
+    const std::vector<uint32_t> in = make_states(n, 4);
+    CHECK(rsim_upload_states(dev, in.data(), n, &s) == RSIM_OK);
+    CHECK(rsim_states_free(s) == RSIM_OK);
+  }
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -120,6 +133,7 @@ int main(int argc, char** argv) {
   rsim_device* dev = nullptr;
   CHECK(rsim_open(0, &dev) == RSIM_OK);
   if (!strcmp(what, "failing_copy")) failing_copy(dev);
+  else if (!strcmp(what, "full_device")) full_device(dev);
   else CHECK(!"a known case");
   CHECK(rsim_close(dev) == RSIM_OK && g_live.empty());
   printf("ok\n");
