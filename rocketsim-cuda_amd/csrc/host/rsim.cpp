@@ -31,6 +31,7 @@ struct rsim_device {
   uint32_t* order_scratch;  // this GPU's copy of the allocation-free order's fixed workspace (rsim_cost_order_noalloc)
   uint32_t* stage;          // ArenaStates on their way to or from the host, at most STAGE_ARENAS (state uploads and downloads)
   uint32_t stage_cap;       // its size in arenas
+  bool stage_full;          // no larger one was to be had since a buffer of this device was last freed
   uint32_t* queue;          // the block queue's counter of rsim_run_queued (one word, reset on the stream by each launch)
 };
 struct rsim_world {
@@ -119,25 +120,33 @@ void unpack(const uint32_t* in, uint32_t n, ArenaState* states) {
 }
 
 // The staging buffer of state uploads and downloads: allocated by the first such call, sized to the largest batch seen up
-// to STAGE_ARENAS (65 MB), freed with the device; where the device has no room for that, as much as it has, down to one
-// block, and without room for that none (stage_cap 0): the host then transposes the whole batch itself. Every call that uses it ends synchronised (finish_transfer), so it is never in use here.
+// to STAGE_ARENAS (65 MB), freed with the device. Where the device has no room for that, as much as it has, down to one
+// block, and without room for that none (stage_cap 0): the host then transposes the whole batch itself. What is held is
+// given up for a larger one only, and after a refusal the next try waits until a buffer of the device is freed. Every call
+// that uses it ends synchronised (finish_transfer), so it is never in use here.
 constexpr uint32_t STAGE_ARENAS = 6144;
 int ensure_stage(rsim_device* dev, uint32_t n) {
   uint32_t want = n < STAGE_ARENAS ? n : STAGE_ARENAS;
-  if (dev->stage_cap >= want) return RSIM_OK;
-  if (dev->stage) (void)hipFree(dev->stage);
-  dev->stage = nullptr;
-  dev->stage_cap = 0;
+  if (dev->stage_cap >= want || dev->stage_full) return RSIM_OK;
+  constexpr uint32_t BLOCK = rs::dev::AOSOA_LANES;
+  uint32_t* larger = nullptr;
   hipError_t e;
-  while ((e = hipMalloc((void**)&dev->stage, (size_t)want * sizeof(ArenaState))) == hipErrorOutOfMemory) {
+  while ((e = hipMalloc((void**)&larger, (size_t)want * sizeof(ArenaState))) == hipErrorOutOfMemory) {
     (void)hipGetLastError();  // tried again smaller
-    dev->stage = nullptr;
-    if (want <= rs::dev::AOSOA_LANES) return RSIM_OK;
-    want = want / 2 > rs::dev::AOSOA_LANES ? want / 2 / rs::dev::AOSOA_LANES * rs::dev::AOSOA_LANES : rs::dev::AOSOA_LANES;
+    dev->stage_full = true;
+    want = want <= BLOCK ? 0 : want / 2 < BLOCK ? BLOCK : want / 2 / BLOCK * BLOCK;
+    if (want <= dev->stage_cap) return RSIM_OK;
   }
   RSIM_HIP(e, "hipMalloc(stage)");
+  if (dev->stage) (void)hipFree(dev->stage);
+  dev->stage = larger;
   dev->stage_cap = want;
   return RSIM_OK;
+}
+// A buffer of the device is gone: a larger staging buffer may fit now.
+void freed(rsim_device* dev) {
+  --dev->live;
+  dev->stage_full = false;
 }
 
 // Arenas staged at a time for a batch of n: all of them, or whole blocks.
@@ -311,7 +320,7 @@ int rsim_world_free(rsim_world* w) {
   if (rc) return rc;
   (void)hipStreamSynchronize(w->dev->stream);
   (void)hipFree(w->d);
-  --w->dev->live;
+  freed(w->dev);
   delete w;
   return RSIM_OK;
 }
@@ -382,7 +391,7 @@ int rsim_states_free(rsim_states* s) {
   if (rc) return rc;
   (void)hipStreamSynchronize(s->dev->stream);
   (void)hipFree(s->d);
-  --s->dev->live;
+  freed(s->dev);
   delete s;
   return RSIM_OK;
 }
@@ -486,7 +495,7 @@ int rsim_words_free(rsim_words* b) {
   if (rc) return rc;
   (void)hipStreamSynchronize(b->dev->stream);
   (void)hipFree(b->d);
-  --b->dev->live;
+  freed(b->dev);
   delete b;
   return RSIM_OK;
 }

@@ -17,7 +17,7 @@ namespace {
 size_t g_room = ~(size_t)0;  // bytes that the device still has
 std::map<void*, size_t> g_live;
 std::vector<std::function<void()>> g_queue;
-int g_copies = 0, g_failing_copy = -1;
+int g_mallocs = 0, g_frees = 0, g_copies = 0, g_failing_copy = -1;
 
 #define CHECK(x)                                             \
   do {                                                       \
@@ -40,6 +40,7 @@ hipError_t hipGetLastError(void) { return hipSuccess; }
 const char* hipGetErrorName(hipError_t) { return "error"; }
 const char* hipGetErrorString(hipError_t) { return "of the test's runtime"; }
 hipError_t hipMalloc(void** p, size_t bytes) {
+  ++g_mallocs;
   *p = nullptr;
   if (bytes > g_room) return hipErrorOutOfMemory;
   g_room -= bytes;
@@ -48,6 +49,7 @@ hipError_t hipMalloc(void** p, size_t bytes) {
   return hipSuccess;
 }
 hipError_t hipFree(void* p) {
+  ++g_frees;
   CHECK(g_live.count(p) == 1);
   g_room += g_live[p];
   g_live.erase(p);
@@ -126,6 +128,30 @@ void full_device(rsim_device* dev) {
     CHECK(rsim_states_free(s) == RSIM_OK);
   }
 }
+// A device with room for a small staging buffer, or none: the transfers after the first neither free it nor ask for more,
+// until a buffer of the device is freed.
+void small_stage(rsim_device*& dev) {
+  const size_t arena = rs::ARENA_WORDS * 4;
+  for (uint32_t room : {0u, 130u, 900u}) {
+    rsim_states *s = nullptr, *other = nullptr;
+    const uint32_t n = 2000;
+    g_room = 2 * rsim_aosoa_words(n) * 4 + room * arena;
+    CHECK(rsim_alloc_states(dev, n, &s) == RSIM_OK && rsim_alloc_states(dev, n, &other) == RSIM_OK);
+    round_trip(dev, s, n, 5);
+    const int mallocs = g_mallocs, frees = g_frees;
+    for (uint32_t k = 0; k < 3; ++k) {
+      round_trip(dev, s, n, 6 + k);
+      CHECK(g_mallocs == mallocs && g_frees == frees);
+    }
+    CHECK(rsim_states_free(other) == RSIM_OK);
+    round_trip(dev, s, n, 9);
+    CHECK(g_room == rsim_aosoa_words(n) * 4 + room * arena - n * arena);  // now the whole batch is staged at once
+    CHECK(rsim_states_free(s) == RSIM_OK);
+    rsim_device* fresh = nullptr;  // the next case starts without a staging buffer
+    CHECK(rsim_open(0, &fresh) == RSIM_OK && rsim_close(dev) == RSIM_OK);
+    dev = fresh;
+  }
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -134,6 +160,7 @@ int main(int argc, char** argv) {
   CHECK(rsim_open(0, &dev) == RSIM_OK);
   if (!strcmp(what, "failing_copy")) failing_copy(dev);
   else if (!strcmp(what, "full_device")) full_device(dev);
+  else if (!strcmp(what, "small_stage")) small_stage(dev);
   else CHECK(!"a known case");
   CHECK(rsim_close(dev) == RSIM_OK && g_live.empty());
   printf("ok\n");
