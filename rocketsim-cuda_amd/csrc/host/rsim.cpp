@@ -120,10 +120,11 @@ void unpack(const uint32_t* in, uint32_t n, ArenaState* states) {
 }
 
 // The staging buffer of state uploads and downloads: allocated by the first such call, sized to the largest batch seen up
-// to STAGE_ARENAS (65 MB), freed with the device. Where the device has no room for that, as much as it has, down to one
-// block, and without room for that none (stage_cap 0): the host then transposes the whole batch itself. What is held is
-// given up for a larger one only, and after a refusal the next try waits until a buffer of the device is freed. Every call
-// that uses it ends synchronised (finish_transfer), so it is never in use here.
+// to STAGE_ARENAS (68 MB), freed with the device or where one of the caller's buffers needs its room. Where the device has
+// no room for that, as much as it has, down to one block, and without room for that none (stage_cap 0): the host then
+// transposes the whole batch itself. What is held is given up for a larger one only, and after a refusal the next try waits
+// until a buffer of the device is freed. Every call that uses it ends synchronised (finish_transfer), so it is never in use
+// here.
 constexpr uint32_t STAGE_ARENAS = 6144;
 int ensure_stage(rsim_device* dev, uint32_t n) {
   uint32_t want = n < STAGE_ARENAS ? n : STAGE_ARENAS;
@@ -142,6 +143,16 @@ int ensure_stage(rsim_device* dev, uint32_t n) {
   dev->stage = larger;
   dev->stage_cap = want;
   return RSIM_OK;
+}
+// A buffer of the caller's: where the device has no room for it, the staging buffer is given back first.
+hipError_t alloc(rsim_device* dev, void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipErrorOutOfMemory || !dev->stage) return e;
+  (void)hipGetLastError();  // tried again
+  (void)hipFree(dev->stage);
+  dev->stage = nullptr;
+  dev->stage_cap = 0;
+  return hipMalloc(p, bytes);
 }
 // A buffer of the device is gone: a larger staging buffer may fit now.
 void freed(rsim_device* dev) {
@@ -178,7 +189,7 @@ int ensure_status(rsim_device* dev, uint32_t n) {
   dev->status = nullptr;
   dev->status_cap = 0;
   uint32_t cap = n < 64 ? 64 : n;
-  RSIM_HIP(hipMalloc((void**)&dev->status, (size_t)cap * sizeof(int32_t)), "hipMalloc(status)");
+  RSIM_HIP(alloc(dev, (void**)&dev->status, (size_t)cap * sizeof(int32_t)), "hipMalloc(status)");
   dev->status_cap = cap;
   return RSIM_OK;
 }
@@ -297,7 +308,7 @@ int rsim_upload_worlds(rsim_device* dev, const void* static_data, uint32_t count
   rsim_world* w = new (std::nothrow) rsim_world{dev, nullptr, count};
   if (!w) return fail(RSIM_ERR_INVALID, "out of host memory");
   const size_t bytes = sizeof(StaticData) * count;
-  hipError_t e = hipMalloc((void**)&w->d, bytes);
+  hipError_t e = alloc(dev, (void**)&w->d, bytes);
   if (e == hipSuccess) e = hipMemcpyAsync(w->d, static_data, bytes, hipMemcpyHostToDevice, dev->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(dev->stream);
   if (e != hipSuccess) {
@@ -333,7 +344,7 @@ int rsim_alloc_states(rsim_device* dev, uint32_t n, rsim_states** out) {
   size_t bytes = rs::dev::aosoa_words(n > 0 ? n : 1) * sizeof(uint32_t);
   rsim_states* s = new (std::nothrow) rsim_states{dev, nullptr, n};
   if (!s) return fail(RSIM_ERR_INVALID, "out of host memory");
-  hipError_t e = hipMalloc((void**)&s->d, bytes);
+  hipError_t e = alloc(dev, (void**)&s->d, bytes);
   if (e == hipSuccess) e = hipMemsetAsync(s->d, 0, bytes, dev->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(dev->stream);
   if (e != hipSuccess) {
@@ -438,7 +449,7 @@ int rsim_alloc_words(rsim_device* dev, uint64_t words, rsim_words** out) {
   rsim_words* b = new (std::nothrow) rsim_words{dev, nullptr, words};
   if (!b) return fail(RSIM_ERR_INVALID, "out of host memory");
   size_t bytes = (words > 0 ? words : 1) * 4;
-  hipError_t e = hipMalloc((void**)&b->d, bytes);
+  hipError_t e = alloc(dev, (void**)&b->d, bytes);
   if (e == hipSuccess) e = hipMemsetAsync(b->d, 0, bytes, dev->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(dev->stream);
   if (e != hipSuccess) {

@@ -22,7 +22,7 @@ def program(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("case", ["failing_copy", "full_device", "small_stage"])
+@pytest.mark.parametrize("case", ["failing_copy", "full_device", "small_stage", "given_back"])
 def test_transfers(program, case):
     r = subprocess.run([program, case], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout

@@ -152,6 +152,27 @@ void small_stage(rsim_device*& dev) {
     dev = fresh;
   }
 }
+// The staging buffer stands in no allocation's way: a buffer that fits only without it gets its room.
+void given_back(rsim_device* dev) {
+  const uint32_t n = 512, worlds = 3;
+  const uint64_t words = rsim_aosoa_words(n);
+  rsim_states *s = nullptr, *t = nullptr;
+  rsim_words* b = nullptr;
+  rsim_world* w = nullptr;
+  CHECK(rsim_alloc_states(dev, n, &s) == RSIM_OK);
+  const std::vector<uint32_t> table((size_t)rs::STATIC_WORDS * worlds);
+  for (int kind = 0; kind < 4; ++kind) {
+    g_room = (size_t)n * rs::ARENA_WORDS * 4;
+    round_trip(dev, s, n, 10 + kind);  // the staging buffer takes all of it
+    CHECK(g_room == 0);
+    if (kind == 0) CHECK(rsim_alloc_states(dev, n, &t) == RSIM_OK && rsim_states_free(t) == RSIM_OK);
+    if (kind == 1) CHECK(rsim_alloc_words(dev, words, &b) == RSIM_OK && rsim_words_free(b) == RSIM_OK);
+    if (kind == 2) CHECK(rsim_upload_worlds(dev, table.data(), worlds, &w) == RSIM_OK && rsim_world_free(w) == RSIM_OK);
+    if (kind == 3) CHECK(rsim_alloc_words(dev, words + 1, &b) == RSIM_ERR_HIP);
+  }
+  round_trip(dev, s, n, 14);
+  CHECK(rsim_states_free(s) == RSIM_OK);
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -161,6 +182,7 @@ int main(int argc, char** argv) {
   if (!strcmp(what, "failing_copy")) failing_copy(dev);
   else if (!strcmp(what, "full_device")) full_device(dev);
   else if (!strcmp(what, "small_stage")) small_stage(dev);
+  else if (!strcmp(what, "given_back")) given_back(dev);
   else CHECK(!"a known case");
   CHECK(rsim_close(dev) == RSIM_OK && g_live.empty());
   printf("ok\n");
