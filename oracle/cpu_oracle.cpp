@@ -274,6 +274,25 @@ uint64_t rsim_cpu_check_move_cells(const StaticData* w, uint64_t seed, uint64_t 
   }
   return bad;
 }
+// How many mesh leaves the next tick's narrowphase jobs of this state walk to, all jobs together and however many a batch
+// holds (for tests that fill the pooled walk's queues).
+uint32_t rsim_cpu_mesh_leaves(const ArenaState* state, const StaticData* w) {
+  ArenaState s = *state;
+  for (int k = 0; k < 4; ++k) run_phase(k, s, *w);
+  Np c = {s, *w, 0, nullptr, nullptr, 0u, s.n_records};
+  uint32_t leaves = 0, jobs = 0;
+  for (uint32_t i = 0; i < s.n_pairs && jobs < (uint32_t)TJ_MAX; ++i) {
+    uint32_t body, mesh_b, leaf;
+    const int kind = mesh_job_of(c, w->proxies[s.pairs[i].proxy0].client_body, w->proxies[s.pairs[i].proxy1].client_body, &body, &mesh_b);
+    if (kind < 0) continue;
+    ++jobs;
+    const Aabb box = kind == TJ_CAR ? car_mesh_frame(c, body, mesh_b).local_box : ball_mesh_box(c, body, mesh_b);
+    BvhCursor cur;
+    cursor_init(cur, w->meshes[mesh_b], box);
+    while (cursor_next_leaf(cur, *w, w->meshes[mesh_b], box, &leaf)) ++leaves;
+  }
+  return leaves;
+}
 uint64_t rsim_cpu_arena_words() { return ARENA_WORDS; }
 uint64_t rsim_cpu_tick_words() { return TICK_WORDS; }
 uint64_t rsim_cpu_static_words() { return STATIC_WORDS; }

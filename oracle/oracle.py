@@ -61,6 +61,8 @@ class Oracle:
         L.rsim_cpu_check_sweep.restype = _u64
         L.rsim_cpu_check_island_sort.argtypes = [_u64, _u64]
         L.rsim_cpu_check_island_sort.restype = _u64
+        L.rsim_cpu_mesh_leaves.argtypes = [_vp, _vp]
+        L.rsim_cpu_mesh_leaves.restype = _u32
         for f in ("rsim_cpu_arena_words", "rsim_cpu_tick_words", "rsim_cpu_static_words", "rsim_cpu_controls_word"):
             getattr(L, f).restype = _u64
         self.L = L
@@ -131,6 +133,10 @@ class Oracle:
     def check_sweep(self, world, state, seed, iters):
         """Mismatches of the broadphase phase against the literal swaps, body by body and axis by axis, over random moves."""
         return int(self.L.rsim_cpu_check_sweep(_p(world), _p(state), seed, iters))
+
+    def mesh_leaves(self, state, world):
+        """Leaves that the next tick's narrowphase jobs of one state walk to."""
+        return int(self.L.rsim_cpu_mesh_leaves(_p(state), _p(world)))
 
     # -- workloads (the same builder source as the product's) --
     def build_world(self, p0=0, p1=0, gravity_z=-650.0, boost_accel_scale=1.0, ball_radius=91.25):

@@ -154,3 +154,27 @@ def test_cars_tied_to_each_other(rsim, oracle, world, device, dev_world, n):
         stood |= ((ray["some"] != 0) & (ray["v"]["ground_stick"]["some"] != 0)).any((1, 2))
     assert stood[1::4].any() and (n < 4 or stood[2::4].any()), "some wheels stood on a car, some on the ball"
     same(device.download_states(d), states, "tied cars %d" % n)
+
+
+@pytest.mark.parametrize("per_wave", [1, 3])
+def test_small_batches_past_the_pooled_queues(rsim, oracle, device, per_wave):
+    """A ball of 800 uu, whose box takes in up to some hundred mesh leaves: the pooled walk of a small batch's wave holds 232
+    leaves, and the arenas are chosen so that waves end below that, on its last slot and past it (each lane then walks its
+    own meshes)."""
+    slots, n = 232, 300 if per_wave == 1 else 900
+    print("[case] %d arenas, %d a wave, around %d leaves a wave" % (n, per_wave, slots), flush=True)
+    world = rsim.build_world(0, 0, ball_radius=800.0)
+    many = rsim.sample_arenas(world, rsim.SCEN_PINCH, 905, 3000)
+    leaves = np.array([oracle.mesh_leaves(s, world) for s in many])
+    waves = np.random.default_rng(906).integers(0, len(many), (20000, per_wave))
+    total = leaves[waves].sum(1)
+    near = np.argsort(np.abs(total - slots), kind="stable")[:n // per_wave * 9 // 10]
+    waves, total = np.concatenate([waves[near], waves[:n // per_wave - len(near)]]), total[near]
+    assert (total < slots).any() and (total == slots).any() and (total > slots).any()
+    states = np.ascontiguousarray(many[waves.ravel()])
+    d, dw, r = device.upload_states(states), device.upload_static(world), device.alloc_words(n)
+    for k in range(3):
+        ctl = rsim.sample_controls(907, k, n)
+        device.sim8(d, dw, device.upload_controls(ctl), r)
+        assert np.array_equal(device.read_words(r), oracle.sim8(states, world, ctl, threads=8)), k
+    same(device.download_states(d), states, "past the pooled queues, %d a wave" % per_wave)
