@@ -161,3 +161,15 @@ def test_queued_run_in_cost_order_with_worlds(rsim, oracle, device):
     gs, gr = queued_run(device, dw, states, ctl, 64, order, 0, variant=dv)
     cs, cr = cpu_decisions_in(oracle, worlds, variant, states, ctl)
     check(gs, gr, cs, cr, "run_queued cost order")
+
+
+@pytest.mark.parametrize("n,scenario", [(32768 + 1, "kickoff"), (65536 + 64 + 1, "open_contact")])
+def test_queued_run_in_its_production_form(rsim, oracle, world, device, dev_world, n, scenario):
+    """Block 64, index order, as many work-groups as are resident, which up to 32,768 arenas is left to rsim_run's waves:
+    just past that, and past the waves that the chip holds; the last block with one arena."""
+    note("run_queued block 64 workgroups 0, %d %s arenas, 2 decisions" % (n, scenario))
+    states = rsim.sample_arenas(world, getattr(rsim, "SCEN_" + scenario.upper()), 341, n)
+    ctl = [rsim.sample_controls(342, d, n) for d in range(2)]
+    gs, gr = queued_run(device, dev_world, states, ctl, 64)
+    cs, cr = cpu_decisions(oracle, world, states, ctl)
+    check(gs, gr, cs, cr, "run_queued %d" % n)
