@@ -513,3 +513,89 @@ def test_gather_states_past_a_one_dimensional_grid(rsim, device):
         assert np.array_equal(device.download_states(got), want)
     finally:
         dst.free()
+
+
+def with_biases(seed):
+    """Initial parameters with biases of the activations' own size (init_params' are zero, so that a bias left out or put in
+    another place would not show)."""
+    p = cm.init_params(seed)
+    rng = np.random.default_rng(seed + 1000)
+    for lo, hi in ((cm.B1, cm.W2), (cm.B2, cm.W3), (cm.B3, cm.PARAMS)):
+        p[lo:hi] = rng.standard_normal(hi - lo) * 0.5
+    return p
+
+
+def prediction_bound(p, feat):
+    """How far fp32 sums can take a row's prediction from ref_forward's: a layer's sum of k terms is off by at most k 2^-23 of
+    the sum of their sizes, its activation by what rounding makes of that interval (for most rows nothing), and what is off
+    in one layer by its weights in the next."""
+    w1, b1, w2, b2, w3, b3 = unpack(p)
+    h, d = bf16(feat), 0.0
+    for w, b in ((bf16(w1), b1), (bf16(w2), b2)):
+        pre = h @ w + b
+        off = np.abs(d) @ np.abs(w) if np.ndim(d) else 0.0
+        off = off + (len(w) + 1) * 2.0**-23 * ((np.abs(h) + d) @ np.abs(w) + np.abs(b))
+        lo, h, up = (bf16(np.maximum(v, 0.0)) for v in (pre - off, pre, pre + off))
+        d = np.maximum(up - h, h - lo)
+    w3 = np.abs(bf16(w3))
+    return d @ w3 + 65 * 2.0**-23 * ((h + d) @ w3 + np.abs(b3))
+
+
+def test_prediction_bound_sees_mistakes():
+    """The bound of the prediction tests with biases, on the host: networks with one thing wrong are past it."""
+    p = with_biases(31)
+    feat = np.clip(np.random.default_rng(32).standard_normal((4097, cm.FEATURES)), -4, 4).astype(np.float32)
+    want, bound = ref_forward(p, feat)[3], prediction_bound(p, feat)
+
+    def past(q, rounding=True):
+        return (np.abs(ref_forward(q, feat, rounding)[3] - want) > bound).mean()
+
+    def without(lo, hi, put):
+        q = p.copy()
+        q[lo:hi] = put(p[lo:hi])
+        return past(q)
+
+    assert past(p) == 0.0
+    assert past(p, rounding=False) > 0.5
+    for lo, hi in ((cm.B1, cm.W2), (cm.B2, cm.W3), (cm.B3, cm.PARAMS)):
+        assert without(lo, hi, np.zeros_like) > 0.9 and without(lo, hi, lambda v: np.roll(v, 1)) > 0.9, lo
+    for k in (cm.B1, cm.B1 + 63, cm.B2 + 4, cm.W3 - 1):  # one bias alone, where its unit is active
+        assert without(k, k + 1, np.zeros_like) > 0.1, k
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 17, 4097, 32768 + 16])
+def test_prediction_with_biases(rsim, device, n):
+    """Every row within what fp32 sums allow (prediction_bound)."""
+    note("cost prediction with biases, %d arenas" % n)
+    p = with_biases(31)
+    feat = np.clip(np.random.default_rng(n).standard_normal((n, cm.FEATURES)), -4, 4).astype(np.float32)
+    model = cm.CostModel(device, p)
+    got = device.read_words(model.predict(device.upload_words(feat.view(np.uint32).ravel()), n)).view(np.float32).reshape(n, 2)
+    off = np.abs(got - ref_forward(p, feat)[3])
+    assert (off <= prediction_bound(p, feat)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b", [33, 4096])
+def test_gradient_with_biases(rsim, device, b):
+    """The gradient with biases in every layer, within 2^-7 of a block's largest entry (as in test_gradient_groups). Rows with
+    a unit so close to its kink that the fp32 sum could put it on the other side are left out of the batch."""
+    note("cost gradients with biases, batch %d" % b)
+    p = with_biases(33)
+    rng = np.random.default_rng(b)
+    feat = np.clip(rng.standard_normal((2 * b, cm.FEATURES)), -4, 4).astype(np.float32)
+    w1, b1, w2, b2, _, _ = unpack(p)
+    x, h1, _, _ = ref_forward(p, feat)
+    kink = np.minimum(np.abs(x @ bf16(w1) + b1).min(1), np.abs(h1 @ bf16(w2) + b2).min(1))
+    feat = np.ascontiguousarray(feat[kink > 65 * 2.0**-23 * 64][:b])
+    assert len(feat) == b
+    target, contact = rng.standard_normal(b).astype(np.float32), (rng.random(b) < 0.4).astype(np.float32)
+    model = cm.CostModel(device, p)
+    up = [device.upload_words(np.ascontiguousarray(v).view(np.uint32).ravel()) for v in (feat, target, contact)]
+    scratch, loss = model.gradients(*up, b)
+    want_loss, want = ref_loss_grad(p, feat, target, contact)
+    got = device.read_words(model.grad).view(np.float32)
+    assert np.abs(device.read_words(loss).view(np.float32) - want_loss).max() <= 2.0**-7 * np.abs(want_loss).max()
+    for lo, hi in ((cm.W1, cm.B1), (cm.B1, cm.W2), (cm.W2, cm.B2), (cm.B2, cm.W3), (cm.W3, cm.B3), (cm.B3, cm.PARAMS)):
+        assert np.abs(got[lo:hi] - want[lo:hi]).max() <= 2.0**-7 * np.abs(want[lo:hi]).max(), lo
