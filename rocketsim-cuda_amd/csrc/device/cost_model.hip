@@ -353,15 +353,24 @@ __global__ void __launch_bounds__(256) k_scatter_words(const uint32_t* __restric
 }
 // AoSoA-64 states: arena i of dst (n arenas) = arena perm[i] of src (n_src arenas); an index past src leaves that arena of
 // dst as it was. The grid walks the words, so all arenas of one word are copied together and the source lines they share
-// are read from HBM once; word w's work-groups are all w % 8 modulo 8, on one XCD and its L2. Eight words in x, their eights
-// in y: a launch takes fewer than 2^32 work-items in x, which one dimension for all words would pass at 1,542,657 arenas.
+// are read from HBM once. With XCD, word w's work-groups are all w % 8 modulo 8, on one XCD and its L2: eight words in x,
+// their eights in y. (A launch takes fewer than 2^32 work-items in x, which one dimension for all words would pass at
+// 1,542,657 arenas.)
+template <bool XCD>
 __global__ void __launch_bounds__(256) k_gather_states(const uint32_t* __restrict__ src, uint32_t n_src,
                                                        const uint32_t* __restrict__ perm, uint32_t* __restrict__ dst, uint32_t n) {
-  const uint32_t w = blockIdx.y * 8u + blockIdx.x % 8u, i = blockIdx.x / 8u * 256u + threadIdx.x;
+  const uint32_t w = XCD ? blockIdx.y * 8u + blockIdx.x % 8u : blockIdx.y;
+  const uint32_t i = (XCD ? blockIdx.x / 8u : blockIdx.x) * 256u + threadIdx.x;
   if (i >= n || w >= (uint32_t)ARENA_WORDS) return;
   uint32_t a = perm[i];
   if (a < n_src) dst[aosoa_index(i, w)] = src[aosoa_index(a, w)];
 }
+// From a sample of one arena in GATHER_SPARSE on, the 32 arenas of a source line have enough readers for the one L2 to pay;
+// a sparser sample of a source past the caches reads most lines for one arena, and a word's reads spread over all XCDs are
+// faster (us without / with: 131,072 to 1,310 arenas 81 / 88, to 3,932 208 / 217, to 6,553 303 / 302, to 9,175 430 / 365,
+// to all 2,554 / 1,855; 800,000 to 24,000 1,240 / 1,325, to 40,000 1,939 / 1,873; but 30,000 to 900 47 / 35, 65,536 to
+// 655 35.0 / 33.5).
+constexpr uint32_t GATHER_SPARSE = 20, GATHER_CACHED = 65536;
 // The same row by row: 4-byte reads at random places, one L2 request each, bound the kernel above (65,536 arenas: 1,148 us
 // without its XCD mapping, 971 us with it). Here a work-group takes one word of all of dst's arenas (up to ROW_DST): the
 // source's row of that word passes through LDS in parts of ROW_PART arenas, read from HBM as whole lines, and every thread
@@ -585,8 +594,10 @@ hipError_t launch_gather_states(hipStream_t st, const uint32_t* src, uint32_t n_
   static_assert(ARENA_WORDS % 8 == 0, "eight words in flight, one per XCD");
   if (n_src >= ROW_MIN && n_src <= ROW_DST && n >= n_src / 2 && n <= ROW_DST)
     k_gather_rows<<<ARENA_WORDS, ROW_THREADS, ROW_PART * sizeof(uint32_t), st>>>(src, n_src, perm, dst, n);
+  else if (n_src <= GATHER_CACHED || n >= n_src / GATHER_SPARSE)
+    k_gather_states<true><<<dim3(blocks_of(n, 256) * 8u, ARENA_WORDS / 8), 256, 0, st>>>(src, n_src, perm, dst, n);
   else
-    k_gather_states<<<dim3(blocks_of(n, 256) * 8u, ARENA_WORDS / 8), 256, 0, st>>>(src, n_src, perm, dst, n);
+    k_gather_states<false><<<dim3(blocks_of(n, 256), ARENA_WORDS), 256, 0, st>>>(src, n_src, perm, dst, n);
   return hipGetLastError();
 }
 

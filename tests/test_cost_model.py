@@ -599,3 +599,20 @@ def test_gradient_with_biases(rsim, device, b):
     assert np.abs(device.read_words(loss).view(np.float32) - want_loss).max() <= 2.0**-7 * np.abs(want_loss).max()
     for lo, hi in ((cm.W1, cm.B1), (cm.B1, cm.W2), (cm.W2, cm.B2), (cm.B2, cm.W3), (cm.W3, cm.B3), (cm.B3, cm.PARAMS)):
         assert np.abs(got[lo:hi] - want[lo:hi]).max() <= 2.0**-7 * np.abs(want[lo:hi]).max(), lo
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 257, 3499, 3500])
+def test_gather_a_sample_of_a_large_source(rsim, device, n):
+    """Samples of 70,000 arenas on both sides of one in 20, where the gather's order of work-groups changes; with indices
+    past the source."""
+    n_src = 70000
+    note("gather_states, %d of %d arenas" % (n, n_src))
+    rng = np.random.default_rng(n)
+    states = rng.integers(0, 2**32, (n_src, rsim.ARENA_WORDS), dtype=np.uint32)
+    src, dst = device.upload_states(states), device.alloc_states(n)
+    idx = rng.integers(0, n_src, n).astype(np.uint32)
+    idx[5::7] = n_src + 3
+    device.gather_states(src, device.upload_words(idx), dst)
+    want = np.where((idx < n_src)[:, None], states[np.minimum(idx, n_src - 1)], np.uint32(0))
+    assert np.array_equal(device.download_states(dst), want)
