@@ -43,7 +43,7 @@ extern "C" {
 #define RSIM_SIM8_UNIMPLEMENTED 0x80000000u /* a tick up to then reached a shape pair V3's port does not implement */
 #define RSIM_SIM8_OVERFLOW 0x40000000u      /* an overflow counter of the state written back is nonzero */
 #define RSIM_SIM8_BAD_VARIANT 0x20000000u   /* (rsim_sim8_variants) the arena's world index is past the table: not stepped */
-#define RSIM_SIM8_BLOCK 64                  /* work-group size in production: one wave64 per AoSoA-64 block */
+#define RSIM_SIM8_BLOCK 64                  /* the block in production: rsim_sim8 and rsim_run choose the wave's shape by n */
 #define RSIM_MAX_BLOCK 256                  /* largest work-group size the tick kernels accept */
 #define RSIM_NUM_PHASES 10                  /* P0, P1, P2, P3a, P3b, P4, P5, P6, P7, P8 (phase.cuh:17-46) */
 #define RSIM_AOSOA_WIDTH 64                 /* arenas per AoSoA block */
@@ -88,7 +88,8 @@ const void* rsim_world_device_ptr(const rsim_world* world);
 int rsim_world_free(rsim_world* world);
 
 /* upload_states / alloc_states (device.rs:73-80): n ArenaStates uploaded and packed to AoSoA-64 on the device; alloc
- * zeroes. */
+ * zeroes. State uploads and downloads go through a staging buffer of at most 68 MB that the device handle keeps from the
+ * first one on; it is freed by rsim_close, or where a buffer or world table of the caller's finds no room beside it. */
 int rsim_upload_states(rsim_device* dev, const void* states, uint32_t n, rsim_states** out);
 int rsim_alloc_states(rsim_device* dev, uint32_t n, rsim_states** out);
 /* Overwrites the n states of an existing buffer (same n) without reallocating. */
@@ -118,8 +119,10 @@ void* rsim_words_device_ptr(rsim_words* buf);
 
 /* sim8 (device.rs:151-168): one decision (8 ticks) of every arena of `states`, in place, asynchronously on the device's
  * stream. controls: >= n * 16 words (rsim_upload_controls). result: >= n words, result[a] the RSIM_SIM8_* word of arena a.
- * block: work-group size, 1..RSIM_MAX_BLOCK (RSIM_SIM8_BLOCK in production); results do not depend on it. trace: null,
- * or >= 8 * rsim_aosoa_words(n) words that receive the state after tick t in slab t - 1 (ticks after a goal are not
+ * block: 1..RSIM_MAX_BLOCK; results do not depend on it. RSIM_SIM8_BLOCK is the one for production: the call then takes
+ * the shape that suits n (to 512 arenas one and to 3,072 three per wave, the states in LDS, an arena on several lanes; to
+ * 32,768 waves of 32 arenas; above, work-groups of 64). Any other block is the work-group's size, a lane per arena. trace:
+ * null, or >= 8 * rsim_aosoa_words(n) words that receive the state after tick t in slab t - 1 (ticks after a goal are not
  * written). */
 int rsim_sim8(rsim_device* dev, rsim_states* states, const rsim_world* world, const rsim_words* controls, rsim_words* result,
               uint32_t block, rsim_words* trace);
@@ -130,13 +133,15 @@ int rsim_sim8_variants(rsim_device* dev, rsim_states* states, const rsim_world* 
                        const rsim_words* controls, rsim_words* result, uint32_t block, rsim_words* trace);
 /* rsim_sim8_variants that also writes each lane's wall-clock ticks (100 MHz) for its decision into `cycles` (>= 2 * n
  * words: n u64). The lanes of a wave share its clock; launched with block 1 every arena has a wave of its own and the
- * count is that arena's own cost (the cost model's labels). No counterpart in the reference. */
+ * count is that arena's own cost (the cost model's labels). With a cycles buffer `block` is the work-group's size at every
+ * n, a lane per arena: at RSIM_SIM8_BLOCK and up to 32,768 arenas that is not the shape that the untimed call would take,
+ * and its clock not that call's. No counterpart in the reference. */
 int rsim_sim8_timed(rsim_device* dev, rsim_states* states, const rsim_world* world, const rsim_words* variant,
                     const rsim_words* controls, rsim_words* result, uint32_t block, rsim_words* trace, rsim_words* cycles);
 
 /* `decisions` consecutive decisions in one launch, asynchronous: the same results as that many rsim_sim8_variants calls
  * (decision d + 1 starts from decision d's written-back state), with each arena held on chip from the first decision to
- * the last instead of being copied out and in between. controls: decisions x n x 16 words (decision-major); results:
+ * the last instead of being copied out and in between. block: as in rsim_sim8. controls: decisions x n x 16 words (decision-major); results:
  * decisions x n words. variant: as in rsim_sim8_variants (null: world 0). No counterpart in the reference; for callers
  * whose controls are known ahead (replays, scripted opponents, benchmarks). */
 int rsim_run(rsim_device* dev, rsim_states* states, const rsim_world* world, const rsim_words* variant, const rsim_words* controls,
@@ -146,7 +151,9 @@ int rsim_run(rsim_device* dev, rsim_states* states, const rsim_world* world, con
  * waves; workgroups 0 = as many as the GPU holds at once, rsim_run_queue_capacity) whose waves each take the next AoSoA
  * block of 64 arenas from a queue and run all `decisions` decisions of it. The queue holds the ceil(n / 64) blocks in
  * the order `order` (a permutation of the block indices, e.g. rsim_cost_block_order's heaviest-first order) or in index
- * order (order null). Same results and states as rsim_run: arenas are independent and each is stepped by one lane.
+ * order (order null). With RSIM_SIM8_BLOCK, workgroups 0, no order and n <= 32,768 the call is rsim_run's: every wave of
+ * such a batch is resident at once, so there is nothing to queue for. Same results and states as rsim_run in every case:
+ * arenas are independent of each other.
  * Asynchronous; calls on one device are ordered by its stream (the queue counter is the device's). No counterpart in
  * the reference. */
 int rsim_run_queued(rsim_device* dev, rsim_states* states, const rsim_world* world, const rsim_words* variant,
@@ -155,7 +162,7 @@ int rsim_run_queued(rsim_device* dev, rsim_states* states, const rsim_world* wor
 uint32_t rsim_run_queue_capacity(rsim_device* dev, uint32_t block); /* resident work-groups of that size (0: unknown) */
 /* One decision as ceil(8 / ticks_per_launch) launches of ticks_per_launch ticks, the state written back to the AoSoA
  * buffer between launches (ticks_per_launch 8 is one launch, as rsim_sim8_variants). Same result words and states as
- * rsim_sim8_variants; a schedule the autotuner measures. Asynchronous. No counterpart in the reference (its sim8 is one
+ * rsim_sim8_variants; a schedule the autotuner measures. block is the work-group's size at every n. Asynchronous. No counterpart in the reference (its sim8 is one
  * launch per decision; step_tick is its one-tick debug kernel, device.rs:96-141). */
 int rsim_sim8_split(rsim_device* dev, rsim_states* states, const rsim_world* world, const rsim_words* variant,
                     const rsim_words* controls, rsim_words* result, uint32_t block, uint32_t ticks_per_launch);

@@ -9,11 +9,15 @@
  *
  * Build: hipcc --offload-arch=gfx950 -I <repo>/include -I <repo>/rocketsim-cuda_amd/csrc with librsim's flags
  * (-ffp-contract=off -fno-fast-math -fno-gpu-flush-denormals-to-zero -fhip-fp32-correctly-rounded-divide-sqrt,
- * -Xclang -target-feature -Xclang -packed-fp32-ops, and -fno-strict-aliasing: load_arena fills the struct through u32
- * words, so a typed read of it straight after is only defined without strict aliasing); other flags can change results.
+ * -Xclang -target-feature -Xclang -packed-fp32-ops, -mllvm -disable-promote-alloca-to-lds, and -fno-strict-aliasing:
+ * load_arena fills the struct through u32 words, so a typed read of it straight after is only defined without strict
+ * aliasing); other flags can change results.
  * Launch: one lane per arena; a kernel that steps arenas takes rsim_dev::lds_bytes(blockDim.x) bytes of dynamic shared
- * memory (the stepper's per-lane LDS slices: traversal stacks, pooled narrowphase stages, solver bank). Lanes may leave
- * early (a >= n) or step different arenas; the wave-pooled stages use whichever lanes are stepping. */
+ * memory (the stepper's per-lane LDS slices: traversal stacks, pooled narrowphase stages, solver bank). The stepper
+ * addresses it from LDS address 0, so such a kernel has no static shared memory: no __shared__ array of its own (what it
+ * needs goes behind the stepper's bytes), and the flag above keeps the compiler from making one. hipFuncGetAttributes'
+ * sharedSizeBytes is 0 for it. Lanes may leave early (a >= n) or step different arenas; the wave-pooled stages use
+ * whichever lanes are stepping. */
 #ifndef RSIM_DEVICE_H
 #define RSIM_DEVICE_H
 

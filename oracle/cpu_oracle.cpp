@@ -74,8 +74,6 @@ void rsim_cpu_static_layout(uint64_t* out) {
 }
 // Word offset of cars[car].controls in ArenaState (for setting controls before a per-phase run).
 uint64_t rsim_cpu_controls_word(int car) { return (offsetof(ArenaState, cars) + car * sizeof(Car) + offsetof(Car, controls)) / 4; }
-// Brute force: move_cells against the remove-then-push sequence it replaces, on `iters` random sorted lists (lengths up
-// to the cap, so overflow is exercised) and random block moves in the given world's grid. Returns the mismatch count.
 // The literal form of P4's island sort (simulation_island_manager.cuh:43-66 and the ascending sort before it) against the
 // register form, over random active lists, some with repeated entries; returns the number of differing lists.
 uint64_t rsim_cpu_check_island_sort(uint64_t seed, uint64_t iters) {
@@ -231,6 +229,8 @@ uint64_t rsim_cpu_check_sweep(const StaticData* w, const uint32_t* state, uint64
   }
   return bad;
 }
+// Brute force: move_cells against the remove-then-push sequence it replaces, on `iters` random sorted lists (lengths up
+// to the cap, so overflow is exercised) and random block moves in the given world's grid. Returns the mismatch count.
 uint64_t rsim_cpu_check_move_cells(const StaticData* w, uint64_t seed, uint64_t iters) {
   uint64_t bad = 0, x = seed | 1;
   auto rnd = [&x]() {

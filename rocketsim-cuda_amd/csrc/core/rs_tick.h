@@ -349,6 +349,7 @@ struct PadScreens {
 };
 #if defined(__HIP_DEVICE_COMPILE__)
 __device__ inline PadScreens pad_screens_split(const ArenaState& s, const StaticData& w) {
+  static_assert(InLds::ARENAS == 3, "the mask below is every third bit");
   constexpr uint32_t ROUND = 64u / InLds::ARENAS;  // roles that every arena has
   const uint32_t arena = split_arena(), role = split_role();
   const V3 pos[NUM_CARS] = {s.cars[0].pos, s.cars[1].pos};

@@ -90,7 +90,7 @@ __global__ void __launch_bounds__(64) k_features(const uint32_t* __restrict__ st
 // registers from the features to the prediction. The weights stay in registers too, as A operands (a column of 16 outputs'
 // weights per lane), and each wave takes every waves-th tile of 16 arenas. Bound by reading the features: 65,536 arenas
 // (12.6 MB) took 1,099 us with the weights staged in LDS by every wave of 64 arenas and the activations re-laid through LDS.
-constexpr uint32_t INFER_WAVES = 2048;  // two per SIMD: a wave's weights (about 130 words per lane) pay off over its tiles
+constexpr uint32_t INFER_WAVES = 2048;  // two per SIMD: a wave's weights and biases (98 words per lane) pay off over its tiles
 __device__ inline v4s weight_frag(const float* __restrict__ w, int in0, int out, int stride, bool used) {
   v4s f = v4s{0, 0, 0, 0};
   if (used)

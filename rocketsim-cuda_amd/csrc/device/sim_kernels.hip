@@ -258,12 +258,15 @@ hipError_t launch_step_tick(hipStream_t st, uint32_t* buf, const StaticData* w, 
 }
 // The lanes of a work-group that asks for SIM8_BLOCK, the production size: one wave, of fewer arenas where the batch leaves
 // SIMDs idle, since a wave pays for the union of its arenas' paths. 32 lanes as long as they fill at most one wave per
-// SIMD; fewer lose more to the half-empty rows of private memory that crowd the caches than their shorter unions gain
-// (ms per decision at 16 / 32 lanes, contact mix: 4,096 arenas 2.75 / 2.96, 8,192 arenas 3.15 / 3.13, 16,384 arenas 3.66 /
-// 3.36, 32,768 arenas 6.67 / 4.06; kickoffs: 4,096 arenas 1.11 / 1.07, 16,384 arenas 1.50 / 1.25; with an earlier tick, at 32 /
-// 64 lanes, contact mix: 4,096 arenas 3.55 / 4.07, 16,384 arenas 4.02 / 4.44, 32,768 arenas 4.91 / 5.18; kickoffs: 3,500
-// arenas 1.33 / 1.35, 16,384 arenas 1.64 / 1.63). Any
-// other size is the caller's own choice.
+// SIMD; fewer lose more to the half-empty rows of private memory that crowd the caches than their shorter unions gain.
+// Ms per decision at 16 / 32 / 64 lanes:
+//   arenas     contact mix          open play            kickoffs
+//    4,096     2.78 / 2.97 / 3.40   2.51 / 2.57 / 2.91   1.11 / 1.07 / 1.07
+//    8,192     3.11 / 3.12 / 3.51   2.78 / 2.64 / 3.00   1.33 / 1.13 / 1.18
+//   16,384     3.63 / 3.34 / 3.72   3.30 / 2.92 / 3.14   1.51 / 1.25 / 1.25
+//   24,576     5.68 / 3.71 / 4.05   5.37 / 3.59 / 3.81   2.82 / 1.45 / 1.43
+//   32,768     6.71 / 4.05 / 4.33   5.90 / 3.79 / 3.94   2.97 / 1.61 / 1.57
+// Any other size is the caller's own choice.
 static uint32_t wave_lanes(uint32_t n, uint32_t block) { return block == SIM8_BLOCK && n <= SPREAD_MAX_N ? 32u : block; }
 hipError_t launch_run(hipStream_t st, const Sim8Args& p, uint32_t decisions, uint32_t block) {
   if (block == SIM8_BLOCK && p.n <= SMALL_MAX_N) return launch_small(st, p, decisions);

@@ -9,7 +9,8 @@
 // An arena's two cars and its ball are lanes of their own in the phases that treat them alike (P0, P1, P2, P6, P8 and the
 // swept boxes of P3a: SPLIT): with the state in LDS another lane reaches it as well, and a phase that did three bodies or two
 // cars in turn takes the time of one. The mesh walks, the batched separating-axis tests and the passes over all boost pads,
-// whose work items any lane can take, are spread over every lane. Ms per decision, one lane an arena -> bodies and cars
+// whose work items any lane can take, are spread over every lane of the wave's arenas: all 64 where a wave has three, 22
+// where it has one (lane = arena + 3 * role either way, and the lanes of arenas it does not have stay idle). Ms per decision, one lane an arena -> bodies and cars
 // split -> walks and tests over all lanes -> boxes and pads too: kickoffs 1,024 arenas 1.01 -> 0.72 -> 0.66 -> 0.61 (P1 109K ->
 // 64K cycles per wave and tick); contact mix 64 arenas 1.36 -> 1.29 -> 1.11 -> 1.07, 1,000 arenas 2.05 -> 1.76 -> 1.52 ->
 // 1.47.

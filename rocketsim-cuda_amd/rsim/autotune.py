@@ -8,6 +8,8 @@ candidate schedule on the device, each captured once in a HIP graph and replayed
     decisions per launch (rsim_run: the arena held in the lane's private memory across decisions);
   - scheduling of the multi-decision launch: one work-group per AoSoA block (rsim_run), or persistent work-groups taking
     blocks from a queue (rsim_run_queued), in index order or heaviest block first by the learned cost model.
+With block 64, batches up to 32,768 arenas run whole decisions on narrower waves (include/rsim.h), split ones do not, and
+their queue in index order is rsim_run.
 The AoSoA width is not a knob: it is the state buffer's format (64, one wave), which every entry point and caller shares.
 
 Every candidate's result words of every decision and its final states must equal the plain per-launch run's (block 64,
