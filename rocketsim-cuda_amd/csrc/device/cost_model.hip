@@ -337,7 +337,7 @@ __global__ void __launch_bounds__(256) k_adam(float* __restrict__ params, float*
 // dst item i = src item perm[i] (words per item contiguous) and its inverse.
 __global__ void __launch_bounds__(256) k_gather_words(const uint32_t* __restrict__ src, const uint32_t* __restrict__ perm,
                                                       uint32_t* __restrict__ dst, uint32_t n, uint32_t words) {
-  size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  size_t e = ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x;
   if (e >= (size_t)n * words) return;
   size_t i = e / words, w = e % words;
   uint32_t j = perm[i];
@@ -345,7 +345,7 @@ __global__ void __launch_bounds__(256) k_gather_words(const uint32_t* __restrict
 }
 __global__ void __launch_bounds__(256) k_scatter_words(const uint32_t* __restrict__ src, const uint32_t* __restrict__ perm,
                                                        uint32_t* __restrict__ dst, uint32_t n, uint32_t words) {
-  size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  size_t e = ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x;
   if (e >= (size_t)n * words) return;
   size_t i = e / words, w = e % words;
   uint32_t j = perm[i];
@@ -585,8 +585,11 @@ hipError_t launch_adam(hipStream_t st, float* params, float* m, float* v, const 
 }
 hipError_t launch_gather_words(hipStream_t st, const uint32_t* src, const uint32_t* perm, uint32_t* dst, uint32_t n, uint32_t words,
                                bool scatter) {
-  if (scatter) k_scatter_words<<<blocks_of((size_t)n * words, 256), 256, 0, st>>>(src, perm, dst, n, words);
-  else k_gather_words<<<blocks_of((size_t)n * words, 256), 256, 0, st>>>(src, perm, dst, n, words);
+  const size_t blocks = ((size_t)n * words + 255) / 256;  // in rows of 2^20: a launch takes fewer than 2^32 work-items in x
+  const unsigned x = blocks < (1u << 20) ? (unsigned)blocks : 1u << 20;
+  const dim3 g(x, (unsigned)((blocks + x - 1) / x));
+  if (scatter) k_scatter_words<<<g, 256, 0, st>>>(src, perm, dst, n, words);
+  else k_gather_words<<<g, 256, 0, st>>>(src, perm, dst, n, words);
   return hipGetLastError();
 }
 hipError_t launch_gather_states(hipStream_t st, const uint32_t* src, uint32_t n_src, const uint32_t* perm, uint32_t* dst,

@@ -616,3 +616,26 @@ def test_gather_a_sample_of_a_large_source(rsim, device, n):
     device.gather_states(src, device.upload_words(idx), dst)
     want = np.where((idx < n_src)[:, None], states[np.minimum(idx, n_src - 1)], np.uint32(0))
     assert np.array_equal(device.download_states(dst), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scatter", [0, 1])
+def test_permute_words_past_a_one_dimensional_grid(rsim, device, scatter):
+    """2^26 + 1 items of 64 words, 64 words more than a launch takes work-items in one dimension (17 GB a buffer): rows at the
+    edges and between, each carried through the large buffers and back out."""
+    n, words = 2**26 + 1, 64
+    note("permute_words, %d items of %d words, scatter %d" % (n, words, scatter))
+    src, dst = device.alloc_words(n * words), device.alloc_words(n * words)
+    try:
+        perm = np.arange(n, dtype=np.uint32)[::-1].copy()
+        rows = np.array([0, 1, 2, 3, 1000, n // 2, n - 2, n - 1])
+        row = lambda r: np.random.default_rng(int(r)).integers(0, 2**32, words, dtype=np.uint32)
+        for r in rows:
+            device.write_words(src.view(int(r) * words, words), row(r))
+        p = device.upload_words(perm)
+        rsim._check(rsim.lib().rsim_permute_words(device.handle, src.handle, p.handle, n, words, scatter, dst.handle), "permute")
+        for r in rows:
+            got = device.read_words(dst.view(int(n - 1 - r) * words, words))
+            assert np.array_equal(got, row(r)), r
+    finally:
+        src.free(), dst.free()
